@@ -46,6 +46,9 @@ EXPORTED_SYMBOLS = (
     "atlas_scan_fwd",
     "atlas_scan_bwd",
     "atlas_window_sum",
+    "atlas_omega_chain_fwd",
+    "atlas_omega_chain_bwd",
+    "atlas_omega_chain_workspace_bytes",
     "atlas_affine_scan_fwd",
     "atlas_affine_scan_bwd",
     "atlas_affine_scan_workspace_bytes",
@@ -150,6 +153,12 @@ def load(path: str | None = None) -> ctypes.CDLL:
     lib.atlas_scan_bwd.argtypes = [i32, i64, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.atlas_window_sum.restype = i32
     lib.atlas_window_sum.argtypes = [i32, i64, i64, i64, i32, i32, vp, vp, vp]
+    lib.atlas_omega_chain_fwd.restype = i32
+    lib.atlas_omega_chain_fwd.argtypes = [i32, i64, i64, i64, i32, i32] + [vp] * 12
+    lib.atlas_omega_chain_bwd.restype = i32
+    lib.atlas_omega_chain_bwd.argtypes = [i32, i64, i64, i64, i32, i32] + [vp] * 18 + [i64, vp]
+    lib.atlas_omega_chain_workspace_bytes.restype = i64
+    lib.atlas_omega_chain_workspace_bytes.argtypes = [i64, i64, i64, i32]
     lib.atlas_affine_scan_fwd.restype = i32
     lib.atlas_affine_scan_fwd.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp, sz, vp]
     lib.atlas_affine_scan_bwd.restype = i32

@@ -210,6 +210,30 @@ int atlas_scan_bwd(int dtype, int64_t n, int64_t t, int64_t d, const void* gates
 int atlas_window_sum(int dtype, int64_t n, int64_t t, int64_t d, int window, int reverse,
                      const void* x, void* y, void* stream);
 
+/* The Omega weight-update chain of one parameter (atlas_pytorch/omega.py:254-322), fused: surprises
+ * [bh, n, p] -> momentum scans of `order` orders (gates `momentum` [order, bh, n], carried
+ * last_momentum [order, bh, p]), the gate [bh, n] (NULL: none), the inclusive window sum over
+ * [buffer (bh, window - 1, p; NULL: zeros); tokens] and the 1 - decay scan from last_update.
+ * update [bh, n + 1, p] is led by last_update, and is zero when every gate is below 1e-3; moments
+ * [order, bh, n, p] (NULL when no backward follows) keeps the momenta; next_momentum [order, bh, p]
+ * and next_buffer [bh, window - 1, p] carry over. order <= 2, window <= 16, rows of one dtype; every
+ * [.., p] pointer 16-byte aligned. */
+int atlas_omega_chain_fwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
+                          const void* decay, const void* last_update, const void* momentum, const void* last_momentum,
+                          const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
+                          void* next_buffer, void* stream);
+
+/* Gradients of atlas_omega_chain_fwd from those of its outputs (each NULL: zero) and the forward's
+ * update and moments. dgate iff gate; dbuffer NULL: not wanted. workspace: at least
+ * atlas_omega_chain_workspace_bytes(bh, n, p, order) bytes. */
+int atlas_omega_chain_bwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
+                          const void* decay, const void* momentum, const void* last_momentum, const void* gate,
+                          const void* update, const void* moments, const void* dupdate, const void* dnext_momentum,
+                          const void* dnext_buffer, void* dsurprise, void* ddecay, void* dlast_update, void* dmomentum,
+                          void* dlast_momentum, void* dgate, void* dbuffer, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+int64_t atlas_omega_chain_workspace_bytes(int64_t bh, int64_t n, int64_t p, int order);
+
 /* Right-affine scan H_t = H_{t-1} A_t + B_t over t = 1..T, fp32 (replaces affine_associative_scan,
  * atlas_pytorch/affine_scan.py:36-158): A [n,t,d,d], B [n,t,r,d], prev = H_0 [n,r,d] (NULL: zero),
  * out = H_1..H_T [n,t,r,d]; r, d <= 64. Chunked on the fp32 matrix cores: the chunks' composed maps,
