@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kBwThreads) void k_buf_bwd(const Geom g, const BwdP
   const bf16* w0 = reinterpret_cast<const bf16*>(p.wsh) + (size_t)bh * g.nc * CH * R::SPM;  // chunk 0
   float* blk = p.scal + (size_t)bh * g.nc * SB::SIZE;                                       // chunk 0
   const float* Bb = a.buf_in + (size_t)bh * H * D * D;
-  stage_rows(sdy, a.dy + tb * D, Lq, CH, MAP_OFF, 1);
+  stage_rows(sdy, a.dy ? a.dy + tb * D : a.q, a.dy ? Lq : 0, CH, MAP_OFF, 1);   // no dy: zeros
   if (s == H) {
     // dq: C[k][q] = sum_s sum_i B_s[i][k] (w(q, s) dy_q[i]); wave w: features 16 w .., both token
     // tiles; A[k][i] = B_s[i][k] straight from memory (lane: column 16 w + tl, rows 16 kq + j)

@@ -117,7 +117,8 @@ __device__ __forceinline__ void rows_load(RowPf<NWL>& pf, int t0, int w) {
     const int row0 = is_k ? t0 - HT + 8 * j
                    : is_v ? t0 - HT + 8 * (j - SRC / 8)
                    : is_q ? t0 + 8 * (j - 2 * SRC / 8) : t0 + 8 * (j - 2 * SRC / 8 - CL / 8);
-    pf.v[u] = bld16(make_rsrc(base + rb, nb), j < NWL ? (uint32_t)(row0 * (D * 2)) + lo : kOob);
+    // (no dy: a loss on the final state alone; an empty resource reads zeros)
+    pf.v[u] = bld16(make_rsrc(base + rb, base ? nb : 0u), j < NWL ? (uint32_t)(row0 * (D * 2)) + lo : kOob);
   }
 }
 template <bool MAPE, int NWL>

@@ -104,7 +104,7 @@ typedef struct atlas_mem_bwd_args {
   const void* lr; const void* decay; const void* beta; const void* gate;
   const float* S_ref; const float* S0; const float* Z0; const float* buffer_in;
   /* incoming gradients; NULL means zero */
-  const void* dy;           /* [bh, T, d_v] (dtype) */
+  const void* dy;           /* [bh, T, d_v] (dtype); NULL: zero */
   const float* dS_T;        /* [bh, d_v, d_k] */
   const float* dZ_T;        /* [bh, d_v, d_k] */
   const float* dbuffer_out; /* [bh, e-1, d_v, d_k] */
