@@ -225,6 +225,23 @@ def load(path: str | None = None) -> ctypes.CDLL:
     return lib
 
 
+_NATIVE = None
+
+
+def native():
+    """The extension module atlas_rnn_amd._host (csrc/host.cpp): the host path of the operators in native
+    code. Raises LibraryMissing if it is not built; there is no other implementation."""
+    global _NATIVE
+    if _NATIVE is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as exc:
+            raise LibraryMissing(f"atlas_rnn_amd._host is not built ({exc}); run `python -m atlas_rnn_amd.build`") from exc
+        _NATIVE = _host
+    return _NATIVE
+
+
 def check(status: int, what: str) -> None:
     if status != OK:
         msg = load().atlas_mem_strerror(status).decode()

@@ -3,7 +3,7 @@
     python -m atlas_rnn_amd.build          # builds atlas_rnn_amd/libatlas_mem.so in place
 
 The library is plain HIP C++ with an extern "C" ABI (include/atlas_mem.h); the Python package
-loads it with ctypes.
+calls it through the extension module atlas_rnn_amd._host (csrc/host.cpp, built here too) and ctypes.
 """
 
 from __future__ import annotations
@@ -20,6 +20,8 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "libatlas_mem.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["abi.hip", "coef.hip", "seg_fwd.hip", "seg_bwd.hip", "scan.hip", "affine.hip", "bwd_scalar.hip", "walk_fwd.hip", "walk_bwd.hip", "tmap.hip", "step.hip", "prologue.hip", "blocks.hip", "factors.hip", "bufwalk.hip", "wgrad.hip", "gemm.hip", "chunk_bwd.hip", "chunk_coef.hip", "chain.hip"]
+HOST_SOURCE = "host.cpp"                 # the host path (torch extension module atlas_rnn_amd._host)
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 ARCH = os.environ.get("ATLAS_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -56,6 +58,24 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found (ROCm is required to build libatlas_mem.so)")
 
 
+def _host_cmds(obj: str, out: str) -> tuple[list[str], list[str]]:
+    """The compile and link commands of the extension module: host code only, against torch's headers
+    and libatlas_mem.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cxx = os.environ.get("CXX", "g++")
+    inc = [f"-I{p}" for p in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])]
+    compile_cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                   "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_host",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
+                   "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj]
+    link_cmd = [cxx, "-shared", obj, "-o", out, *(f"-L{p}" for p in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch",
+                "-ltorch_python", "-lc10_hip", "-ltorch_hip", f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN"]
+    return compile_cmd, link_cmd
+
+
 def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -68,7 +88,8 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 def build(verbose: bool = False) -> str:
-    """Compile every HIP source for gfx950 and link libatlas_mem.so. Always recompiles."""
+    """Compile every HIP source for gfx950, link libatlas_mem.so and build the extension module
+    atlas_rnn_amd._host on it. Always recompiles."""
     hipcc = _hipcc()
     obj_dir = os.path.join(PKG_DIR, "_build")
     os.makedirs(obj_dir, exist_ok=True)
@@ -78,11 +99,16 @@ def build(verbose: bool = False) -> str:
         obj = os.path.join(obj_dir, src.replace(".hip", ".o"))
         objs.append(obj)
         cmds.append([hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj])
+    host_obj, host_tmp = os.path.join(obj_dir, "host.o"), HOST_PATH + ".tmp"
+    host_compile, host_link = _host_cmds(host_obj, host_tmp)
+    cmds.insert(0, host_compile)   # the longest one first
     with ThreadPoolExecutor(max_workers=min(len(cmds), max(1, (os.cpu_count() or 2) // 2))) as ex:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB_PATH)
+    _run(host_link, verbose)
+    os.replace(host_tmp, HOST_PATH)
     return LIB_PATH
 
 

@@ -127,85 +127,6 @@ def _problem(cfg: RecurrenceConfig, bh, T, dk, dv, momentum, gate, has_buffer, d
     return p
 
 
-class MemoryRecurrenceFn(torch.autograd.Function):
-    """y, S_T, Z_T, buffer_out = recurrence(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer).
-
-    k, q, v, lr, decay, beta, gate: same dtype (fp32 or bf16), contiguous; states fp32.
-    Z_T / buffer_out are empty tensors when momentum is off / window == 1.
-    """
-
-    @staticmethod
-    def forward(ctx, k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg: RecurrenceConfig):
-        # outputs a loss does not use get no gradient tensor (the kernels treat a missing dS_T,
-        # dZ_T or buffer_out gradient as zero without reading one)
-        ctx.set_materialize_grads(False)
-        lib = _lib.load()
-        check_operands(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, window=cfg.window, dtype=k.dtype,
-                       contiguous=True)
-        bh, T, dk = k.shape
-        dv = v.shape[-1]
-        momentum = beta is not None
-        prob = _problem(cfg, bh, T, dk, dv, momentum, gate, buf is not None, k.dtype)
-        _lib.check(lib.atlas_mem_validate(ctypes.byref(prob)), "atlas_mem_validate")
-        dev = k.device
-        y = torch.empty(bh, T, dv, device=dev, dtype=k.dtype)
-        S_T = torch.empty(bh, dv, dk, device=dev, dtype=torch.float32)
-        Z_T = torch.empty(bh, dv, dk, device=dev, dtype=torch.float32) if momentum else None
-        e = cfg.window
-        buf_out = torch.empty(bh, e - 1, dv, dk, device=dev, dtype=torch.float32) if e > 1 else None
-        # segment-start states and aggregates: the forward writes them (it needs them for its own
-        # second pass) and the backward re-reads them
-        nbytes = lib.atlas_mem_saved_bytes(ctypes.byref(prob))
-        saved = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
-        a = _lib.FwdArgs(k=_ptr(k), q=_ptr(q), v=_ptr(v), lr=_ptr(lr), decay=_ptr(decay), beta=_ptr(beta),
-                         gate=_ptr(gate), S_ref=_ptr(S_ref), S0=_ptr(S0), Z0=_ptr(Z0), buffer_in=_ptr(buf),
-                         y=_ptr(y), S_T=_ptr(S_T), Z_T=_ptr(Z_T), buffer_out=_ptr(buf_out))
-        _lib.check(lib.atlas_mem_fwd(ctypes.byref(prob), ctypes.byref(a), _ptr(saved), _stream(dev)), "atlas_mem_fwd")
-        ctx.cfg = cfg
-        ctx.prob = prob
-        ctx.momentum = momentum
-        ctx.save_for_backward(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, saved)
-        empty = torch.empty(0, device=dev)
-        return y, S_T, (Z_T if Z_T is not None else empty), (buf_out if buf_out is not None else empty)
-
-    @staticmethod
-    def backward(ctx, dy, dS_T, dZ_T, dbuf_out):
-        lib = _lib.load()
-        k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, saved = ctx.saved_tensors
-        prob = ctx.prob
-        dev = k.device
-        bh, T, dk = k.shape
-        dv_ = v.shape[-1]
-        f32 = torch.float32
-        dy = _aligned(dy.to(k.dtype)) if dy is not None else None
-        dS_T = _aligned(dS_T.float()) if dS_T is not None else None
-        dZ_T = _aligned(dZ_T.float()) if (dZ_T is not None and ctx.momentum and dZ_T.numel() > 0) else None
-        dbuf_out = _aligned(dbuf_out.float()) if (dbuf_out is not None and dbuf_out.numel() > 0) else None
-        dk_ = torch.empty_like(k)
-        dq_ = torch.empty_like(q)
-        dv_t = torch.empty_like(v)
-        dlr = torch.empty_like(lr)
-        ddecay = torch.empty_like(decay)
-        dbeta = torch.empty_like(beta) if beta is not None else None
-        dgate = torch.empty_like(gate) if gate is not None else None
-        dS_ref = torch.empty(bh, dv_, dk, device=dev, dtype=f32)
-        dS0 = torch.empty(bh, dv_, dk, device=dev, dtype=f32)
-        dZ0 = torch.empty(bh, dv_, dk, device=dev, dtype=f32) if ctx.momentum else None
-        dbuf_in = torch.empty_like(buf) if buf is not None else None
-        ws_bytes = lib.atlas_mem_bwd_workspace_bytes(ctypes.byref(prob))
-        ws = torch.empty((ws_bytes + 3) // 4, device=dev, dtype=f32)
-        a = _lib.BwdArgs(k=_ptr(k), q=_ptr(q), v=_ptr(v), lr=_ptr(lr), decay=_ptr(decay), beta=_ptr(beta),
-                         gate=_ptr(gate), S_ref=_ptr(S_ref), S0=_ptr(S0), Z0=_ptr(Z0), buffer_in=_ptr(buf),
-                         dy=_ptr(dy), dS_T=_ptr(dS_T), dZ_T=_ptr(dZ_T), dbuffer_out=_ptr(dbuf_out),
-                         dk=_ptr(dk_), dq=_ptr(dq_), dv=_ptr(dv_t), dlr=_ptr(dlr), ddecay=_ptr(ddecay),
-                         dbeta=_ptr(dbeta), dgate=_ptr(dgate), dS_ref=_ptr(dS_ref), dS0=_ptr(dS0),
-                         dZ0=_ptr(dZ0), dbuffer_in=_ptr(dbuf_in))
-        _lib.check(lib.atlas_mem_bwd(ctypes.byref(prob), ctypes.byref(a), _ptr(saved), _ptr(ws),
-                                     ctypes.c_size_t(ws_bytes), _stream(dev)), "atlas_mem_bwd")
-        return (dk_, dq_, dv_t, dlr, ddecay, dbeta, dgate, dS_ref, dS0,
-                dZ0 if Z0 is not None else None, dbuf_in, None)
-
-
 def _aligned(x: Tensor | None) -> Tensor | None:
     """x contiguous with a 16-byte aligned start (the C ABI rejects other pointers)."""
     if x is None:
@@ -250,52 +171,22 @@ def symmetrized_tables(proj: Tensor, d: int, dtype) -> tuple[Tensor, Tensor]:
     [x; vec(x x^T)] proj = [x; vec(x x^T)] P' with P'[a][b] = proj[a][b] + proj[b][a] above the
     diagonal, proj[a][a] on it and zeros below. Nothing is cached here: the owner of proj keeps the
     tables (PolynomialFeatureMap does, per dtype and device) and passes them to tensor_feature_map."""
-    lib = _lib.load()
-    dev = proj.device
-    m = proj.shape[1]
-    p = _aligned(proj.detach().to(dtype))
-    ps = torch.empty_like(p)
-    pst = torch.empty(m, p.shape[0], device=dev, dtype=p.dtype)
-    _lib.check(lib.atlas_tensor_map_symmetrize(_dt_code(p), d, m, _ptr(p), _ptr(ps), _ptr(pst), _stream(dev)),
-               "atlas_tensor_map_symmetrize")
-    return ps, pst
+    if dtype not in _DTYPES:
+        raise ValueError(f"symmetrized_tables: dtype {dtype} (the kernels take bfloat16 or float32)")
+    _require_gpu(proj)
+    return _lib.native().symmetrized(proj, d, dtype)
 
 
-class _TensorMapFn(torch.autograd.Function):
-    """atlas_tensor_map_fwd / _bwd: x [n, d] and P [d + d*d, m] (bf16 or fp32, P in x's dtype as the
-    reference casts it) -> phi [n, m], followed by the elementwise polynomial of `degree` (1: none);
-    P is a constant (a registered buffer in the reference, so it has no gradient)."""
+class _TensorMapFn:
+    """The tensor map's autograd node (csrc/host.cpp): x [n, d] and P [d + d*d, m] (bf16 or fp32, P in
+    x's dtype as the reference casts it) -> phi [n, m], followed by the elementwise polynomial of
+    `degree` (1: none); P is a constant (a registered buffer in the reference, so it has no gradient)."""
 
     @staticmethod
-    def forward(ctx, x, proj, degree, tables=None):
-        dev = _require_gpu(x, proj)
-        lib = _lib.load()
-        lead, d, m = x.shape[:-1], x.shape[-1], proj.shape[-1]
-        x2 = _aligned(x.reshape(-1, d))
-        ps, pst = tables if tables is not None else symmetrized_tables(proj, d, x.dtype)
-        n = x2.shape[0]
-        out = torch.empty(n, m, device=dev, dtype=x.dtype)
-        pre = torch.empty(n, m, device=dev, dtype=x.dtype) if degree > 1 else None
-        _lib.check(lib.atlas_tensor_map_fwd_sym(_dt_code(x2), n, d, m, degree, _ptr(x2), _ptr(pst), _ptr(out),
-                                                _ptr(pre), _stream(dev)), "atlas_tensor_map_fwd_sym")
-        p = ps
-        ctx.save_for_backward(x2, p, pre)
-        ctx.lead = lead
-        ctx.degree = degree
-        return out.reshape(*lead, m)
-
-    @staticmethod
-    def backward(ctx, dout):
-        x2, p, pre = ctx.saved_tensors
-        dev = x2.device
-        lib = _lib.load()
-        n, d = x2.shape
-        m = p.shape[-1]
-        g = _aligned(dout.reshape(-1, m).to(x2.dtype))
-        dx = torch.empty_like(x2)
-        _lib.check(lib.atlas_tensor_map_bwd_sym(_dt_code(x2), n, d, m, ctx.degree, _ptr(x2), _ptr(p), _ptr(pre),
-                                                _ptr(g), _ptr(dx), _stream(dev)), "atlas_tensor_map_bwd_sym")
-        return dx.reshape(*ctx.lead, d), None, None, None
+    def apply(x, proj, degree, tables=None):
+        _require_gpu(x, proj)
+        ps, pst = tables if tables is not None else (None, None)
+        return _lib.native().tensor_map(x, proj, degree, ps, pst)
 
 
 def _tables_ok(tables, proj: Tensor, dtype) -> bool:
@@ -335,97 +226,30 @@ def _poly_map(x: Tensor, degree: int) -> Tensor:
     return out.to(x.dtype)
 
 
-class _BlockSplitFn(torch.autograd.Function):
-    """phi, psi [BH, T, Dk], v [BH, T, Dv], S_ref [BH, Dv, Dk] -> the stacked 64-wide operands of the
-    state blocks (atlas_block_split / atlas_block_merge): phi_b, psi_b, nv_b [NB BH, T, 64] with
-    nv = v - S_ref phi, block r = (i * Dk/64 + j) * BH + bh."""
-
-    @staticmethod
-    def forward(ctx, phi, psi, v, S_ref):
-        lib = _lib.load()
-        bh, T, dk = phi.shape
-        dv = v.shape[-1]
-        nb = (dk // _BLOCK) * (dv // _BLOCK)
-        phi, psi, v, S_ref = _aligned(phi), _aligned(psi), _aligned(v), _aligned(S_ref.float())
-        out = [torch.empty(nb * bh, T, _BLOCK, device=phi.device, dtype=phi.dtype) for _ in range(3)]
-        _lib.check(lib.atlas_block_split(_dt_code(phi), bh, T, dk, dv, _ptr(phi), _ptr(psi), _ptr(v), _ptr(S_ref),
-                                         _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _stream(phi.device)),
-                   "atlas_block_split")
-        ctx.save_for_backward(phi, S_ref)
-        ctx.dv = dv
-        return tuple(out)
-
-    @staticmethod
-    def backward(ctx, dphi_b, dpsi_b, dnv_b):
-        lib = _lib.load()
-        phi, S_ref = ctx.saved_tensors
-        bh, T, dk = phi.shape
-        dv = ctx.dv
-        z = lambda g: torch.zeros(dk // _BLOCK * (dv // _BLOCK) * bh, T, _BLOCK, device=phi.device,
-                                  dtype=phi.dtype) if g is None else _aligned(g.to(phi.dtype))
-        dphi_b, dpsi_b, dnv_b = z(dphi_b), z(dpsi_b), z(dnv_b)
-        dphi = torch.empty_like(phi)
-        dpsi = torch.empty_like(phi)
-        dvv = torch.empty(bh, T, dv, device=phi.device, dtype=phi.dtype)
-        parts = torch.empty(bh, lib.atlas_block_parts(T), dv, dk, device=phi.device, dtype=torch.float32)
-        _lib.check(lib.atlas_block_merge(_dt_code(phi), bh, T, dk, dv, _ptr(phi), _ptr(S_ref), _ptr(dphi_b),
-                                         _ptr(dpsi_b), _ptr(dnv_b), _ptr(dphi), _ptr(dpsi), _ptr(dvv), _ptr(parts),
-                                         _stream(phi.device)), "atlas_block_merge")
-        return dphi, dpsi, dvv, parts.sum(dim=1)
-
-
 _REPLICATE, _REPLICA_SUM = 0, 1
 
 
-def _replicas(op: int, nrep: int, xs):
-    """atlas_replicas over a list of tensors (one launch per dtype, up to four arrays each):
-    _REPLICATE gives [nrep * x.shape[0], ...] (x repeated along the first axis), _REPLICA_SUM the
-    sum of the nrep replicas stacked along the first axis of x."""
-    lib = _lib.load()
-    xs = [x.contiguous() for x in xs]
-    if op == _REPLICA_SUM:
-        for x in xs:
-            if x.shape[0] % nrep != 0:
-                raise ValueError(f"replica sum: first axis {x.shape[0]} is not a multiple of {nrep} replicas")
-    outs = [torch.empty(((nrep * x.shape[0]) if op == _REPLICATE else (x.shape[0] // nrep),) + tuple(x.shape[1:]),
-                        device=x.device, dtype=x.dtype) for x in xs]
-    for dt in {x.dtype for x in xs}:
-        idx = [i for i, x in enumerate(xs) if x.dtype == dt]
-        for c0 in range(0, len(idx), 4):
-            grp = idx[c0:c0 + 4]
-            cnt = len(grp)
-            n64 = (ctypes.c_int64 * cnt)(*[(xs[i] if op == _REPLICATE else outs[i]).numel() for i in grp])
-            vp = ctypes.c_void_p * cnt
-            _lib.check(lib.atlas_replicas(op, _DTYPES[dt], cnt, nrep, n64, vp(*[xs[i].data_ptr() for i in grp]),
-                                          vp(*[outs[i].data_ptr() for i in grp]), _stream(xs[0].device)),
-                       "atlas_replicas")
-    return outs
-
-
-class _ReplicateFn(torch.autograd.Function):
-    """Each tensor repeated nrep times along its first axis; the adjoint sums the replicas."""
+class _ReplicateFn:
+    """Each tensor repeated nrep times along its first axis; the adjoint sums the replicas
+    (atlas_replicas, one launch per dtype, up to four arrays each)."""
 
     @staticmethod
-    def forward(ctx, nrep, *xs):
-        ctx.nrep = nrep
-        return tuple(_replicas(_REPLICATE, nrep, xs))
-
-    @staticmethod
-    def backward(ctx, *gs):
-        return (None,) + tuple(_replicas(_REPLICA_SUM, ctx.nrep, gs))
+    def apply(nrep, *xs):
+        return tuple(_lib.native().replicate(nrep, list(xs)))
 
 
-class _ReplicaSumFn(torch.autograd.Function):
+class _ReplicaSumFn:
     """The sum of the nrep replicas stacked along each tensor's first axis; the adjoint repeats."""
 
     @staticmethod
-    def forward(ctx, nrep, *xs):
-        ctx.nrep = nrep
-        return tuple(_replicas(_REPLICA_SUM, nrep, xs))
+    def apply(nrep, *xs):
+        return tuple(_lib.native().replica_sum(nrep, list(xs)))
 
-    @staticmethod
-    def backward(ctx, *gs):
-        return (None,) + tuple(_replicas(_REPLICATE, ctx.nrep, gs))
+
+def _replicas(op: int, nrep: int, xs):
+    """_REPLICATE gives [nrep * x.shape[0], ...] (x repeated along the first axis), _REPLICA_SUM the sum
+    of the nrep replicas stacked along the first axis of x."""
+    return (_ReplicateFn if op == _REPLICATE else _ReplicaSumFn).apply(nrep, *xs)
 
 
 def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
@@ -464,7 +288,8 @@ def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
     pst = lambda t: padf(t, (0, pad_k, 0, pad_v))
     S_ref, S0, Z0, buffer = pst(S_ref), pst(S0), pst(Z0), pst(buffer)
     nb = nbv * nbk
-    kb, qb, vb = _BlockSplitFn.apply(phi, psi, vv, S_ref)
+    _dt_code(phi)   # fp32 or bf16
+    kb, qb, vb = _lib.native().block_split(phi, psi, vv, S_ref)   # its adjoint: atlas_block_merge
 
     def stack_state(x):        # [BH, ..., Dv, Dk] -> [(i, j, bh), ..., 64, 64]
         if x is None:
@@ -476,7 +301,7 @@ def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
         return x.reshape(nb * bh, *mid, _BLOCK, _BLOCK)
 
     # the per-token scalars of every block: one replicating launch (its adjoint: one summing launch)
-    scal = [t for t in (lr, decay, beta, gate) if t is not None]
+    scal = [t if t.dtype == phi.dtype else t.to(phi.dtype) for t in (lr, decay, beta, gate) if t is not None]
     reps = iter(_ReplicateFn.apply(nb, *scal))
     lr_b, decay_b, beta_b, gate_b = [None if t is None else next(reps) for t in (lr, decay, beta, gate)]
     S0b, Z0b, Bb = stack_state(S0), stack_state(Z0), stack_state(buffer)
@@ -501,29 +326,6 @@ def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
         return x[..., :dv, :dk]
 
     return y[..., :dv], unblock(S_T), unblock(Z_T), unblock(B)
-
-
-def _memory_step(cfg: RecurrenceConfig, args, states):
-    """One token without autograd (atlas_mem_step): the generation step of
-    atlas_pytorch/rnn_transformer.py:863-900 through the cell's recurrence at T = 1."""
-    k, q, v, lr, decay, beta, gate = args
-    S_ref, S0, Z0, buf = states
-    lib = _lib.load()
-    bh, _, dk = k.shape
-    dv = v.shape[-1]
-    dev = k.device
-    momentum = beta is not None
-    e = cfg.window
-    prob = _problem(cfg, bh, 1, dk, dv, momentum, gate, buf is not None, k.dtype)
-    y = torch.empty(bh, 1, dv, device=dev, dtype=k.dtype)
-    S_T = torch.empty(bh, dv, dk, device=dev, dtype=torch.float32)
-    Z_T = torch.empty_like(S_T) if momentum else None
-    buf_out = torch.empty(bh, e - 1, dv, dk, device=dev, dtype=torch.float32) if e > 1 else None
-    a = _lib.FwdArgs(k=_ptr(k), q=_ptr(q), v=_ptr(v), lr=_ptr(lr), decay=_ptr(decay), beta=_ptr(beta),
-                     gate=_ptr(gate), S_ref=_ptr(S_ref), S0=_ptr(S0), Z0=_ptr(Z0), buffer_in=_ptr(buf),
-                     y=_ptr(y), S_T=_ptr(S_T), Z_T=_ptr(Z_T), buffer_out=_ptr(buf_out))
-    _lib.check(lib.atlas_mem_step(ctypes.byref(prob), ctypes.byref(a), _stream(dev)), "atlas_mem_step")
-    return y, S_T, Z_T, buf_out
 
 
 # ---------------------------------------------------------------------------------------------
@@ -647,6 +449,13 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
     buffer [BH, e-1, d_v, d_k]. Returns (y [BH,T,d_v] in the input dtype, S_T, Z_T or None,
     buffer_out or None) with fp32 states.
     """
+    if clamp_every is not None and k.dim() == 3 and clamp_every >= k.shape[1]:
+        clamp_every = None        # no clamp point before the last token (the final clamp is clamp_final's)
+    out = _lib.native().recurrence(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
+                                   map_degree if map_mode == 'elementwise' else 1, clamp_every, bool(clamp_final))
+    if out is not None:
+        return out
+    # everything the kernels do not take as it is: other head sizes, calls in pieces, and the errors
     dev = _require_gpu(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer)
     dt = k.dtype if k.dtype in _DTYPES else torch.float32
     if k.dim() != 3 or v.dim() != 3:
@@ -675,15 +484,11 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
         return (y[..., :dk], S_T[..., :dk, :dk], None if Z_T is None else Z_T[..., :dk, :dk],
                 None if B is None else B[..., :dk, :dk])
     e = window
-    if clamp_every is not None and clamp_every >= T:
-        clamp_every = None        # no clamp point before the last token (the final clamp is clamp_final's)
     cfg = RecurrenceConfig(window=e, map_mode=map_mode, map_degree=map_degree,
                            clamp_every=clamp_every, clamp_final=clamp_final)
     args = [_canon(t, dt) for t in (k, q, v, lr, decay, beta, gate)]
     states = [_canon(t, torch.float32) for t in (S_ref, S0, Z0 if beta is not None else None,
                                                   buffer if e > 1 else None)]
-    if T == 1 and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (*args, *states))):
-        return _memory_step(cfg, args, states)   # decode: one launch, no saved buffer
     # window - 1 longer than the chunk implied by clamp_every, or clamp_every without a divisor
     # usable as a chunk: run one call per scan chunk (atlas_pytorch/rnn_memory.py:584-601),
     # carrying S, Z and the buffer, S_ref fixed.
@@ -705,8 +510,7 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
             ys.append(y)
         return torch.cat(ys, dim=1), S, Z, B
     _lib.check(status, "atlas_mem_validate")
-    y, S_T, Z_T, buf_out = MemoryRecurrenceFn.apply(*args, *states, cfg)
-    return y, S_T, (Z_T if beta is not None else None), (buf_out if e > 1 else None)
+    raise RuntimeError("memory_recurrence: a valid problem was not taken by the native path")
 
 
 class AtlasOmegaFunction:
@@ -915,136 +719,6 @@ def _dt_code(t: Tensor) -> int:
     return _DTYPES[t.dtype]
 
 
-def _sum_partials(items):
-    """atlas_partials_sum: items of (partials [rows, ...] fp32, out dtype, out shape) -> the sums over
-    the rows, one launch for all of them (deterministic order)."""
-    lib = _lib.load()
-    parts = [_aligned(p.reshape(p.shape[0], -1)) for p, _, _ in items]
-    outs = [torch.empty(p.shape[1], device=p.device, dtype=dt) for p, (_, dt, _) in zip(parts, items)]
-    cnt = len(parts)
-    I32, VP = ctypes.c_int * cnt, ctypes.c_void_p * cnt
-    _lib.check(lib.atlas_partials_sum(cnt, parts[0].shape[0], I32(*[p.shape[1] for p in parts]),
-                                      VP(*[p.data_ptr() for p in parts]), VP(*[o.data_ptr() for o in outs]),
-                                      I32(*[_DTYPES[o.dtype] for o in outs]), _stream(parts[0].device)),
-               "atlas_partials_sum")
-    return [o.reshape(shape) for o, (_, _, shape) in zip(outs, items)]
-
-
-class _PrologueFn:
-    """xn = RMSNorm(x) and the three depthwise convolutions of xn (atlas_prologue_fwd / _bwd), called
-    by hand from _CellPrologueFn (ctx is a _HandCtx); the backward returns its parameter gradients as
-    per-workgroup partials for one _sum_partials call."""
-
-    @staticmethod
-    def forward(ctx, x, norm_w, wq, wk, wv, conv_k, eps):
-        lib = _lib.load()
-        B, T, dim = x.shape
-        x = _aligned(x)
-        conv = conv_k > 1
-        xn = torch.empty_like(x)
-        qi = torch.empty_like(x) if conv else None
-        ki = torch.empty_like(x) if conv else None
-        vi = torch.empty_like(x) if conv else None
-        inv = torch.empty(B, T, device=x.device, dtype=torch.float32)
-        taps = [_aligned(w.reshape(dim, conv_k)) if conv else None for w in (wq, wk, wv)]
-        _lib.check(lib.atlas_prologue_fwd(_dt_code(x), B, T, dim, conv_k, float(eps), _ptr(x), _ptr(norm_w),
-                                          _ptr(taps[0]), _ptr(taps[1]), _ptr(taps[2]), _ptr(xn), _ptr(qi), _ptr(ki),
-                                          _ptr(vi), _ptr(inv), _stream(x.device)), "atlas_prologue_fwd")
-        ctx.save_for_backward(x, norm_w, *(t if t is not None else torch.empty(0) for t in taps), inv)
-        ctx.conv_k = conv_k
-        ctx.wshape = tuple(wq.shape) if conv else None
-        if not conv:
-            return xn          # the caller uses xn for q_in, k_in and v_in
-        return xn, qi, ki, vi
-
-    @staticmethod
-    def backward(ctx, dxn, *dconv):
-        lib = _lib.load()
-        x, norm_w, tq, tk, tv, inv = ctx.saved_tensors
-        B, T, dim = x.shape
-        K = ctx.conv_k
-        conv = K > 1
-        z = lambda t: torch.zeros_like(x) if t is None else _aligned(t.to(x.dtype))
-        dxn = z(dxn)
-        dqi, dki, dvi = (z(g) for g in dconv) if conv else (None, None, None)
-        nwg = lib.atlas_prologue_num_workgroups(B, T)
-        dx = torch.empty_like(x)
-        dnw = torch.empty(nwg, dim, device=x.device, dtype=torch.float32)
-        dcv = torch.empty(nwg, 3, dim, K, device=x.device, dtype=torch.float32) if conv else None
-        _lib.check(lib.atlas_prologue_bwd(_dt_code(x), B, T, dim, K, _ptr(x), _ptr(norm_w),
-                                          _ptr(tq if conv else None), _ptr(tk if conv else None),
-                                          _ptr(tv if conv else None), _ptr(inv), _ptr(dxn), _ptr(dqi), _ptr(dki),
-                                          _ptr(dvi), _ptr(dx), _ptr(dnw), _ptr(dcv), _stream(x.device)),
-                   "atlas_prologue_bwd")
-        parts = [(dnw, norm_w.dtype, tuple(norm_w.shape))]
-        if conv:
-            parts.append((dcv, x.dtype, (3, *ctx.wshape)))
-        return dx, parts
-
-
-class _HeadsFn:
-    """Head split, MultiheadRMSNorm of q / k and the gate sigmoids (atlas_heads_fwd / _bwd), called by
-    hand from _CellPrologueFn; the backward returns its parameter gradients as partials."""
-
-    @staticmethod
-    def forward(ctx, ql, kl, vl, zl, q_gamma, k_gamma, bias, heads, d):
-        lib = _lib.load()
-        B, T, _ = ql.shape
-        nG = bias.numel() // heads if bias is not None else 0
-        dev = ql.device
-        ql, kl, vl = _aligned(ql), _aligned(kl), _aligned(vl)
-        zl = _aligned(zl) if nG else None
-        qg = _aligned(q_gamma.reshape(heads, d)) if q_gamma is not None else None
-        kg = _aligned(k_gamma.reshape(heads, d)) if k_gamma is not None else None
-        q = torch.empty(B * heads, T, d, device=dev, dtype=ql.dtype)
-        k = torch.empty_like(q)
-        v = torch.empty_like(q)
-        gates = torch.empty(nG, B * heads, T, device=dev, dtype=ql.dtype) if nG else None
-        _lib.check(lib.atlas_heads_fwd(_dt_code(ql), B, T, heads, d, nG, _ptr(ql), _ptr(kl), _ptr(vl), _ptr(zl),
-                                       _ptr(qg), _ptr(kg), _ptr(bias), _ptr(q), _ptr(k), _ptr(v), _ptr(gates),
-                                       _stream(dev)), "atlas_heads_fwd")
-        e0 = torch.empty(0, device=dev)
-        ctx.save_for_backward(ql, kl, qg if qg is not None else e0, kg if kg is not None else e0,
-                              gates if gates is not None else e0)
-        ctx.meta = (heads, d, nG, q_gamma is not None, None if q_gamma is None else tuple(q_gamma.shape),
-                    None if bias is None else bias.dtype)
-        if nG:
-            return (q, k, v, *gates.unbind(0))
-        return q, k, v
-
-    @staticmethod
-    def backward(ctx, dq, dk, dv, *dgates):
-        lib = _lib.load()
-        ql, kl, qg, kg, gates = ctx.saved_tensors
-        heads, d, nG, norm, gshape, bdt = ctx.meta
-        B, T, _ = ql.shape
-        dev = ql.device
-        z = lambda t: torch.zeros(B * heads, T, d, device=dev, dtype=ql.dtype) if t is None else _aligned(t.to(ql.dtype))
-        dq, dk, dv = z(dq), z(dk), z(dv)
-        dg = None
-        if nG:
-            dg = torch.stack([g.to(ql.dtype) if g is not None else torch.zeros(B * heads, T, device=dev, dtype=ql.dtype)
-                              for g in dgates])
-        nwg = lib.atlas_prologue_num_workgroups(B, T)
-        dql, dkl, dvl = torch.empty_like(ql), torch.empty_like(kl), torch.empty_like(ql)
-        dzl = torch.empty(B, T, nG * heads, device=dev, dtype=ql.dtype) if nG else None
-        dqg = torch.empty(nwg, heads, d, device=dev, dtype=torch.float32) if norm else None
-        dkg = torch.empty_like(dqg) if norm else None
-        dbias = torch.empty(nwg, nG * heads, device=dev, dtype=torch.float32) if nG else None
-        _lib.check(lib.atlas_heads_bwd(_dt_code(ql), B, T, heads, d, nG, _ptr(ql), _ptr(kl),
-                                       _ptr(qg if norm else None), _ptr(kg if norm else None),
-                                       _ptr(gates if nG else None), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dg), _ptr(dql),
-                                       _ptr(dkl), _ptr(dvl), _ptr(dzl), _ptr(dqg), _ptr(dkg), _ptr(dbias), _stream(dev)),
-                   "atlas_heads_bwd")
-        parts = {}
-        if norm:
-            parts["qg"] = (dqg, qg.dtype, gshape)
-            parts["kg"] = (dkg, kg.dtype, gshape)
-        if nG:
-            parts["b"] = (dbias, bdt, (nG * heads,))
-        return dql, dkl, dvl, dzl, parts
-
-
 def _wgrads(pairs, dtype) -> list:
     """dW = dy^T x over every leading axis of dy [..., o] and x [..., i], for each (dy, x) of pairs
     (the same token count). bf16 operands go to atlas_linear_wgrad_batch, all layers in one launch
@@ -1052,34 +726,7 @@ def _wgrads(pairs, dtype) -> list:
     summed in a fixed order): 16384 tokens x 512 x 512 took 67 us through a transposed copy and a
     batched hipBLASLt product, whose plain form (one product with K = 16384 on few output tiles)
     took 100 us. fp32 operands keep torch's product over token slices."""
-    dys = [dy.reshape(-1, dy.shape[-1]) for dy, _ in pairs]
-    xs = [x.reshape(-1, x.shape[-1]) for _, x in pairs]
-    n = dys[0].shape[0]
-    if all(d.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and d.shape[-1] % 8 == 0 and x.shape[-1] % 8 == 0
-           and d.shape[0] == n and x.shape[0] == n for d, x in zip(dys, xs)) and dtype in _DTYPES:
-        lib = _lib.load()
-        dys, xs = [_aligned(d) for d in dys], [_aligned(x) for x in xs]
-        dev = dys[0].device
-        cnt = len(dys)
-        I32, VP = ctypes.c_int * cnt, ctypes.c_void_p * cnt
-        os_, is_ = I32(*[d.shape[1] for d in dys]), I32(*[x.shape[1] for x in xs])
-        ws_bytes = lib.atlas_linear_wgrad_batch_workspace_bytes(cnt, n, os_, is_)
-        ws = torch.empty(max(ws_bytes, 16) // 4, device=dev, dtype=torch.float32)
-        dws = [torch.empty(d.shape[1], x.shape[1], device=dev, dtype=dtype) for d, x in zip(dys, xs)]
-        _lib.check(lib.atlas_linear_wgrad_batch(_DTYPES[dtype], cnt, n, os_, is_, VP(*[d.data_ptr() for d in dys]),
-                                                VP(*[x.data_ptr() for x in xs]), VP(*[w.data_ptr() for w in dws]),
-                                                _ptr(ws), ws_bytes, _stream(dev)), "atlas_linear_wgrad_batch")
-        return dws
-    out = []
-    for dy2, x2 in zip(dys, xs):
-        o, i = dy2.shape[-1], x2.shape[-1]
-        S = next((c for c in (8, 4, 2) if n % c == 0 and n // c >= 1024), 1)
-        if S == 1:
-            out.append((dy2.t() @ x2).to(dtype))
-            continue
-        a = dy2.view(S, n // S, o).transpose(1, 2).contiguous()   # both operands row-major (no transposed views)
-        out.append(torch.bmm(a, x2.view(S, n // S, i).contiguous()).float().sum(0).to(dtype))
-    return out
+    return _lib.native().wgrads([dy for dy, _ in pairs], [x for _, x in pairs], dtype)
 
 
 def _wgrad(dy: Tensor, x: Tensor, dtype) -> Tensor:
@@ -1093,118 +740,14 @@ _GEMM_NT, _GEMM_NN = 0, 1
 def _products(layout: int, acts, weights):
     """atlas_linear_batch: up to four bf16 products in one launch. NT: acts[i] [..., k] x
     weights[i] [n, k] -> [..., n] (y = x W^T); NN: acts[i] [..., k] x weights[i] [k, n] -> [..., n]
-    (dx = dy W). Falls back to torch for other dtypes or sizes that are not multiples of 8."""
-    ok = all(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.shape[-1] % 8 == 0
-             and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 for a, w in zip(acts, weights))
-    m = acts[0].numel() // acts[0].shape[-1]
-    if not ok or any(a.numel() // a.shape[-1] != m for a in acts):
-        if layout == _GEMM_NT:
-            return [torch.nn.functional.linear(a, w) for a, w in zip(acts, weights)]
-        return [a @ w for a, w in zip(acts, weights)]
-    lib = _lib.load()
-    dev = acts[0].device
-    a2 = [_aligned(a.reshape(m, a.shape[-1])) for a in acts]
-    w2 = [_aligned(w) for w in weights]
-    ns = [w.shape[0] if layout == _GEMM_NT else w.shape[1] for w in w2]
-    ks = [a.shape[-1] for a in a2]
-    outs = [torch.empty(m, nn, device=dev, dtype=torch.bfloat16) for nn in ns]
-    cnt = len(a2)
-    I32 = ctypes.c_int * cnt
-    VP = ctypes.c_void_p * cnt
-    _lib.check(lib.atlas_linear_batch(layout, cnt, m, I32(*ns), I32(*ks), VP(*[a.data_ptr() for a in a2]),
-                                      VP(*[w.data_ptr() for w in w2]), VP(*[o.data_ptr() for o in outs]),
-                                      _stream(dev)), "atlas_linear_batch")
-    return [o.reshape(*a.shape[:-1], nn) for o, a, nn in zip(outs, acts, ns)]
-
-
-class _LinearFn(torch.autograd.Function):
-    """y = x W^T with its input gradient on atlas_linear_batch and the weight gradient of _wgrad."""
-
-    @staticmethod
-    def forward(ctx, x, w):
-        ctx.save_for_backward(x, w)
-        return _products(_GEMM_NT, [x], [w])[0]
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, w = ctx.saved_tensors
-        dx = _products(_GEMM_NN, [dy], [w])[0] if ctx.needs_input_grad[0] else None
-        dw = _wgrad(dy, x, w.dtype) if ctx.needs_input_grad[1] else None
-        return dx, dw
+    (dx = dy W). torch's products for other dtypes or sizes that are not multiples of 8."""
+    return _lib.native().products(layout, list(acts), list(weights))
 
 
 def linear(x: Tensor, w: Tensor) -> Tensor:
-    """x W^T without bias, with the token-split weight gradient of _LinearFn."""
-    return _LinearFn.apply(x, w)
-
-
-class _HandCtx:
-    """Stands in for autograd's ctx where one Function composes other Functions' forward and
-    backward by hand."""
-
-    def set_materialize_grads(self, value):
-        pass
-
-    def save_for_backward(self, *tensors):
-        self.saved_tensors = tensors
-
-
-class _CellPrologueFn(torch.autograd.Function):
-    """The whole prologue as ONE autograd node: the RMSNorm / conv kernel, the four projections
-    (one atlas_linear_batch launch), the head-split kernel, and in the backward their adjoints in
-    reverse order (the four input gradients in one launch) with the weight gradients of _wgrad.
-    One node and batched products keep the host's per-step work down (the prologue is bound by
-    host issue at C5's layer shape, not by its kernels)."""
-
-    @staticmethod
-    def forward(ctx, x, norm_w, wq, wk, wv, Wq, Wk, Wv, Wg, bg, qg, kg, conv_k, eps, heads, d):
-        cp, ch = _HandCtx(), _HandCtx()
-        conv = conv_k > 1
-        if conv:
-            xn, qi, ki, vi = _PrologueFn.forward(cp, x, norm_w, wq, wk, wv, conv_k, eps)
-        else:
-            xn = _PrologueFn.forward(cp, x, norm_w, None, None, None, 0, eps)
-            qi = ki = vi = xn
-        if Wg is not None:
-            ql, kl, vl, zl = _products(_GEMM_NT, [qi, ki, vi, xn], [Wq, Wk, Wv, Wg])
-        else:
-            (ql, kl, vl), zl = _products(_GEMM_NT, [qi, ki, vi], [Wq, Wk, Wv]), None
-        outs = _HeadsFn.forward(ch, ql, kl, vl, zl, qg, kg, bg, heads, d)
-        e0 = torch.empty(0, device=x.device)
-        ctx.save_for_backward(qi, ki, vi, xn, Wq, Wk, Wv, Wg if Wg is not None else e0)
-        ctx.cp, ctx.ch, ctx.conv, ctx.has_g = cp, ch, conv, Wg is not None
-        return (xn, *outs)
-
-    @staticmethod
-    def backward(ctx, dxn, dq, dk, dv, *dgates):
-        qi, ki, vi, xn, Wq, Wk, Wv, Wg = ctx.saved_tensors
-        dql, dkl, dvl, dzl, hparts = _HeadsFn.backward(ctx.ch, dq, dk, dv, *dgates)
-        if ctx.has_g:
-            dqi, dki, dvi, dxg = _products(_GEMM_NN, [dql, dkl, dvl, dzl], [Wq, Wk, Wv, Wg])
-        else:
-            dqi, dki, dvi = _products(_GEMM_NN, [dql, dkl, dvl], [Wq, Wk, Wv])
-        pairs = [(dql, qi), (dkl, ki), (dvl, vi)] + ([(dzl, xn)] if ctx.has_g else [])
-        dws = _wgrads(pairs, Wq.dtype)
-        dWq, dWk, dWv = dws[:3]
-        dWg = dws[3] if ctx.has_g else None
-        dsum = dxn
-        if ctx.has_g:
-            dsum = dxg if dsum is None else dsum + dxg
-        if ctx.conv:
-            dx, pparts = _PrologueFn.backward(ctx.cp, dsum, dqi, dki, dvi)
-        else:
-            dsum = dqi + dki + dvi + (dsum if dsum is not None else 0)
-            dx, pparts = _PrologueFn.backward(ctx.cp, dsum)
-        # every parameter gradient of the two kernels from their partials, in one launch
-        names = [n for n in ("qg", "kg", "b") if n in hparts]
-        sums = _sum_partials(pparts + [hparts[n] for n in names])
-        dnorm = sums[0]
-        dtq = dtk = dtv = None
-        if ctx.conv:
-            dtq, dtk, dtv = sums[1].unbind(0)
-        got = dict(zip(names, sums[len(pparts):]))
-        return (dx, dnorm, dtq, dtk, dtv, dWq, dWk, dWv, dWg, got.get("b"), got.get("qg"), got.get("kg"),
-                None, None, None, None)
+    """x W^T without bias: the product and its input gradient on atlas_linear_batch, the weight gradient
+    split over the tokens (_wgrads)."""
+    return _lib.native().linear(x, w)
 
 
 def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj_weights, gate_weights, gate_biases,
@@ -1223,21 +766,13 @@ def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj
     _require_gpu(x, norm_weight)
     if x.dim() != 3:
         raise ValueError(f"x must be [B, T, dim], got {tuple(x.shape)}")
-    dt = x.dtype
-    cast = lambda t: None if t is None else t.to(dt)
-    conv_k = 0
-    if conv_weights is not None:
-        conv_k = conv_weights[0].shape[-1]
-        if conv_k > 8:
-            raise ValueError("the fused prologue supports depthwise convolutions of up to 8 taps")
-    wq, wk, wv = (cast(w) for w in conv_weights) if conv_weights is not None else (None, None, None)
-    if conv_k <= 1:
-        wq = wk = wv = None
-    Wg = torch.cat([cast(w) for w in gate_weights], dim=0) if gate_weights else None
-    bias = torch.cat([cast(b) for b in gate_biases]).contiguous() if gate_weights else None
-    out = _CellPrologueFn.apply(x, norm_weight.to(dt).contiguous(), wq, wk, wv, cast(proj_weights[0]),
-                                cast(proj_weights[1]), cast(proj_weights[2]), Wg, bias, cast(q_gamma), cast(k_gamma),
-                                conv_k if conv_k > 1 else 0, eps, heads, dim_head)
+    _dt_code(x)   # fp32 or bf16
+    if conv_weights is not None and conv_weights[0].shape[-1] > 8:
+        raise ValueError("the fused prologue supports depthwise convolutions of up to 8 taps")
+    # one autograd node for all of it, with the products and weight gradients batched (csrc/host.cpp)
+    out = _lib.native().cell_prologue(x, norm_weight, float(eps), list(conv_weights) if conv_weights is not None else [],
+                                      list(proj_weights), list(gate_weights or ()), list(gate_biases or ()) if gate_weights
+                                      else [], q_gamma, k_gamma, heads, dim_head)
     return out[0], out[1], out[2], out[3], list(out[4:])
 
 

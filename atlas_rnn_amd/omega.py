@@ -22,8 +22,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .functional import (_DTYPES, AssocScan, _aligned, _ptr, _stream, assoc_scan, tensor_feature_map,
-                         window_sum)
+from .functional import AssocScan, assoc_scan, tensor_feature_map, window_sum
 
 __all__ = ["_sliding_sum_along_n", "assoc_scan", "AssocScan", "omega_store_chain", "apply_poly_features",
            "OmegaPolyFeatures", "OMEGA_GATE_OFF", "newtonschulz5"]
@@ -72,87 +71,11 @@ def newtonschulz5(t: Tensor, steps: int = 5, eps: float = 1e-7,
     return x.contiguous().to(dt)
 
 
-class _OmegaChainFn(torch.autograd.Function):
-    """omega_store_chain's chain in one kernel each way (atlas_omega_chain_fwd / _bwd): every tensor of
-    surprise's dtype and contiguous, surprise [BH, n, P]. Returns (update [BH, n+1, P], next momentum
-    [O, BH, P], next buffer [BH, e-1, P]); the last two are empty without momentum / a window."""
-
-    @staticmethod
-    def forward(ctx, surprise, decay, last_update, am, last_momentum, gate, buf, window):
-        ctx.set_materialize_grads(False)
-        lib = _lib.load()
-        BH, n, p = surprise.shape
-        O = 0 if am is None else am.shape[0]
-        new = lambda *shape: torch.empty(shape, device=surprise.device, dtype=surprise.dtype)
-        update = new(BH, n + 1, p)
-        moms = new(O, BH, n, p) if O and any(ctx.needs_input_grad) else None
-        next_lm = new(O, BH, p)
-        next_buf = new(BH, window - 1, p)
-        _lib.check(lib.atlas_omega_chain_fwd(
-            _DTYPES[surprise.dtype], BH, n, p, O, window, _ptr(surprise), _ptr(decay), _ptr(last_update), _ptr(am),
-            _ptr(last_momentum), _ptr(gate), _ptr(buf), _ptr(update), _ptr(moms), _ptr(next_lm if O else None),
-            _ptr(next_buf if window > 1 else None), _stream(surprise.device)), "atlas_omega_chain_fwd")
-        ctx.save_for_backward(surprise, decay, am, last_momentum, gate, update, moms)
-        ctx.window, ctx.has_buf = window, buf is not None
-        return update, next_lm, next_buf
-
-    @staticmethod
-    def backward(ctx, dup, dlm, dbuf_out):
-        lib = _lib.load()
-        surprise, decay, am, last_momentum, gate, update, moms = ctx.saved_tensors
-        BH, n, p = surprise.shape
-        O = 0 if am is None else am.shape[0]
-        e = ctx.window
-        dup, dlm, dbuf_out = (_aligned(g) if g is not None and g.numel() else None for g in (dup, dlm, dbuf_out))
-        like = lambda t: None if t is None else torch.empty_like(t)
-        ds, dd, dam, dlm0, dg = (like(t) for t in (surprise, decay, am, last_momentum, gate))
-        dlast = torch.empty(BH, p, device=surprise.device, dtype=surprise.dtype)
-        dbuf = torch.empty(BH, e - 1, p, device=surprise.device, dtype=surprise.dtype) if ctx.has_buf else None
-        nbytes = lib.atlas_omega_chain_workspace_bytes(BH, n, p, O)
-        ws = torch.empty((nbytes + 3) // 4, device=surprise.device, dtype=torch.float32)
-        _lib.check(lib.atlas_omega_chain_bwd(
-            _DTYPES[surprise.dtype], BH, n, p, O, e, _ptr(surprise), _ptr(decay), _ptr(am), _ptr(last_momentum),
-            _ptr(gate), _ptr(update), _ptr(moms), _ptr(dup), _ptr(dlm), _ptr(dbuf_out), _ptr(ds), _ptr(dd),
-            _ptr(dlast), _ptr(dam), _ptr(dlm0), _ptr(dg), _ptr(dbuf), _ptr(ws), nbytes, _stream(surprise.device)),
-            "atlas_omega_chain_bwd")
-        return ds, dd, dlast, dam, dlm0, dg, dbuf, None
-
-
 def _fused_chain(surprise, decay, last_update, am, last_momentum, gate, window, buf):
-    """The chain on _OmegaChainFn, or None where its kernels do not apply: one dtype (fp32 or bf16) on
-    one GPU for the surprises and the scalars, at most two momentum orders and a window of at most 16
-    (the kernels hold both in registers), and sizes inside their index ranges. The separate scans and
-    window sums serve everything else."""
-    dt, dev = surprise.dtype, surprise.device
-    if dt not in _DTYPES or not surprise.is_cuda or window > 16:
-        return None
-    tensors = [t for t in (decay, am, gate) if t is not None]
-    carried = [t for t in (last_update, last_momentum, buf) if t is not None]
-    if any(t.dtype != dt for t in tensors) or any(t.device != dev for t in tensors + carried):
-        return None
-    if (am is not None and not 1 <= am.shape[0] <= 2) or (am is None and last_momentum is not None):
-        return None
-    BH, n = surprise.shape[:2]
-    param = surprise.shape[2:]
-    if surprise.numel() == 0 or BH > 65535 or n > 1 << 24 or surprise.numel() // (BH * n) > 1 << 31:
-        return None
-    p = surprise.numel() // (BH * n)
-
-    def shaped(t, *shape):   # views only where the shape differs: each is a node of the autograd graph
-        return t if t.shape == shape else t.reshape(shape)
-
-    def flat(t, *lead):
-        return None if t is None else _aligned(shaped(t if t.dtype == dt else t.to(dt), *lead, p))
-
-    O = 0 if am is None else am.shape[0]
-    e = window
-    update, next_lm, next_buf = _OmegaChainFn.apply(
-        flat(surprise, BH, n), shaped(decay, BH, n).contiguous(), flat(last_update, BH),
-        None if am is None else shaped(am, O, BH, n).contiguous(), flat(last_momentum, O, BH),
-        None if gate is None else gate.contiguous(), flat(buf, BH, e - 1) if e > 1 else None, e)
-    update = shaped(update, BH, n + 1, *param)
-    return (update, update[:, -1], shaped(next_lm, O, BH, *param) if O else None,
-            shaped(next_buf, BH, e - 1, *param) if e > 1 else None)
+    """The chain in one kernel each way (atlas_omega_chain_fwd / _bwd), or None where they do not apply:
+    one dtype (fp32 or bf16) on one GPU for the surprises and the scalars, at most two momentum orders
+    and a window of at most 16. The separate scans and window sums serve everything else."""
+    return _lib.native().omega_chain(surprise, decay, last_update, am, last_momentum, gate, window, buf)
 
 
 def omega_store_chain(surprise: Tensor, decay_factor: Tensor, last_update: Tensor, *,
@@ -200,8 +123,7 @@ def omega_store_chain(surprise: Tensor, decay_factor: Tensor, last_update: Tenso
                     tuple(omega_buf.shape) == (BH, omega_window - 1, *surprise.shape[2:])):
                 fused = _fused_chain(surprise, decay_factor, last_update, adaptive_momentum,
                                      last_momentum if adaptive_momentum is not None else None,
-                                     omega_gate if omega_gate is None or omega_gate.shape == (BH, n) else
-                                     omega_gate.reshape(BH, n), omega_window,
+                                     omega_gate, omega_window,
                                      omega_buf if omega_window > 1 else None)
                 if fused is not None:
                     return fused
