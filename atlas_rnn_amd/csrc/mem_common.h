@@ -200,6 +200,79 @@ __device__ __forceinline__ typename MM<T>::frag frag_scale(typename MM<T>::frag 
   }
 }
 
+// Whole-K operands of a 16 x 16 tile product: every fragment of K values of a row (kop_row) or of a
+// transposed matrix (kop_tr) read up front, then K / KS products back to back. bf16 keeps the natural k
+// order. fp32 takes k = 16 jj + 4 (lane >> 4) + i at step 4 jj + i (a sum over k does not depend on its
+// order), so that a lane's values of a row are float4 reads: K / 16 LDS reads instead of K / 4, and with
+// a pitch of 16 n + 4 floats the transposed reads of the four lane groups fall on distinct banks.
+template <typename T, int K>
+struct KOp {
+  static constexpr int N = sizeof(T) == 2 ? K / 32 : K / 4;
+  typename MM<T>::frag f[N];
+};
+// LDS pitch padding that goes with them
+template <typename T> constexpr int kLdsPad = sizeof(T) == 2 ? 8 : 4;
+
+template <typename T, int K>
+__device__ __forceinline__ KOp<T, K> kop_row(const T* p, int ld, int r0) {
+  KOp<T, K> o;
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int q = 0; q < K / 32; ++q) o.f[q] = frag_ld_row<T>(p, ld, r0, 32 * q);
+  } else {
+    const int l = lane_id();
+    const T* q = p + (r0 + (l & 15)) * ld + 4 * (l >> 4);
+#pragma unroll
+    for (int j = 0; j < K / 16; ++j) {
+      const float4 v = *reinterpret_cast<const float4*>(q + 16 * j);
+      o.f[4 * j] = v.x; o.f[4 * j + 1] = v.y; o.f[4 * j + 2] = v.z; o.f[4 * j + 3] = v.w;
+    }
+  }
+  return o;
+}
+template <typename T, int K>
+__device__ __forceinline__ KOp<T, K> kop_tr(const T* p, int ld, int r0) {
+  KOp<T, K> o;
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int q = 0; q < K / 32; ++q) o.f[q] = frag_ld_tr<T>(p, ld, r0, 32 * q);
+  } else {
+    const int l = lane_id();
+    const T* q = p + 4 * (l >> 4) * ld + r0 + (l & 15);
+#pragma unroll
+    for (int j = 0; j < K / 16; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.f[4 * j + i] = q[(16 * j + i) * ld];
+  }
+  return o;
+}
+// the operand with each k value times w[k] (fp32)
+template <typename T, int K>
+__device__ __forceinline__ KOp<T, K> kop_scale(const KOp<T, K>& a, const float* w) {
+  KOp<T, K> o;
+  const int l = lane_id();
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int q = 0; q < K / 32; ++q)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o.f[q][e] = static_cast<T>(static_cast<float>(a.f[q][e]) * w[32 * q + 8 * (l >> 4) + e]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < K / 16; ++j) {
+      const float* v = w + 16 * j + 4 * (l >> 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.f[4 * j + i] = a.f[4 * j + i] * v[i];
+    }
+  }
+  return o;
+}
+template <typename T, int K>
+__device__ __forceinline__ f32x4 kop_mma(const KOp<T, K>& a, const KOp<T, K>& b, f32x4 c) {
+#pragma unroll
+  for (int q = 0; q < KOp<T, K>::N; ++q) c = MM<T>::mma(a.f[q], b.f[q], c);
+  return c;
+}
+
 // Sum over the 16 lanes of each row (lanes 16r .. 16r+15), returned in every lane of the row:
 // four DPP row rotations (row_ror 8, 4, 2, 1) on the VALU, no LDS traffic.
 __device__ __forceinline__ float row_sum16(float x) {

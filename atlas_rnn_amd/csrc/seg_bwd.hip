@@ -274,30 +274,30 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg_agg(const Geom g, const
 // ---------------------------------------------------------------------------------------------
 // main reverse walk
 // ---------------------------------------------------------------------------------------------
-template <typename T, int CH, int D>
+template <typename T, int CH, int D, int HP>
 struct BwdSegSmem {
-  static constexpr int SPM = CH + kHaloPad;
-  static constexpr bool kStatesInLds = sizeof(T) == 2;   // fp32 reads S_in / Z_in from the saved chunk states
+  static constexpr int SP = SrcRows<T, CH, HP>::SP, SPK = SrcRows<T, CH, HP>::SPK;
+  static constexpr int LD = D + kLdsPad<T>, LC = CH + kLdsPad<T>, LQ = SPK + kLdsPad<T>;   // pitches
   // adjoint at the chunk end and the chunk-start state, transposed: X^T[k][i] = X[i][k]
-  alignas(16) T sref[D][D + 8];
-  alignas(16) T dSeT[D][D + 8];
-  alignas(16) T dZeT[D][D + 8];
-  alignas(16) T SinT[kStatesInLds ? D : 1][D + 8];
-  alignas(16) T ZinT[kStatesInLds ? D : 1][D + 8];
-  T phi[SPM][D + 8];
-  T psi[CH][D + 8];
-  T dy[CH][D + 8];
-  T deltaT[SPM][D + 8];    // v_s staged by the loads, then delta^T[s][i]
+  alignas(16) T sref[D][LD];
+  alignas(16) T dSeT[D][LD];
+  alignas(16) T dZeT[D][LD];
+  alignas(16) T SinT[D][LD];
+  alignas(16) T ZinT[D][LD];
+  T phi[SPK][LD];
+  T psi[CH][LD];
+  T dy[CH][LD];
+  T deltaT[SP][LD];        // v_s staged by the loads, then delta^T[s][i]
   struct {
-    T QT[SPM][CH + 8];   // Q^T[s][q],  Q[q][s] = Ws[s, q-1] (psi_q . phi_s)
-    T Qp[CH][SPM + 8];   // Q'[q][s] = Ws[s, q-1] (dy_q . delta_s)
-    T QpT[SPM][CH + 8];
-    alignas(16) T dDT[SPM][D + 8];   // dDelta^T[s][i]
+    T QT[SP][LC];          // Q^T[s][q],  Q[q][s] = Ws[s, q-1] (psi_q . phi_s)
+    T Qp[CH][LQ];          // Q'[q][s] = Ws[s, q-1] (dy_q . delta_s)
+    T QpT[SP][LC];
+    alignas(16) T dDT[SPK][LD];   // dDelta^T[s][i]
   } g;
-  T wsh[CH][SPM + 8];      // Ws[s, tau-1]
-  float Lm[CH][SPM + 1];   // (dy_q . delta_s)(psi_q . phi_s)
+  T wsh[CH][LQ];           // Ws[s, tau-1]
+  float Lm[CH][SP + 1];    // (dy_q . delta_s)(psi_q . phi_s)
   ChunkScalars<CH> sc;
-  float hS[SPM], hZ[SPM], fS[CH], fZ[CH];
+  float hS[CH + kHaloPad], hZ[CH + kHaloPad], fS[CH], fZ[CH];
   float gram[4];
   float red[kSegWaves][4][4];   // per wave and lane row: partial Grams
   // followed by the halo carry: float carry[2][H][2 * D] (dynamic size)
@@ -307,15 +307,15 @@ struct BwdSegSmem {
 // the sources, q, dy of the targets, the scalars and gates, the coefficient record, the Ws[s, t-1]
 // block and the saved chunk-start state tiles of this wave. Every load is unconditional from
 // an in-bounds address; masks are applied in store().
-template <typename T, int CH, int D>
+template <typename T, int CH, int D, int HP>
 struct BwdPrefetch {
-  static constexpr int SPM = CH + kHaloPad;
+  static constexpr int SPM = CH + kHaloPad, SP = CH + HP;
   static constexpr int NTD = D / 16;
   static constexpr int NT2 = (NTD * NTD + kSegWaves - 1) / kSegWaves;
-  static constexpr int NVS = (SPM * (D / 8) + kSegThreads - 1) / kSegThreads;
+  static constexpr int NVS = (SP * (D / 8) + kSegThreads - 1) / kSegThreads;
   static constexpr int NVT = (CH * (D / 8) + kSegThreads - 1) / kSegThreads;
   static constexpr int REC4 = CoefRec<CH>::SIZE / 4;
-  static constexpr int NV_WSH = (CH * SPM / 8 + kSegThreads - 1) / kSegThreads;
+  static constexpr int NV_WSH = (CH * SP / 8 + kSegThreads - 1) / kSegThreads;
   Vec8<T> rk[NVS], rv[NVS], rq[NVT], rd[NVT], wsv[NV_WSH];
   float rc0, rc1, rc2, rc3;
   unsigned okS, okT;
@@ -333,7 +333,7 @@ struct BwdPrefetch {
       const int idx = tid + j * kSegThreads;
       const int s = idx / (D / 8), c8 = idx % (D / 8);
       const int pp = t0 - H + s;
-      const bool ok = s < SPM && s < H + L && pp >= 0;
+      const bool ok = s < SP && s < H + L && pp >= 0;
       const size_t row = ok ? tb + pp : r0;
       rk[j] = vec8_load(a.k + row * D + c8 * 8);
       rv[j] = vec8_load(a.v + row * D + c8 * 8);
@@ -357,8 +357,8 @@ struct BwdPrefetch {
     const T* wsh_c = reinterpret_cast<const T*>(p.wsh) + ((size_t)bh * g.nc + c) * CH * SPM;
 #pragma unroll
     for (int j = 0; j < NV_WSH; ++j) {
-      const int v = tid + j * kSegThreads;
-      wsv[j] = vec8_load(wsh_c + (size_t)(v < CH * SPM / 8 ? v : 0) * 8);
+      const int v = tid + j * kSegThreads, vc = v < CH * SP / 8 ? v : 0;
+      wsv[j] = vec8_load(wsh_c + (size_t)(vc / (SP / 8)) * SPM + (vc % (SP / 8)) * 8);
     }
     const float* Zin_g = Sin_g + (size_t)D * D;
 #pragma unroll
@@ -380,7 +380,7 @@ struct BwdPrefetch {
     for (int j = 0; j < NVS; ++j) {
       const int idx = tid + j * kSegThreads;
       const int s = idx / (D / 8), c8 = idx % (D / 8);
-      if (s < SPM) {
+      if (s < SP) {
         const bool ok = (okS >> j) & 1u;
         Vec8<T> x = rk[j].masked(ok);
         if (g.map_mode == MAP_ELEMENTWISE) x = x.mapped(g.map_deg);
@@ -404,28 +404,27 @@ struct BwdPrefetch {
 #pragma unroll
     for (int j = 0; j < NV_WSH; ++j) {
       const int v = tid + j * kSegThreads;
-      if (v < CH * SPM / 8) wsv[j].store(&sm.wsh[(v * 8) / SPM][(v * 8) % SPM]);
+      if (v < CH * SP / 8) wsv[j].store(&sm.wsh[v / (SP / 8)][(v % (SP / 8)) * 8]);
     }
     if (tid < CH) { sm.fS[tid] = 0.f; sm.fZ[tid] = 0.f; }
     for (int s = tid; s < SPM; s += kSegThreads) { sm.hS[s] = 0.f; sm.hZ[s] = 0.f; }
   }
 };
 
-template <typename T, int CH, int D>
+template <typename T, int CH, int D, int HP>
 __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const BwdPtrs<T> a, const SegGeom sg,
                                                            const BwdSegPtrs p) {
   if (geom_skip(g)) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  typedef BwdSegSmem<T, CH, D> Sm;
-  constexpr int SPM = Sm::SPM;
-  constexpr bool SIL = Sm::kStatesInLds;
+  typedef BwdSegSmem<T, CH, D, HP> Sm;
+  constexpr int SPM = CH + kHaloPad, SP = Sm::SP, SPK = Sm::SPK, LD = Sm::LD, LC = Sm::LC, LQ = Sm::LQ;
   constexpr int NTD = D / 16;
   constexpr int NT2 = (NTD * NTD + kSegWaves - 1) / kSegWaves;   // owned state tiles per wave
   typedef MM<T> M;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int seg = blockIdx.x, bh = blockIdx.y;
   const int H = g.H, e = g.e;
-  constexpr int NTS = SPM / 16, NTC = CH / 16;
+  constexpr int NTS = SP / 16, NTC = CH / 16;
   static_assert(SPM <= 64, "backward source tile: coefficient lanes 0..63, decay columns 64..64+CH");
   const size_t tb = (size_t)bh * g.T;
   const size_t sb = (size_t)bh * D * D;
@@ -458,9 +457,17 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
   float* carry = reinterpret_cast<float*>(smem_raw + carry_offset<Sm>());   // [2][H][2D], 16-byte aligned
   for (int idx = tid; idx < D * D; idx += kSegThreads) sm.sref[idx / D][idx % D] = from_f32<T>(a.S_ref[sb + idx]);
   for (int idx = tid; idx < 2 * H * 2 * D; idx += kSegThreads) carry[idx] = 0.f;
+  if constexpr (SPK > SP) {   // the source rows past SP: zeros, never written again
+    for (int idx = tid; idx < (SPK - SP) * D; idx += kSegThreads) {
+      sm.phi[SP + idx / D][idx % D] = from_f32<T>(0.f);
+      sm.g.dDT[SP + idx / D][idx % D] = from_f32<T>(0.f);
+    }
+    for (int idx = tid; idx < CH * (SPK - SP); idx += kSegThreads)
+      sm.g.Qp[idx / (SPK - SP)][SP + idx % (SPK - SP)] = from_f32<T>(0.f);
+  }
 
   // ---- 3. reverse walk
-  BwdPrefetch<T, CH, D> pf;
+  BwdPrefetch<T, CH, D, HP> pf;
   if (c_begin < c_end) pf.load(g, a, p, bh, c_end - 1, rw + (size_t)(c_end - 1) * 2 * D * D, tid, lane, wave);
   for (int c = c_end - 1; c >= c_begin; --c) {
     // per-lane indices re-derived every chunk: keeps the compiler from hoisting every per-lane
@@ -498,10 +505,8 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         // rows i0..i0+3 of column k are contiguous in the transposed copies
         store4<T>(&sm.dSeT[k][i0], dS[j][0], dS[j][1], dS[j][2], dS[j][3]);
         store4<T>(&sm.dZeT[k][i0], dZ[j][0], dZ[j][1], dZ[j][2], dZ[j][3]);
-        if constexpr (SIL) {
-          store4<T>(&sm.SinT[k][i0], sv[0], sv[1], sv[2], sv[3]);
-          store4<T>(&sm.ZinT[k][i0], zv[0], zv[1], zv[2], zv[3]);
-        }
+        store4<T>(&sm.SinT[k][i0], sv[0], sv[1], sv[2], sv[3]);
+        store4<T>(&sm.ZinT[k][i0], zv[0], zv[1], zv[2], zv[3]);
       }
       gss = row_sum16(gss); gsz = row_sum16(gsz); gzz = row_sum16(gzz);
       if ((lane & 15) == 0) {
@@ -550,10 +555,7 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NT1 - 1);
         const bool valid = NT1 % kSegWaves == 0 || wave + kSegWaves * j < NT1;
         const int m0 = (tile % NTD) * 16, n0 = (tile / NTD) * 16;   // m: rows i, n: sources s
-        f32x4 acc = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS)
-          acc = M::mma(frag_ld_row<T>(&sm.sref[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.phi[0][0], D + 8, n0, k0), acc);
+        const f32x4 acc = kop_mma(kop_row<T, D>(&sm.sref[0][0], LD, m0), kop_row<T, D>(&sm.phi[0][0], LD, n0), zero4());
         if (valid) {
           const int s = n0 + (lane & 15), i0 = m0 + 4 * (lane >> 4);
           const int pp = t0 - H + s;
@@ -574,12 +576,8 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NTQ - 1);
         const bool valid = NTQ % kSegWaves == 0 || wave + kSegWaves * j < NTQ;
         const int m0 = (tile / NTS) * 16, n0 = (tile % NTS) * 16;
-        f32x4 kk = zero4(), k3 = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS) {
-          kk = M::mma(frag_ld_row<T>(&sm.psi[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.phi[0][0], D + 8, n0, k0), kk);
-          k3 = M::mma(frag_ld_row<T>(&sm.dy[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.deltaT[0][0], D + 8, n0, k0), k3);
-        }
+        const f32x4 kk = kop_mma(kop_row<T, D>(&sm.psi[0][0], LD, m0), kop_row<T, D>(&sm.phi[0][0], LD, n0), zero4());
+        const f32x4 k3 = kop_mma(kop_row<T, D>(&sm.dy[0][0], LD, m0), kop_row<T, D>(&sm.deltaT[0][0], LD, n0), zero4());
         if (valid) {
           const int s = n0 + (lane & 15);
 #pragma unroll
@@ -605,16 +603,10 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NT4 - 1);
         const bool valid = NT4 % kSegWaves == 0 || wave + kSegWaves * j < NT4;
         const int m0 = (tile / NTS) * 16, n0 = (tile % NTS) * 16;
-        f32x4 az = zero4(), as = zero4(), aq = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS) {
-          const typename M::frag fb = frag_ld_row<T>(&sm.phi[0][0], D + 8, n0, k0);
-          as = M::mma(frag_ld_tr<T>(&sm.dSeT[0][0], D + 8, m0, k0), fb, as);
-          az = M::mma(frag_ld_tr<T>(&sm.dZeT[0][0], D + 8, m0, k0), fb, az);
-        }
-#pragma unroll
-        for (int k0 = 0; k0 < CH; k0 += M::KS)
-          aq = M::mma(frag_ld_tr<T>(&sm.dy[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.g.QT[0][0], CH + 8, n0, k0), aq);
+        const KOp<T, D> fb = kop_row<T, D>(&sm.phi[0][0], LD, n0);
+        const f32x4 as = kop_mma(kop_tr<T, D>(&sm.dSeT[0][0], LD, m0), fb, zero4());
+        const f32x4 az = kop_mma(kop_tr<T, D>(&sm.dZeT[0][0], LD, m0), fb, zero4());
+        const f32x4 aq = kop_mma(kop_tr<T, CH>(&sm.dy[0][0], LD, m0), kop_row<T, CH>(&sm.g.QT[0][0], LC, n0), zero4());
         if (valid) {
           const int s = n0 + (lane & 15);
           const float wz = sm.sc.wzend[s], ws = sm.sc.wsend[s];
@@ -643,34 +635,10 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NT7 - 1);
         const bool valid = NT7 % kSegWaves == 0 || wave + kSegWaves * j < NT7;
         const int m0 = (tile % NTD) * 16, n0 = (tile / NTD) * 16;   // m: features k, n: targets q
-        f32x4 as = zero4(), az = zero4(), aq = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS) {
-          const typename M::frag fb = frag_ld_row<T>(&sm.dy[0][0], D + 8, n0, k0);
-          if constexpr (SIL) {
-            as = M::mma(frag_ld_row<T>(&sm.SinT[0][0], D + 8, m0, k0), fb, as);
-            az = M::mma(frag_ld_row<T>(&sm.ZinT[0][0], D + 8, m0, k0), fb, az);
-          } else {   // S_in[i][k] straight from the saved fp32 state (16 consecutive k per row i)
-            typename M::frag fs;
-            {
-              const int kb = k0 + (lane >> 4) * M::KL;
-              const float* q = Sin_g + (size_t)kb * D + m0 + (lane & 15);
-              if constexpr (M::KL == 1) fs = static_cast<T>(clamp_in ? clamp100(q[0]) : q[0]);
-              else {
-#pragma unroll
-                for (int ee = 0; ee < M::KL; ++ee) {
-                  const float x = q[(size_t)ee * D];
-                  fs[ee] = static_cast<T>(clamp_in ? clamp100(x) : x);
-                }
-              }
-            }
-            as = M::mma(fs, fb, as);
-            az = M::mma(frag_ld_or_zero<T>(g.momentum ? Zin_g : nullptr, 1, D, m0, k0), fb, az);
-          }
-        }
-#pragma unroll
-        for (int k0 = 0; k0 < SPM; k0 += M::KS)
-          aq = M::mma(frag_ld_tr<T>(&sm.phi[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.g.Qp[0][0], SPM + 8, n0, k0), aq);
+        const KOp<T, D> fb = kop_row<T, D>(&sm.dy[0][0], LD, n0);
+        const f32x4 as = kop_mma(kop_row<T, D>(&sm.SinT[0][0], LD, m0), fb, zero4());
+        const f32x4 az = kop_mma(kop_row<T, D>(&sm.ZinT[0][0], LD, m0), fb, zero4());
+        const f32x4 aq = kop_mma(kop_tr<T, SPK>(&sm.phi[0][0], LD, m0), kop_row<T, SPK>(&sm.g.Qp[0][0], LQ, n0), zero4());
         const int t = n0 + (lane & 15), kq = m0 + 4 * (lane >> 4);
         const float ac = sm.sc.acoef[t], kc = sm.sc.kcoef[t];
         float ps[4], dpsi[4], fsp = 0.f, fzp = 0.f;
@@ -687,7 +655,7 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
             f32x4 ab = zero4();
 #pragma unroll
             for (int k0 = 0; k0 < D; k0 += M::KS)
-              ab = M::mma(frag_ld<T>(Bs, 1, D, m0, k0), frag_ld_row<T>(&sm.dy[0][0], D + 8, n0, k0), ab);
+              ab = M::mma(frag_ld<T>(Bs, 1, D, m0, k0), frag_ld_row<T>(&sm.dy[0][0], LD, n0, k0), ab);
             const float w = to_f32(sm.wsh[t][s]);
             float lm = 0.f;
 #pragma unroll
@@ -750,10 +718,7 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
     for (int j = 0; j < NT2; ++j) {   // G6: dS_ref[i, k] += sum_s dDelta[i, s] phi_s[k]
       const int tile = min(wave + kSegWaves * j, NTD * NTD - 1);
       const int m0 = (tile / NTD) * 16, n0 = (tile % NTD) * 16;
-      f32x4 acc = zero4();
-#pragma unroll
-      for (int k0 = 0; k0 < SPM; k0 += M::KS)
-        acc = M::mma(frag_ld_tr<T>(&sm.g.dDT[0][0], D + 8, m0, k0), frag_ld_tr<T>(&sm.phi[0][0], D + 8, n0, k0), acc);
+      const f32x4 acc = kop_mma(kop_tr<T, SPK>(&sm.g.dDT[0][0], LD, m0), kop_tr<T, SPK>(&sm.phi[0][0], LD, n0), zero4());
 #pragma unroll
       for (int r = 0; r < 4; ++r) dsr[j][r] += acc[r];
     }
@@ -777,7 +742,7 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
               for (int ee = 0; ee < M::KL; ++ee)
                 fa[ee] = static_cast<T>(to_f32(sm.dy[qb + ee][i]) * to_f32(sm.wsh[qb + ee][s]));
             }
-            acc = M::mma(fa, frag_ld_tr<T>(&sm.psi[0][0], D + 8, n0, k0), acc);
+            acc = M::mma(fa, frag_ld_tr<T>(&sm.psi[0][0], LD, n0, k0), acc);
           }
           if (valid) {
 #pragma unroll
@@ -799,17 +764,11 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NT5 - 1);
         const bool valid = NT5 % kSegWaves == 0 || wave + kSegWaves * j < NT5;
         const int m0 = (tile % NTD) * 16, n0 = (tile / NTD) * 16;   // m: features k, n: sources s
-        f32x4 a1 = zero4(), a2 = zero4(), a3 = zero4(), a4 = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS) {
-          const typename M::frag fb = frag_ld_row<T>(&sm.deltaT[0][0], D + 8, n0, k0);
-          a1 = M::mma(frag_ld_row<T>(&sm.dZeT[0][0], D + 8, m0, k0), fb, a1);
-          a2 = M::mma(frag_ld_row<T>(&sm.dSeT[0][0], D + 8, m0, k0), fb, a2);
-          a4 = M::mma(frag_ld_tr<T>(&sm.sref[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.g.dDT[0][0], D + 8, n0, k0), a4);
-        }
-#pragma unroll
-        for (int k0 = 0; k0 < CH; k0 += M::KS)
-          a3 = M::mma(frag_ld_tr<T>(&sm.psi[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.g.QpT[0][0], CH + 8, n0, k0), a3);
+        const KOp<T, D> fb = kop_row<T, D>(&sm.deltaT[0][0], LD, n0);
+        const f32x4 a1 = kop_mma(kop_row<T, D>(&sm.dZeT[0][0], LD, m0), fb, zero4());
+        const f32x4 a2 = kop_mma(kop_row<T, D>(&sm.dSeT[0][0], LD, m0), fb, zero4());
+        const f32x4 a4 = kop_mma(kop_tr<T, D>(&sm.sref[0][0], LD, m0), kop_row<T, D>(&sm.g.dDT[0][0], LD, n0), zero4());
+        const f32x4 a3 = kop_mma(kop_tr<T, CH>(&sm.psi[0][0], LD, m0), kop_row<T, CH>(&sm.g.QpT[0][0], LC, n0), zero4());
         const int s = n0 + (lane & 15), kq = m0 + 4 * (lane >> 4);
         const int pp = t0 - H + s;
         if (valid && s < H + L && pp >= 0) {
@@ -850,13 +809,8 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
         const int tile = min(wave + kSegWaves * j, NTD * NTD - 1);
         const bool valid = (NTD * NTD) % kSegWaves == 0 || wave + kSegWaves * j < NTD * NTD;
         const int m0 = (tile / NTD) * 16, n0 = (tile % NTD) * 16;
-        f32x4 aa = zero4(), ak = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < CH; k0 += M::KS) {
-          const typename M::frag fb = frag_ld_tr<T>(&sm.psi[0][0], D + 8, n0, k0);
-          aa = M::mma(frag_ld_tr_kscaled<T>(&sm.dy[0][0], D + 8, m0, k0, sm.sc.acoef), fb, aa);
-          ak = M::mma(frag_ld_tr_kscaled<T>(&sm.dy[0][0], D + 8, m0, k0, sm.sc.kcoef), fb, ak);
-        }
+        const KOp<T, CH> fb = kop_tr<T, CH>(&sm.psi[0][0], LD, n0), fy = kop_tr<T, CH>(&sm.dy[0][0], LD, m0);
+        const f32x4 aa = kop_mma(kop_scale(fy, sm.sc.acoef), fb, zero4()), ak = kop_mma(kop_scale(fy, sm.sc.kcoef), fb, zero4());
         if (valid) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -880,7 +834,7 @@ __global__ __launch_bounds__(kSegThreads) void k_bwd_seg(const Geom g, const Bwd
     {
       typedef ScalarBlock<CH> SB;
       float* blk = p.scal + ((size_t)bh * g.nc + c) * SB::SIZE;
-      for (int idx = tid; idx < CH * SPM; idx += kSegThreads) blk[SB::LM + idx] = sm.Lm[idx / SPM][idx % SPM];
+      for (int idx = tid; idx < CH * SPM; idx += kSegThreads) blk[SB::LM + idx] = idx % SPM < SP ? sm.Lm[idx / SPM][idx % SPM] : 0.f;
       for (int idx = tid; idx < SPM; idx += kSegThreads) { blk[SB::HS + idx] = sm.hS[idx]; blk[SB::HZ + idx] = sm.hZ[idx]; }
       if (tid < CH) { blk[SB::FS + tid] = sm.fS[tid]; blk[SB::FZ + tid] = sm.fZ[tid]; }
       if (tid < 4) blk[SB::GRAM + tid] = tid < 3 ? sm.gram[tid] : 0.f;
@@ -966,9 +920,16 @@ __global__ __launch_bounds__(kThreads) void k_seg_reduce_dsref(const Geom g, int
   out[(size_t)bh * n + idx] = acc;
 }
 
-template <typename T, int CH, int D>
-size_t bwd_seg_smem_bytes(int H) {
-  return carry_offset<BwdSegSmem<T, CH, D>>() + (size_t)2 * H * 2 * D * sizeof(float);
+template <typename T, int CH, int D, int HP>
+static hipError_t launch_bwd_walk(const Geom& g, const BwdPtrs<T>& a, const SegGeom& sg, const BwdSegPtrs& p,
+                                  hipStream_t stream) {
+  typedef BwdSegSmem<T, CH, D, HP> Sm;
+  static_assert(carry_offset<Sm>() + 2 * HP * 2 * D * sizeof(float) <= 160 * 1024, "one workgroup's LDS");
+  const size_t smem = carry_offset<Sm>() + (size_t)2 * g.H * 2 * D * sizeof(float);
+  const hipError_t err = set_dyn_smem(reinterpret_cast<const void*>(&k_bwd_seg<T, CH, D, HP>), smem);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((k_bwd_seg<T, CH, D, HP>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg, p);
+  return hipGetLastError();
 }
 
 hipError_t launch_walk_bwd_kernel(const Geom& g, const BwdPtrs<bf16>& a, const SegGeom& sg, const BwdSegPtrs& p,
@@ -1030,14 +991,17 @@ hipError_t launch_bwd_seg(const Geom& g, const BwdPtrs<T>& a, const SegGeom& sg,
     }
   }
   if (!walk) {
-    const size_t smem = bwd_seg_smem_bytes<T, CH, D>(g.H);
-    err = set_dyn_smem(reinterpret_cast<const void*>(&k_bwd_seg<T, CH, D>), smem);
-    if (err != hipSuccess) return err;
     prof_name(KID_BWD_CHUNK, "k_bwd_seg");
     prof_begin(KID_BWD_CHUNK, stream);
-    hipLaunchKernelGGL((k_bwd_seg<T, CH, D>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg, p);
+    // Windows up to 17 span a halo of 16 source slots, longer ones 32 (bf16 only: an fp32 call's chunks
+    // of 16 tokens bound its window). fp32 d = 64 e = 4 (32 rows of 1024 tokens): 213 us with 32 slots
+    // and the chunk-start states read from memory inside the products; with 16 slots the states fit in
+    // LDS and the operands are float4 reads: 106 us.
+    err = hipErrorInvalidValue;
+    if (g.H <= 16) err = launch_bwd_walk<T, CH, D, 16>(g, a, sg, p, stream);
+    else if constexpr (sizeof(T) == 2) err = launch_bwd_walk<T, CH, D, 32>(g, a, sg, p, stream);
     prof_end(KID_BWD_CHUNK, stream);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if (err != hipSuccess) return err;
   }
   // the specialised path runs the fixup inside the scalar-chain launch when the two are independent
   // (no token gates, whose gradients the fixup forms from the chains' output; no buffer_out gradient)
@@ -1069,8 +1033,7 @@ hipError_t launch_bwd_seg(const Geom& g, const BwdPtrs<T>& a, const SegGeom& sg,
 
 #define ATLAS_INST_BWD_SEG(T, CH, D)                                                                  \
   template hipError_t launch_bwd_seg<T, CH, D>(const Geom&, const BwdPtrs<T>&, const SegGeom&,        \
-                                               const BwdSegPtrs&, hipStream_t, bool, const AggOverFwd*); \
-  template size_t bwd_seg_smem_bytes<T, CH, D>(int);
+                                               const BwdSegPtrs&, hipStream_t, bool, const AggOverFwd*);
 
 ATLAS_INST_BWD_SEG(bf16, 32, 64)
 ATLAS_INST_BWD_SEG(float, 16, 64)

@@ -69,6 +69,16 @@ struct ScalarBlock {
   static_assert(SIZE % 4 == 0, "16-byte aligned blocks");
 };
 
+// Source rows a chunk's products span in the general kernels: the chunk's tokens and a halo of HP = 16
+// (windows up to 17) or 32 slots. Products over the sources run over SPK rows (bf16: whole 32-wide k
+// steps); the rows past SP hold zeros. The records in memory keep the pitch CH + kHaloPad.
+template <typename T, int CH, int HP>
+struct SrcRows {
+  static constexpr int SP = CH + HP;
+  static constexpr int SPK = sizeof(T) == 2 ? (SP + 31) / 32 * 32 : SP;
+  static_assert(SP % 16 == 0 && HP <= kHaloPad, "whole tiles of sources");
+};
+
 // Window weight of the source t - j for target t: the token gate of the source, the lag gate
 // w[t][j], or 1.
 __device__ __forceinline__ float src_w(int gate_mode, float ug, const float* wl, int e, int t, int j) {

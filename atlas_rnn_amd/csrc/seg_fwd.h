@@ -2,8 +2,8 @@
 //
 // Every chunk is a handful of small GEMMs separated by workgroup barriers; with 8 waves per CU the
 // barriers and LDS latency, not the matrix cores, set the pace. All tile counts and k extents are
-// therefore compile-time (the source tile always spans SPM = CH + 32 rows, padded rows are zero)
-// so that each wave's fragment loads are issued together ahead of its MFMA chains.
+// therefore compile-time (the source tile spans CH + 16 or CH + 32 rows by the window, padded rows are
+// zero) so that each wave's fragment loads are issued together ahead of its MFMA chains.
 #pragma once
 
 #include "mem_common.h"
@@ -12,19 +12,20 @@
 
 namespace atlas {
 
-template <typename T, int CH, int D, bool FULL>
+template <typename T, int CH, int D, int HP, bool FULL>
 struct SegFwdSmem {
-  static constexpr int SPM = CH + kHaloPad;
-  alignas(16) T phi[SPM][D + 8];   // phi[s][k]
-  alignas(16) T vd[SPM][D + 8];    // v[s][i] staged by the loads, then delta[s][i]
-  alignas(16) T sref[D][D + 8];
+  static constexpr int SP = SrcRows<T, CH, HP>::SP, SPK = SrcRows<T, CH, HP>::SPK;
+  static constexpr int LD = D + kLdsPad<T>, LQ = SPK + kLdsPad<T>;   // pitches
+  alignas(16) T phi[SPK][LD];      // phi[s][k]
+  alignas(16) T vd[SPK][LD];       // v[s][i] staged by the loads, then delta[s][i]
+  alignas(16) T sref[D][LD];
   ChunkScalars<CH> sc;
   // full walk only
-  T psi[FULL ? CH : 1][D + 8];
-  T Q[FULL ? CH : 1][SPM + 8];
-  T Sb[FULL ? D : 1][D + 8];
-  T Zb[FULL ? D : 1][D + 8];
-  T wsh[FULL ? CH : 1][SPM + 8];       // Ws[s, tau-1]
+  T psi[FULL ? CH : 1][LD];
+  T Q[FULL ? CH : 1][LQ];
+  T Sb[FULL ? D : 1][LD];
+  T Zb[FULL ? D : 1][LD];
+  T wsh[FULL ? CH : 1][LQ];        // Ws[s, tau-1]
 };
 
 // Per-thread register prefetch of one chunk's inputs (issued one chunk ahead).
@@ -32,31 +33,27 @@ struct SegFwdSmem {
 // chunk's first token, absent optional inputs to `decay`); the raw values are kept with validity
 // flags and only converted and masked in store(). A load under a condition whose value is
 // converted inside the same branch would make the wave wait for each load in turn.
-template <typename T, int CH, int D, bool FULL>
+template <typename T, int CH, int D, int HP, bool FULL>
 struct ChunkPrefetch {
-  static constexpr int SPM = CH + kHaloPad;
-  static constexpr int NV_PHI = (SPM * D / 8 + kSegThreads - 1) / kSegThreads;
+  static constexpr int SPM = CH + kHaloPad, SP = CH + HP;
+  static constexpr int NV_PHI = (SP * D / 8 + kSegThreads - 1) / kSegThreads;
   static constexpr int NV_PSI = FULL ? (CH * D / 8 + kSegThreads - 1) / kSegThreads : 0;
-  static constexpr int NWL = (CH * kMaxWindow + kSegThreads - 1) / kSegThreads;
   static constexpr int REC4 = CoefRec<CH>::SIZE / 4;
-  static constexpr int NV_WSH = FULL ? (CH * SPM / 8 + kSegThreads - 1) / kSegThreads : 0;
-  static_assert(REC4 <= kSegThreads && SPM % 8 == 0, "record / wsh prefetch");
+  static constexpr int NV_WSH = FULL ? (CH * SP / 8 + kSegThreads - 1) / kSegThreads : 0;
+  static_assert(REC4 <= kSegThreads && SP % 8 == 0, "record / wsh prefetch");
   Vec8<T> phi[NV_PHI];
   Vec8<T> vv[NV_PHI];
   Vec8<T> psi[NV_PSI > 0 ? NV_PSI : 1];
   Vec8<T> wsv[NV_WSH > 0 ? NV_WSH : 1];
   float rc0, rc1, rc2, rc3;   // this thread's float4 of the coefficient record
-  T alpha, eta, beta, ug;
-  T wl[NWL];
-  unsigned ok_phi, ok_psi, ok_wl;
-  bool ok_t, ok_ug, pad_ug;
+  unsigned ok_phi, ok_psi;
 
   // rec_c / wsh_c: this chunk's coefficient record and Ws[s, t-1] block (k_chunk_coef)
   __device__ __forceinline__ void load(const Geom& g, const FwdPtrs<T>& a, size_t tb, int t0, int L,
                                        const float* rec_c, const T* wsh_c) {
     const int tid = threadIdx.x, H = g.H;
     const size_t r0 = tb + t0;                          // always a valid token row
-    ok_phi = 0; ok_psi = 0; ok_wl = 0;
+    ok_phi = 0; ok_psi = 0;
     {
       const float4 r4 = reinterpret_cast<const float4*>(rec_c)[tid < REC4 ? tid : 0];
       rc0 = r4.x; rc1 = r4.y; rc2 = r4.z; rc3 = r4.w;
@@ -64,8 +61,8 @@ struct ChunkPrefetch {
     if constexpr (FULL) {
 #pragma unroll
       for (int j = 0; j < NV_WSH; ++j) {
-        const int v = tid + j * kSegThreads;
-        wsv[j] = vec8_load(wsh_c + (size_t)(v < CH * SPM / 8 ? v : 0) * 8);
+        const int v = tid + j * kSegThreads, vc = v < CH * SP / 8 ? v : 0;
+        wsv[j] = vec8_load(wsh_c + (size_t)(vc / (SP / 8)) * SPM + (vc % (SP / 8)) * 8);
       }
     }
 #pragma unroll
@@ -74,7 +71,7 @@ struct ChunkPrefetch {
       {   // phi and v: 8 consecutive features of source s per lane
         const int s = v / (D / 8), c8 = v % (D / 8);
         const int p = t0 - H + s;
-        const bool ok = s < SPM && s < H + L && p >= 0;
+        const bool ok = s < SP && s < H + L && p >= 0;
         const size_t off = (ok ? tb + p : r0) * D + c8 * 8;
         phi[j] = vec8_load(a.k + off);
         vv[j] = vec8_load(a.v + off);
@@ -91,26 +88,6 @@ struct ChunkPrefetch {
         ok_psi |= (ok ? 1u : 0u) << j;
       }
     }
-    ok_t = tid < L;
-    const size_t rt = ok_t ? r0 + tid : r0;
-    alpha = a.decay[rt];
-    eta = a.lr[rt];
-    const T* bp = (g.momentum && a.beta) ? a.beta : a.decay;
-    beta = bp[rt];
-    const T* gp = a.gate ? a.gate : a.decay;
-    {
-      const int p = t0 - H + tid;
-      ok_ug = g.gate_mode == GATE_TOKEN && tid < SPM && tid < H + L && p >= 0;
-      pad_ug = g.gate_mode == GATE_TOKEN && tid < SPM && tid < H + L && p < 0;
-      ug = gp[ok_ug ? tb + p : r0];
-    }
-#pragma unroll
-    for (int j = 0; j < NWL; ++j) {
-      const int idx = tid + j * kSegThreads;
-      const bool ok = g.gate_mode == GATE_LAG && idx < CH * g.e && idx / g.e < L;
-      wl[j] = gp[ok ? r0 * g.e + idx : r0];
-      ok_wl |= (ok ? 1u : 0u) << j;
-    }
   }
 
   template <typename Sm>
@@ -120,7 +97,7 @@ struct ChunkPrefetch {
     for (int j = 0; j < NV_PHI; ++j) {
       const int v = tid + j * kSegThreads;
       const int s = v / (D / 8), c8 = v % (D / 8);
-      if (s < SPM) {
+      if (s < SP) {
         const bool ok = (ok_phi >> j) & 1u;
         Vec8<T> x = phi[j].masked(ok);
         if (g.map_mode == MAP_ELEMENTWISE) x = x.mapped(g.map_deg);
@@ -145,20 +122,7 @@ struct ChunkPrefetch {
 #pragma unroll
       for (int j = 0; j < NV_WSH; ++j) {
         const int v = tid + j * kSegThreads;
-        if (v < CH * SPM / 8) wsv[j].store(&sm.wsh[(v * 8) / SPM][(v * 8) % SPM]);
-      }
-    }
-    if (tid < CH) {
-      sm.sc.alpha[tid] = ok_t ? to_f32(alpha) : 1.f;
-      sm.sc.eta[tid] = ok_t ? to_f32(eta) : 0.f;
-      sm.sc.beta[tid] = ok_t ? (g.momentum ? to_f32(beta) : 0.f) : 1.f;
-    }
-    if (g.gate_mode == GATE_TOKEN && tid < SPM) sm.sc.ug[tid] = ok_ug ? to_f32(ug) : (pad_ug ? 1.f : 0.f);
-    if (g.gate_mode == GATE_LAG) {
-#pragma unroll
-      for (int j = 0; j < NWL; ++j) {
-        const int idx = tid + j * kSegThreads;
-        if (idx < CH * g.e) sm.sc.wl[idx] = ((ok_wl >> j) & 1u) ? to_f32(wl[j]) : 0.f;
+        if (v < CH * SP / 8) wsv[j].store(&sm.wsh[v / (SP / 8)][(v % (SP / 8)) * 8]);
       }
     }
   }
@@ -177,17 +141,17 @@ enum WalkMode { WALK_AGG = 0, WALK_FULL = 1 };
 // Wave roles per chunk: P1 all waves run G1 (and G2 for the full walk); P3 all waves run G3 (y,
 // full walk), then G4 on the state tiles they own, updating the states, which they hold in
 // registers.
-template <typename T, int CH, int D, int MODE>
+template <typename T, int CH, int D, int HP, int MODE>
 __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, const SegGeom& sg, float* agg,
                                             const float* seg_states, float* rw, float* final_raw,
                                             const float* coef, const T* wsh_all, unsigned char* smem_raw) {
   constexpr bool AGG = MODE == WALK_AGG;
   constexpr bool FULL = MODE == WALK_FULL;
-  typedef SegFwdSmem<T, CH, D, FULL> Sm;
+  typedef SegFwdSmem<T, CH, D, HP, FULL> Sm;
   Sm& sm = *reinterpret_cast<Sm*>(smem_raw);
-  constexpr int SPM = Sm::SPM;
+  constexpr int SPM = CH + kHaloPad, SP = Sm::SP, SPK = Sm::SPK, LD = Sm::LD, LQ = Sm::LQ;
   constexpr int NTD = D / 16;                    // 16-wide tiles along D
-  constexpr int NTS = SPM / 16;                  // 16-wide tiles along the sources
+  constexpr int NTS = SP / 16;                   // 16-wide tiles along the sources
   typedef MM<T> M;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int seg = blockIdx.x, bh = blockIdx.y;
@@ -198,6 +162,15 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
 
   // ---- S_ref (bf16/fp32 operand copy)
   for (int idx = tid; idx < D * D; idx += kSegThreads) sm.sref[idx / D][idx % D] = from_f32<T>(a.S_ref[sb + idx]);
+  if constexpr (SPK > SP) {   // the source rows past SP: zeros, never written again
+    for (int idx = tid; idx < (SPK - SP) * D; idx += kSegThreads) {
+      sm.phi[SP + idx / D][idx % D] = from_f32<T>(0.f);
+      sm.vd[SP + idx / D][idx % D] = from_f32<T>(0.f);
+    }
+    if constexpr (FULL)
+      for (int idx = tid; idx < CH * (SPK - SP); idx += kSegThreads)
+        sm.Q[idx / (SPK - SP)][SP + idx % (SPK - SP)] = from_f32<T>(0.f);
+  }
 
   // ---- state registers: the NTD x NTD state tiles are spread over the waves, NOWN tiles of one
   // row tile per wave.
@@ -236,7 +209,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
   constexpr int REC = CoefRec<CH>::SIZE;
   const float* coef_row = coef + (size_t)bh * g.nc * REC;
   const T* wsh_row = FULL ? wsh_all + (size_t)bh * g.nc * CH * SPM : nullptr;
-  ChunkPrefetch<T, CH, D, FULL> pf;
+  ChunkPrefetch<T, CH, D, HP, FULL> pf;
   if (c_begin < c_end) {
     const int t0 = c_begin * g.Lc;
     pf.load(g, a, tb, t0, min(g.T, t0 + g.Lc) - t0, coef_row + (size_t)c_begin * REC,
@@ -291,10 +264,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
         const int tile = min(wave + NGW * j, NT1 - 1);
         const bool valid = NT1 % NGW == 0 || wave + NGW * j < NT1;
         const int m0 = (tile % NTD) * 16, n0 = (tile / NTD) * 16;   // m: rows i, n: sources
-        f32x4 acc = zero4();
-#pragma unroll
-        for (int k0 = 0; k0 < D; k0 += M::KS)
-          acc = M::mma(frag_ld_row<T>(&sm.sref[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.phi[0][0], D + 8, n0, k0), acc);
+        const f32x4 acc = kop_mma(kop_row<T, D>(&sm.sref[0][0], LD, m0), kop_row<T, D>(&sm.phi[0][0], LD, n0), zero4());
         if (valid) {
           // rows i0..i0+3 of source s are contiguous in vd: v read and delta written in place
           const int s = n0 + (lane & 15), i0 = m0 + 4 * (lane >> 4);
@@ -314,10 +284,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
           const int tt = min(wave + NGW * j, NT2 - 1);
           const bool valid = NT2 % NGW == 0 || wave + NGW * j < NT2;
           const int m0 = (tt % NTS) * 16, n0 = (tt / NTS) * 16;   // m: sources s, n: targets tau
-          f32x4 acc = zero4();
-#pragma unroll
-          for (int k0 = 0; k0 < D; k0 += M::KS)
-            acc = M::mma(frag_ld_row<T>(&sm.phi[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.psi[0][0], D + 8, n0, k0), acc);
+          const f32x4 acc = kop_mma(kop_row<T, D>(&sm.phi[0][0], LD, m0), kop_row<T, D>(&sm.psi[0][0], LD, n0), zero4());
           if (valid) {
             const int t = n0 + (lane & 15), s0 = m0 + 4 * (lane >> 4);
             store4<T>(&sm.Q[t][s0], acc[0] * to_f32(sm.wsh[t][s0]), acc[1] * to_f32(sm.wsh[t][s0 + 1]),
@@ -338,16 +305,10 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
         const bool valid = NT3 % kSegWaves == 0 || wave + kSegWaves * j < NT3;
         {
           const int m0 = (tile % NTD) * 16, n0 = (tile / NTD) * 16;   // m: rows i, n: targets tau
-          f32x4 aq = zero4(), as = zero4(), az = zero4();
-#pragma unroll
-          for (int k0 = 0; k0 < SPM; k0 += M::KS)
-            aq = M::mma(frag_ld_tr<T>(&sm.vd[0][0], D + 8, m0, k0), frag_ld_row<T>(&sm.Q[0][0], SPM + 8, n0, k0), aq);
-#pragma unroll
-          for (int k0 = 0; k0 < D; k0 += M::KS) {
-            const typename M::frag fb = frag_ld_row<T>(&sm.psi[0][0], D + 8, n0, k0);
-            as = M::mma(frag_ld_row<T>(&sm.Sb[0][0], D + 8, m0, k0), fb, as);
-            az = M::mma(frag_ld_row<T>(&sm.Zb[0][0], D + 8, m0, k0), fb, az);
-          }
+          const f32x4 aq = kop_mma(kop_tr<T, SPK>(&sm.vd[0][0], LD, m0), kop_row<T, SPK>(&sm.Q[0][0], LQ, n0), zero4());
+          const KOp<T, D> fb = kop_row<T, D>(&sm.psi[0][0], LD, n0);
+          const f32x4 as = kop_mma(kop_row<T, D>(&sm.Sb[0][0], LD, m0), fb, zero4());
+          const f32x4 az = kop_mma(kop_row<T, D>(&sm.Zb[0][0], LD, m0), fb, zero4());
           // a lane holds rows i0..i0+3 of y for one target t
           const int t = n0 + (lane & 15), i0 = m0 + 4 * (lane >> 4);
           const float ac = sm.sc.acoef[t], kc = sm.sc.kcoef[t];
@@ -360,7 +321,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
               f32x4 ab = zero4();
 #pragma unroll
               for (int k0 = 0; k0 < D; k0 += M::KS)
-                ab = M::mma(frag_ld<T>(Bs, D, 1, m0, k0), frag_ld_row<T>(&sm.psi[0][0], D + 8, n0, k0), ab);
+                ab = M::mma(frag_ld<T>(Bs, D, 1, m0, k0), frag_ld_row<T>(&sm.psi[0][0], LD, n0, k0), ab);
               const float w = to_f32(sm.wsh[t][s]);
 #pragma unroll
               for (int r = 0; r < 4; ++r) yv[r] -= w * ab[r];
@@ -377,28 +338,16 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
       const bool do_clamp = !AGG && clamp_after(g, t1);
       const bool mid = FULL && g.Lmid > 0 && L > g.Lmid;
       const int m0 = mt * 16;
-      constexpr int NKS = SPM / M::KS;
+      const KOp<T, SPK> fd = kop_tr<T, SPK>(&sm.vd[0][0], LD, m0);
       if constexpr (FULL) {
         if (mid) {   // state after token Lmid - 1 (never a clamp point), from the chunk-start state
           float* rw_mid = rw + ((size_t)bh * g.ncb + (size_t)c * rb + 1) * 2 * D * D;
-          typename M::frag fsm[NKS], fzm[NKS];
-#pragma unroll
-          for (int kk = 0; kk < NKS; ++kk) {
-            const typename M::frag fd = frag_ld_tr<T>(&sm.vd[0][0], D + 8, m0, kk * M::KS);
-            const int sb = kk * M::KS + (lane >> 4) * M::KL;
-            fsm[kk] = frag_scale<T>(fd, &sm.sc.wsmid[sb]);
-            fzm[kk] = frag_scale<T>(fd, &sm.sc.wzmid[sb]);
-          }
+          const KOp<T, SPK> fsm = kop_scale(fd, sm.sc.wsmid), fzm = kop_scale(fd, sm.sc.wzmid);
 #pragma unroll
           for (int jn = 0; jn < NOWN; ++jn) {
             const int n0 = (nt0 + jn) * 16;
-            f32x4 aum = zero4(), avm = zero4();
-#pragma unroll
-            for (int kk = 0; kk < NKS; ++kk) {
-              const typename M::frag fb = frag_ld_tr<T>(&sm.phi[0][0], D + 8, n0, kk * M::KS);
-              aum = M::mma(fsm[kk], fb, aum);
-              avm = M::mma(fzm[kk], fb, avm);
-            }
+            const KOp<T, SPK> fb = kop_tr<T, SPK>(&sm.phi[0][0], LD, n0);
+            const f32x4 aum = kop_mma(fsm, fb, zero4()), avm = kop_mma(fzm, fb, zero4());
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int i = m0 + 4 * (lane >> 4) + r, k = n0 + (lane & 15);
@@ -416,27 +365,15 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
           }
         }
       }
-      typename M::frag fs[NKS], fz[NKS];
-#pragma unroll
-      for (int kk = 0; kk < NKS; ++kk) {
-        const typename M::frag fd = frag_ld_tr<T>(&sm.vd[0][0], D + 8, m0, kk * M::KS);
-        const int sb = kk * M::KS + (lane >> 4) * M::KL;
-        fs[kk] = frag_scale<T>(fd, &sm.sc.wsend[sb]);
-        fz[kk] = frag_scale<T>(fd, &sm.sc.wzend[sb]);
-      }
+      const KOp<T, SPK> fs = kop_scale(fd, sm.sc.wsend), fz = kop_scale(fd, sm.sc.wzend);
       // raw end state -> the next chunk's saved start state (within the segment: the next segment's
       // workgroup writes its own start state, from the segment scan)
       float* rw_next = (FULL && c + 1 < c_end) ? rw + ((size_t)bh * g.ncb + (size_t)(c + 1) * rb) * 2 * D * D : nullptr;
 #pragma unroll
       for (int jn = 0; jn < NOWN; ++jn) {
         const int n0 = (nt0 + jn) * 16;
-        f32x4 au = zero4(), av = zero4();
-#pragma unroll
-        for (int kk = 0; kk < NKS; ++kk) {
-          const typename M::frag fb = frag_ld_tr<T>(&sm.phi[0][0], D + 8, n0, kk * M::KS);
-          au = M::mma(fs[kk], fb, au);
-          av = M::mma(fz[kk], fb, av);
-        }
+        const KOp<T, SPK> fb = kop_tr<T, SPK>(&sm.phi[0][0], LD, n0);
+        const f32x4 au = kop_mma(fs, fb, zero4()), av = kop_mma(fz, fb, zero4());
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = m0 + 4 * (lane >> 4) + r, k = n0 + (lane & 15);

@@ -33,12 +33,12 @@ namespace atlas {
 
 // Two workgroups per CU (16 waves, at most 128 VGPRs each) for the bf16 configurations, whose
 // aggregate-pass LDS fits twice in 160 KB.
-template <typename T, int CH, int D>
+template <typename T, int CH, int D, int HP>
 __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_fwd_seg_agg(const Geom g, const FwdPtrs<T> a, const SegGeom sg,
                                                                float* agg, const float* coef) {
   if (geom_skip(g)) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  fwd_segment<T, CH, D, WALK_AGG>(g, a, sg, agg, nullptr, nullptr, nullptr, coef, nullptr, smem_raw);
+  fwd_segment<T, CH, D, HP, WALK_AGG>(g, a, sg, agg, nullptr, nullptr, nullptr, coef, nullptr, smem_raw);
 }
 
 // grid (D * D / kThreads + H', BH): segment-start states
@@ -104,41 +104,54 @@ hipError_t launch_fwd_seg_scan(const Geom& g, const FwdPtrs<T>& a, const SegGeom
 template hipError_t launch_fwd_seg_scan<bf16, 64>(const Geom&, const FwdPtrs<bf16>&, const SegGeom&, const float*,
                                                   float*, hipStream_t);
 
-template <typename T, int CH, int D>
+template <typename T, int CH, int D, int HP>
 __global__ __launch_bounds__(kSegThreads) void k_fwd_seg(const Geom g, const FwdPtrs<T> a, const SegGeom sg,
                                                            const float* seg_states, float* rw, float* final_raw,
                                                            const float* coef, const T* wsh) {
   if (geom_skip(g)) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  fwd_segment<T, CH, D, WALK_FULL>(g, a, sg, nullptr, seg_states, rw, final_raw, coef, wsh, smem_raw);
+  fwd_segment<T, CH, D, HP, WALK_FULL>(g, a, sg, nullptr, seg_states, rw, final_raw, coef, wsh, smem_raw);
 }
 
-template <typename T, int CH, int D>
-hipError_t launch_fwd_seg(const Geom& g, const FwdPtrs<T>& a, const SegGeom& sg, float* agg, float* seg_states,
+template <typename T, int CH, int D, int HP>
+static hipError_t launch_fwd_seg_hp(const Geom& g, const FwdPtrs<T>& a, const SegGeom& sg, float* agg, float* seg_states,
                           float* rw, float* final_raw, float* coef, T* wsh, hipStream_t stream) {
   // the chunk coefficient records (coef, wsh) are formed by the caller first
   hipError_t err = hipSuccess;
   if (sg.nseg > 1) {
-    const size_t smem = sizeof(SegFwdSmem<T, CH, D, false>);
-    err = set_dyn_smem(reinterpret_cast<const void*>(&k_fwd_seg_agg<T, CH, D>), smem);
+    const size_t smem = sizeof(SegFwdSmem<T, CH, D, HP, false>);
+    err = set_dyn_smem(reinterpret_cast<const void*>(&k_fwd_seg_agg<T, CH, D, HP>), smem);
     if (err != hipSuccess) return err;
     prof_name(KID_FWD_SEG_AGG, "k_fwd_seg_agg");
     prof_begin(KID_FWD_SEG_AGG, stream);
-    hipLaunchKernelGGL((k_fwd_seg_agg<T, CH, D>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg, agg,
+    hipLaunchKernelGGL((k_fwd_seg_agg<T, CH, D, HP>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg, agg,
                        (const float*)coef);
     prof_end(KID_FWD_SEG_AGG, stream);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   if ((err = launch_fwd_seg_scan<T, D>(g, a, sg, agg, seg_states, stream)) != hipSuccess) return err;
-  const size_t smem = sizeof(SegFwdSmem<T, CH, D, true>);
-  err = set_dyn_smem(reinterpret_cast<const void*>(&k_fwd_seg<T, CH, D>), smem);
+  const size_t smem = sizeof(SegFwdSmem<T, CH, D, HP, true>);
+  err = set_dyn_smem(reinterpret_cast<const void*>(&k_fwd_seg<T, CH, D, HP>), smem);
   if (err != hipSuccess) return err;
   prof_name(KID_FWD_WALK, "k_fwd_seg");
   prof_begin(KID_FWD_WALK, stream);
-  hipLaunchKernelGGL((k_fwd_seg<T, CH, D>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg,
+  hipLaunchKernelGGL((k_fwd_seg<T, CH, D, HP>), dim3(sg.nseg, g.BH), dim3(kSegThreads), smem, stream, g, a, sg,
                      (const float*)seg_states, rw, final_raw, (const float*)coef, (const T*)wsh);
   prof_end(KID_FWD_WALK, stream);
   return hipGetLastError();
+}
+
+// Windows up to 17 span a halo of 16 source slots, longer ones 32 (bf16 only: an fp32 call's backward
+// chunks of 16 tokens bound its window). With 32 slots for every window, fp32 d = 64 e = 4 (32 rows of
+// 1024 tokens) took 65 us here and 36 us for the aggregates, of which a third were products with zeros;
+// with 16, and float4 operand reads, 48 and 22 us.
+template <typename T, int CH, int D>
+hipError_t launch_fwd_seg(const Geom& g, const FwdPtrs<T>& a, const SegGeom& sg, float* agg, float* seg_states,
+                          float* rw, float* final_raw, float* coef, T* wsh, hipStream_t stream) {
+  if (g.H <= 16) return launch_fwd_seg_hp<T, CH, D, 16>(g, a, sg, agg, seg_states, rw, final_raw, coef, wsh, stream);
+  if constexpr (sizeof(T) == 2)
+    return launch_fwd_seg_hp<T, CH, D, 32>(g, a, sg, agg, seg_states, rw, final_raw, coef, wsh, stream);
+  return hipErrorInvalidValue;
 }
 
 #define ATLAS_INST_FWD_SEG(T, CH, D) \
