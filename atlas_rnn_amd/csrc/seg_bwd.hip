@@ -1016,7 +1016,22 @@ hipError_t launch_bwd_seg(const Geom& g, const BwdPtrs<T>& a, const SegGeom& sg,
       if (err != hipSuccess) return err;
     }
   }
-  if (!walk && (err = launch_bwd_scalar<T, CH>(g, a, p, stream)) != hipSuccess) return err;
+  if (!walk) {
+    // The specialised path's scalar chains (one wave per chunk of 32, windows up to 17) read the same
+    // records at any head size: 64 rows of 777 tokens, d = 32: 13 us against 28 as table products.
+    bool chains = false;
+    if constexpr (sizeof(T) == 2 && CH == 32) {
+      chains = g.H <= 16 && g.Lc == 32;
+      if (chains) {
+        prof_name(KID_BWD_SCALAR, "k_scalar_chain");
+        prof_begin(KID_BWD_SCALAR, stream);
+        err = launch_scalar_chain(g, a, p, sg, false, stream);
+        prof_end(KID_BWD_SCALAR, stream);
+      }
+    }
+    if (!chains) err = launch_bwd_scalar<T, CH>(g, a, p, stream);
+    if (err != hipSuccess) return err;
+  }
   if (fixup_in_chain) return hipSuccess;
   prof_begin(KID_BWD_FIXUP, stream);
   hipLaunchKernelGGL((k_bwd_seg_fixup<T, D>), dim3(sg.nseg, g.BH), dim3(kThreads), 0, stream, g, a, sg, p,
