@@ -152,22 +152,37 @@ struct Plan {
 #define ATLAS_CHUNK_COEF 1
 #endif
 
-// Segments per head-batch row: enough (segment, bh) workgroups for one per CU (the walks hold a
-// CU's LDS, so a second round of workgroups would only queue behind the first); a single segment
-// when S is clamped at scan_chunk_len boundaries (not affine). The CU count is MI355X's, fixed so
-// that the saved / workspace sizes do not depend on the device queried.
+// Segments per head-batch row: one (segment, row) workgroup per CU (the walks hold most of a CU's LDS,
+// so that workgroups past that queue for a second round), or two where `share` of them fit; a single
+// segment when S is clamped at scan_chunk_len boundaries (not affine). Of the counts up to
+// ceil(slots / BH) the one with the shortest schedule is taken, rounds of workgroups times chunks per
+// segment: rounding up alone gave 40 rows 7 segments, 280 workgroups on 256 CUs, two rounds of a seventh
+// of the row instead of one of a sixth (fp32 d = 64: 40 rows of 1024 tokens 347 -> 296 us a step, 12 of
+// 4096 518 -> 339; bf16: 12 of 4096 132 -> 98, 160 of 500 172 -> 139). In units of a chunk's step: a
+// segment's start costs about one, more than one segment needs the aggregate passes (a quarter of the
+// step), eight segments' aggregates in the scans half a chunk, and two workgroups on a CU take
+// 1.45 times one's time. The CU count is MI355X's, fixed so that the saved / workspace sizes do not depend
+// on the device queried.
 constexpr int kCUs = 256;
-SegGeom make_seg(const Geom& g) {
+SegGeom make_seg(const Geom& g, int share) {
   SegGeom s{};
-  int G;
-  if (g.clamp_every > 0) {
-    G = g.nc;
-  } else {
-    const int want = g.BH >= kCUs ? 1 : (kCUs + g.BH - 1) / g.BH;
-    G = (g.nc + want - 1) / want;
+  int G = g.nc;
+  if (g.clamp_every == 0) {
+    const int slots = share * kCUs;
+    const int most = g.BH >= slots ? 1 : (slots + g.BH - 1) / g.BH;
+    double best = 0.;
+    for (int want = 1; want <= most && want <= g.nc; ++want) {
+      const int Gw = (g.nc + want - 1) / want, n = (g.nc + Gw - 1) / Gw;
+      const int64_t wgs = (int64_t)g.BH * n, rest = wgs % slots;
+      const double full = share == 1 ? 1. : 1.45;
+      const double rounds = (double)(wgs / slots) * full + (rest == 0 ? 0. : rest <= kCUs ? 1. : full);
+      const double cost = rounds * (Gw + 1.) * (n > 1 ? 1.25 : 1.) + n / 16.;
+      if (want == 1 || cost < best) {
+        best = cost;
+        G = Gw;
+      }
+    }
   }
-  if (G < 1) G = 1;
-  if (G > g.nc) G = g.nc;
   s.G = G;
   s.nseg = (g.nc + G - 1) / G;
   s.agg_stride = 2 * g.DV * g.DK + 16;
@@ -183,7 +198,7 @@ int largest_divisor_at_most(int n, int cap) {
   return 1;
 }
 
-Plan make_plan(const atlas_mem_problem* p, bool serial_clamp = false) {
+Plan make_plan_shared(const atlas_mem_problem* p, bool serial_clamp, int share) {
   Plan pl{};
   pl.ok = false;
   pl.status = ATLAS_MEM_ERR_ARG;
@@ -223,7 +238,7 @@ Plan make_plan(const atlas_mem_problem* p, bool serial_clamp = false) {
   // clamp points on forward-chunk ends: segment-parallel with the clamp points checked (dual)
   pl.dual = !serial_clamp && p->clamp_every > 0 && p->clamp_every % CH == 0 && p->clamp_every < p->seq_len;
   if (pl.dual) g.clamp_every = 0;
-  pl.sg = make_seg(g);
+  pl.sg = make_seg(g, share);
   pl.cbwd = ATLAS_CHUNK_BWD && p->dtype == ATLAS_DT_BF16 && !pl.dual && walk_fwd_supported(g) &&
             chunk_bwd_supported(g, pl.sg);
   if (pl.cbwd) g.Lmid = 0;
@@ -243,6 +258,8 @@ Plan make_plan(const atlas_mem_problem* p, bool serial_clamp = false) {
   pl.status = ATLAS_MEM_OK;
   return pl;
 }
+
+Plan make_plan(const atlas_mem_problem* p, bool serial_clamp = false);
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -307,6 +324,21 @@ BwdLayout bwd_layout(const Plan& pl) {
   L.badj = off; off += align256(walk_with_buffer(pl) ? (size_t)g.BH * bufw::kAdjFloats * sizeof(float) : 0);
   L.total = off;
   return L;
+}
+
+// Scratch of atlas_mem_bwd_noalloc (below).
+constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
+
+// bf16 heads of 32: two workgroups share a CU (LDS below 64 KB), so the rows are cut for 512: 64 rows of
+// 777 tokens 117 -> 103 us a step, 32 of 4096 195 -> 166, 16 of 2000 82 -> 81. (fp32 heads of 32 got
+// slower with 512: 217 -> 235 us at 64 rows of 777.) Not where the larger workspace would no longer
+// fit the static scratch.
+Plan make_plan(const atlas_mem_problem* p, bool serial_clamp) {
+  const Plan one = make_plan_shared(p, serial_clamp, 1);
+  if (!one.ok || one.esize != 2 || one.g.DK != 32 || one.g.clamp_every > 0) return one;
+  const Plan two = make_plan_shared(p, serial_clamp, 2);
+  if (bwd_layout(two).total > kNoAllocScratchBytes && bwd_layout(one).total <= kNoAllocScratchBytes) return one;
+  return two;
 }
 
 // `saved` of a dual plan: the flag (256 bytes), then the segment-parallel sequence's layout, then the
@@ -470,7 +502,6 @@ int run_bwd_plan(const atlas_mem_problem* prob, const Plan& pl, const atlas_mem_
 // up once per device with that device current (the entry point's first call there) and kept in
 // scratch_dev. Calls that overlap on one GPU share the array and race; every call overwrites what
 // it reads (the backward never relies on zeroed workspace), so nothing has to be cleared.
-constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;
