@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "atlas_mem_saved_bytes",
     "atlas_mem_bwd_workspace_bytes",
     "atlas_mem_fwd",
+    "atlas_mem_infer",
     "atlas_mem_bwd",
     "atlas_mem_bwd_noalloc",
     "atlas_mem_noalloc_scratch_bytes",
@@ -133,6 +134,8 @@ def load(path: str | None = None) -> ctypes.CDLL:
     lib.atlas_mem_bwd_workspace_bytes.argtypes = [P]
     lib.atlas_mem_fwd.restype = i32
     lib.atlas_mem_fwd.argtypes = [P, ctypes.POINTER(FwdArgs), vp, vp]
+    lib.atlas_mem_infer.restype = i32
+    lib.atlas_mem_infer.argtypes = [P, ctypes.POINTER(FwdArgs), vp, vp]
     lib.atlas_mem_step.restype = i32
     lib.atlas_mem_step.argtypes = [P, ctypes.POINTER(FwdArgs), vp]
     lib.atlas_mem_step_factored.restype = i32

@@ -115,12 +115,19 @@ struct RecurrenceFn : public Function<RecurrenceFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& q, const Tensor& v, const Tensor& lr,
                                const Tensor& decay, const OptTensor& beta, const OptTensor& gate, const Tensor& S_ref,
                                const Tensor& S0, const OptTensor& Z0, const OptTensor& buf,
-                               const atlas_mem_problem& prob) {
+                               const atlas_mem_problem& prob, bool infer) {
     // outputs a loss does not use get no gradient tensor (a missing one counts as zero)
     ctx->set_materialize_grads(false);
     const RecOut o = rec_outputs(prob, k);
     const Tensor saved = scratch(k, (int64_t)atlas_mem_saved_bytes(&prob));
     const atlas_mem_fwd_args a = fwd_args(k, q, v, lr, decay, get(beta), get(gate), S_ref, S0, get(Z0), get(buf), o);
+    if (infer) {   // no input asks for a gradient: nothing for a backward is formed or kept
+      check(atlas_mem_infer(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
+      variable_list out{o.y, o.S_T};
+      if (o.Z_T.defined()) out.push_back(o.Z_T);
+      if (o.buf.defined()) out.push_back(o.buf);
+      return out;
+    }
     check(atlas_mem_fwd(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
     ctx->save_for_backward({k, q, v, lr, decay, get(beta), get(gate), S_ref, S0, get(Z0), get(buf), saved});
     ctx->saved_data["prob"] = std::string(reinterpret_cast<const char*>(&prob), sizeof(prob));
@@ -154,7 +161,7 @@ struct RecurrenceFn : public Function<RecurrenceFn> {
     a.dk = mptr(dk); a.dq = mptr(dq); a.dv = mptr(dv); a.dlr = mptr(dlr); a.ddecay = mptr(dd); a.dbeta = mptr(db);
     a.dgate = mptr(dg); a.dS_ref = mfptr(dS_ref); a.dS0 = mfptr(dS0); a.dZ0 = mfptr(dZ0); a.dbuffer_in = mfptr(dbuf);
     check(atlas_mem_bwd(&prob, &a, fptr(saved), mptr(ws), ws_bytes, stream_of(k)), "atlas_mem_bwd");
-    return {dk, dq, dv, dlr, dd, db, dg, dS_ref, dS0, Z0.defined() ? dZ0 : Tensor(), dbuf, Tensor()};
+    return {dk, dq, dv, dlr, dd, db, dg, dS_ref, dS0, Z0.defined() ? dZ0 : Tensor(), dbuf, Tensor(), Tensor()};
   }
 };
 
@@ -212,11 +219,11 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
   const Tensor Src = !S_ref.defined() || S_ref.is_same(S0) ? S0c : canon(S_ref, at::kFloat);
   const Tensor Zc = canon(Z0, at::kFloat), Bc = canon(buf, at::kFloat);
   RecOut o;
+  bool grad = false;
+  if (at::GradMode::is_enabled())
+    for (const Tensor* t : {&kc, &qc, &vc, &lc, &dc, &bc, &gc, &Src, &S0c, &Zc, &Bc})
+      grad = grad || (t->defined() && t->requires_grad());
   if (T == 1) {
-    bool grad = false;
-    if (at::GradMode::is_enabled())
-      for (const Tensor* t : {&kc, &qc, &vc, &lc, &dc, &bc, &gc, &Src, &S0c, &Zc, &Bc})
-        grad = grad || (t->defined() && t->requires_grad());
     if (!grad) {   // decode: one launch, no saved buffer (rnn_transformer.py:863-900 through the cell at T = 1)
       o = rec_outputs(p, kc);
       const atlas_mem_fwd_args a = fwd_args(kc, qc, vc, lc, dc, bc, gc, Src, S0c, Zc, Bc, o);
@@ -224,7 +231,8 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
       return o;
     }
   }
-  const variable_list out = RecurrenceFn::apply(kc, qc, vc, lc, dc, opt(bc), opt(gc), Src, S0c, opt(Zc), opt(Bc), p);
+  const variable_list out = RecurrenceFn::apply(kc, qc, vc, lc, dc, opt(bc), opt(gc), Src, S0c, opt(Zc), opt(Bc), p,
+                                                !grad);
   size_t i = 0;
   o.y = out[i++];
   o.S_T = out[i++];

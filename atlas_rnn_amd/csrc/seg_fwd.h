@@ -229,7 +229,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
     const int rb = g.Lmid > 0 ? 2 : 1;        // backward chunks per forward chunk
     if constexpr (FULL) {
       // the segment's start state (later chunk starts are written as the previous chunk ends)
-      if (owns && c == c_begin) {
+      if (rw && owns && c == c_begin) {   // (rw null: no backward follows)
         float* dst = rw + ((size_t)bh * g.ncb + (size_t)c * rb) * 2 * D * D;
 #pragma unroll
         for (int jn = 0; jn < NOWN; ++jn)
@@ -368,7 +368,7 @@ __device__ __forceinline__ void fwd_segment(const Geom& g, const FwdPtrs<T>& a, 
       const KOp<T, SPK> fs = kop_scale(fd, sm.sc.wsend), fz = kop_scale(fd, sm.sc.wzend);
       // raw end state -> the next chunk's saved start state (within the segment: the next segment's
       // workgroup writes its own start state, from the segment scan)
-      float* rw_next = (FULL && c + 1 < c_end) ? rw + ((size_t)bh * g.ncb + (size_t)(c + 1) * rb) * 2 * D * D : nullptr;
+      float* rw_next = (FULL && rw && c + 1 < c_end) ? rw + ((size_t)bh * g.ncb + (size_t)(c + 1) * rb) * 2 * D * D : nullptr;
 #pragma unroll
       for (int jn = 0; jn < NOWN; ++jn) {
         const int n0 = (nt0 + jn) * 16;

@@ -138,6 +138,11 @@ size_t atlas_mem_bwd_workspace_bytes(const atlas_mem_problem* prob);
 int atlas_mem_fwd(const atlas_mem_problem* prob, const atlas_mem_fwd_args* args,
                   float* saved, void* stream);
 
+/* The same results where no backward follows (a prefill): what only atlas_mem_bwd reads is not formed.
+ * `scratch` has atlas_mem_saved_bytes bytes; atlas_mem_bwd must not be given it. */
+int atlas_mem_infer(const atlas_mem_problem* prob, const atlas_mem_fwd_args* args,
+                    float* scratch, void* stream);
+
 /* One token (seq_len == 1, forward only) without a saved buffer: the decode / streaming step of
  * RNNMemoryTransformer.generate (atlas_pytorch/rnn_transformer.py:863-900), which runs the cell's
  * recurrence (atlas_pytorch/rnn_memory.py:605-730) one token at a time. Same problem and argument
@@ -236,14 +241,14 @@ int64_t atlas_omega_chain_workspace_bytes(int64_t bh, int64_t n, int64_t p, int 
 
 /* Right-affine scan H_t = H_{t-1} A_t + B_t over t = 1..T, fp32 (replaces affine_associative_scan,
  * atlas_pytorch/affine_scan.py:36-158): A [n,t,d,d], B [n,t,r,d], prev = H_0 [n,r,d] (NULL: zero),
- * out = H_1..H_T [n,t,r,d]; r, d <= 64. Chunked on the fp32 matrix cores: the chunks' composed maps,
- * a chain over chunks, then every chunk's states. `workspace` (atlas_affine_scan_workspace_bytes) is
+ * out = H_1..H_T [n,t,r,d]; r, d <= 64. On the fp32 matrix cores, in one pass over the steps where the rows
+ * fill the card, else in chunks: their composed maps, a chain over chunks, then every chunk's states. `workspace` (atlas_affine_scan_workspace_bytes) is
  * caller-owned scratch; pointers 4-byte aligned. */
 int atlas_affine_scan_fwd(int n, int t, int r, int d, const float* A, const float* B, const float* prev,
                           float* out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Gradients of atlas_affine_scan_fwd given its output H (= out): dA [n,t,d,d], dB [n,t,r,d] and
- * dprev [n,r,d] (may be NULL) for the output gradient dout [n,t,r,d]. The adjoint is the same chunked
+ * dprev [n,r,d] (may be NULL) for the output gradient dout [n,t,r,d]. The adjoint is the same
  * scan run backwards over A^T; same workspace size as the forward. */
 int atlas_affine_scan_bwd(int n, int t, int r, int d, const float* A, const float* H, const float* prev,
                           const float* dout, float* dA, float* dB, float* dprev, void* workspace,
