@@ -225,22 +225,25 @@ __device__ __forceinline__ void walk_fwd(const Geom& g, const FwdPtrs<bf16>& a, 
   float seg_a = 1.f, seg_k = 0.f, seg_b = 1.f;
   const int i0 = 16 * it + 4 * gq;
   const int rb = g.Lmid > 0 ? 2 : 1;
-  // saved states (walk_common.h layout): block of backward chunk cb at rw_row + cb * kStateBlk
-  // (rows of g.ncb blocks with mid points; of g.nc blocks, one per chunk, without)
-  unsigned char* rw_row =
-      FULL && rw ? reinterpret_cast<unsigned char*>(rw) + (size_t)bh * (rb == 2 ? g.ncb : g.nc) * kStateBlk : nullptr;
+  // saved states (walk_common.h layout): the blocks of the segment's backward chunks, from cb0 on, of a row of
+  // g.ncb blocks with mid points, of g.nc, one per chunk, without; none where no backward follows (rw null:
+  // the stores are out of range)
+  const int cb0 = c_begin * rb;
+  const rsrc_t rws = FULL && rw ? make_rsrc(reinterpret_cast<unsigned char*>(rw) +
+                                                ((size_t)bh * (rb == 2 ? g.ncb : g.nc) + cb0) * kStateBlk,
+                                            (uint32_t)((c_end - c_begin) * rb) * (uint32_t)kStateBlk)
+                                : make_rsrc(nullptr, 0u);
   // this lane's 8-byte half of the fragments of its tiles j = 0, 1
   const uint32_t f2o[2] = {frag_off(2 * th, it >> 1, lane) + (it & 1) * 8,
                            frag_off(2 * th + 1, it >> 1, lane) + (it & 1) * 8};
   auto save_state = [&](int cb, const float (&Sv)[2][4], const float (&Zv)[2][4]) {
-    if (!rw_row) return;   // no backward follows
-    unsigned char* blk = rw_row + (size_t)cb * kStateBlk;
+    const int so = (cb - cb0) * (int)kStateBlk;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      *reinterpret_cast<uint2*>(blk + f2o[j]) =
-          make_uint2(pack_bf16x2(Sv[j][0], Sv[j][1]), pack_bf16x2(Sv[j][2], Sv[j][3]));
-      *reinterpret_cast<uint2*>(blk + kStateBytes + f2o[j]) =
-          make_uint2(pack_bf16x2(Zv[j][0], Zv[j][1]), pack_bf16x2(Zv[j][2], Zv[j][3]));
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2v{pack_bf16x2(Sv[j][0], Sv[j][1]), pack_bf16x2(Sv[j][2], Sv[j][3])}, rws,
+                                            (int)f2o[j], so, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2v{pack_bf16x2(Zv[j][0], Zv[j][1]), pack_bf16x2(Zv[j][2], Zv[j][3])}, rws,
+                                            (int)(f2o[j] + kStateBytes), so, 0);
     }
   };
 
