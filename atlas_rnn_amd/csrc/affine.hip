@@ -13,10 +13,10 @@
 //   kChain   : per n: the chunk-start states X_{c+1} = X_c P_c + Q_c, chunks as steps
 //   kApply   : per (n, chunk > 0): the chunk's states from X_c
 // A step is a product of 512 cycles in the matrix cores (D = 64) and takes about 790, 0.33 us, where the operands
-// come from the infinity cache, and 0.45 from HBM. Before (three passes of 64-step chunks with every
-// wave on its own rows and 2 products a step): forward and backward together 1760 -> 1355 us at 32 x 1024 steps of
-// 64 x 64, 974 -> 535 at 16 x 1024, 888 -> 465 at 8, 828 -> 141 at 2, 548 -> 79 at 8 x 300 of 32 x 64, 697 -> 104 at 20 x 400 of
-// 16 x 16; the largest is bound by the 7 x 537 MB it moves and by its 128 workgroups' pull on them.
+// come from the infinity cache, and 0.45 to 0.5 from HBM. Before (three passes of 64-step chunks with every
+// wave on its own rows and 2 products a step), forward and backward together: 32 x 1024 steps of 64 x 64 1760 -> 1340
+// us, 16 x 1024 974 -> 819, 8 x 1024 888 -> 492, 2 x 1024 829 -> 142, 8 x 300 of 32 x 64 547 -> 78, 20 x 400 of 16 x 16
+// 697 -> 99. The largest moves 9 x 537 MB, its scans at 3.1 TB/s: 128 workgroups' pull on three streams.
 //
 // Backward: with the adjoint G_t = dL/dH_t,  G_T = dout_T,  G_t = dout_t + G_{t+1} A_{t+1}^T, so G is the
 // same scan run backwards in time over the transposed matrices (REV, written straight into dB = G). Then k_aff_grad_a forms dA_t = H_{t-1}^T G_t for every (n, t) and
