@@ -374,12 +374,25 @@ void set_flag(Plan& pl, const int* flag, int run, int reset, int check) {
 
 bool misaligned(const void* p, size_t a) { return p && (reinterpret_cast<uintptr_t>(p) % a) != 0; }
 
+// The chunk coefficient records in a plan's saved buffer. Both sequences of a dual plan have the same chunks, and
+// the records depend on the per-token scalars only, so the exact one reads those the fast one formed (a
+// launch less: 32 rows of 4096 tokens with a buffer and a clamp 251.0 -> 248.7 us a step, the cell 655.8 -> 653.8).
+struct Records {
+  unsigned char *coef, *wsh, *bcoef, *bwsh;
+};
+Records records_in(const Plan& pl, const void* saved) {
+  const SavedLayout SL = saved_layout(pl);
+  unsigned char* sv = static_cast<unsigned char*>(const_cast<void*>(saved));
+  return Records{sv + SL.coef, sv + SL.wsh, sv + SL.bcoef, sv + SL.bwsh};
+}
+
 // infer: no backward follows. The chunk-start states, the states between a forward chunk's backward chunks
 // (their products too) and the backward's coefficient records are left out; y, S_T, Z_T and buffer_out are the
 // same bit for bit, since nothing reads them in the forward
 // (16 rows of 1000 tokens with a carried buffer, bf16 d = 64: 41.9 -> 37.5 us a call).
 template <typename T>
-int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream_t s, bool infer) {
+int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream_t s, bool infer,
+            const Records* made = nullptr) {
   FwdPtrs<T> a;
   a.k = (const T*)x->k; a.q = (const T*)x->q; a.v = (const T*)x->v;
   a.lr = (const T*)x->lr; a.decay = (const T*)x->decay; a.beta = (const T*)x->beta; a.gate = (const T*)x->gate;
@@ -392,8 +405,9 @@ int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream
   float* agg = reinterpret_cast<float*>(sv + SL.agg);
   float* final_raw = reinterpret_cast<float*>(sv + SL.final_raw);
   float* rw = infer ? nullptr : reinterpret_cast<float*>(sv + SL.rw);
-  float* coef = reinterpret_cast<float*>(sv + SL.coef);
-  T* wsh = reinterpret_cast<T*>(sv + SL.wsh);
+  const Records rec = made ? *made : records_in(pl, saved);
+  float* coef = reinterpret_cast<float*>(rec.coef);
+  T* wsh = reinterpret_cast<T*>(rec.wsh);
   Geom g = pl.g;
   if (infer) {
     if (g.Lmid % 8 != 0) return ATLAS_MEM_ERR_LAUNCH;   // refused with a backward: refused here too
@@ -402,15 +416,15 @@ int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream
   const bool brec = !pl.cbwd && !infer;
   // chunk coefficient records of the forward and of the backward (one launch, inputs only)
   constexpr int CHF = sizeof(T) == 2 ? 64 : 32, CHB = sizeof(T) == 2 ? 32 : 16;
-  hipError_t err = hipErrorInvalidValue;
+  hipError_t err = made ? hipSuccess : hipErrorInvalidValue;
   if constexpr (sizeof(T) == 2) {
-    if (pl.ccoef)
+    if (!made && pl.ccoef)
       err = launch_chunk_coef_fwd(g, a.decay, a.lr, a.beta, a.gate, coef, wsh, s);
   }
-  if (!pl.ccoef)
+  if (!made && !pl.ccoef)
     err = launch_chunk_coef_pair<T, CHF, CHB>(
-        g, pl.gb, a.decay, a.lr, a.beta, a.gate, coef, wsh, brec ? reinterpret_cast<float*>(sv + SL.bcoef) : nullptr,
-        brec ? reinterpret_cast<T*>(sv + SL.bwsh) : nullptr, s);
+        g, pl.gb, a.decay, a.lr, a.beta, a.gate, coef, wsh, brec ? reinterpret_cast<float*>(rec.bcoef) : nullptr,
+        brec ? reinterpret_cast<T*>(rec.bwsh) : nullptr, s);
   if (err != hipSuccess) return ATLAS_MEM_ERR_LAUNCH;
   err = hipErrorInvalidValue;
   if (g.DK == 64) {
@@ -437,7 +451,8 @@ int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream
 }
 
 template <typename T>
-int run_bwd(const Plan& pl, const atlas_mem_bwd_args* x, const float* saved, void* ws, hipStream_t s) {
+int run_bwd(const Plan& pl, const atlas_mem_bwd_args* x, const float* saved, void* ws, hipStream_t s,
+            const Records* made = nullptr) {
   const Geom& gb = pl.gb;
   const BwdLayout L = bwd_layout(pl);
   const SavedLayout SL = saved_layout(pl);
@@ -462,8 +477,9 @@ int run_bwd(const Plan& pl, const atlas_mem_bwd_args* x, const float* saved, voi
   p.halo_part = gb.H > 0 ? reinterpret_cast<float*>(w + L.halo) : nullptr;
   p.dw = gb.gate_mode == ATLAS_GATE_TOKEN ? reinterpret_cast<float*>(w + L.dw) : nullptr;
   // formed by the forward (read only here)
-  p.coef = const_cast<float*>(reinterpret_cast<const float*>(sv + SL.bcoef));
-  p.wsh = const_cast<unsigned char*>(sv + SL.bwsh);
+  const Records rec = made ? *made : records_in(pl, saved);
+  p.coef = reinterpret_cast<float*>(rec.bcoef);
+  p.wsh = rec.bwsh;
   p.scal = reinterpret_cast<float*>(w + L.scal);
   p.buf_adj = walk_with_buffer(pl) ? reinterpret_cast<float*>(w + L.badj) : nullptr;
   hipError_t err = hipErrorInvalidValue;
@@ -488,8 +504,9 @@ int check_bwd_args(const atlas_mem_problem& p, const atlas_mem_bwd_args* args, c
 // The backward of a plan (of both flag-selected sequences for a dual plan).
 int run_bwd_plan(const atlas_mem_problem* prob, const Plan& pl, const atlas_mem_bwd_args* args, const float* saved,
                  void* ws, hipStream_t s) {
-  auto one = [&](const Plan& q, const float* sv) {
-    return prob->dtype == ATLAS_DT_BF16 ? run_bwd<bf16>(q, args, sv, ws, s) : run_bwd<float>(q, args, sv, ws, s);
+  auto one = [&](const Plan& q, const float* sv, const Records* made = nullptr) {
+    return prob->dtype == ATLAS_DT_BF16 ? run_bwd<bf16>(q, args, sv, ws, s, made)
+                                        : run_bwd<float>(q, args, sv, ws, s, made);
   };
   if (!pl.dual) return one(pl, saved);
   Plan fast = pl, exact = make_plan(prob, true);
@@ -500,7 +517,8 @@ int run_bwd_plan(const atlas_mem_problem* prob, const Plan& pl, const atlas_mem_
   set_flag(exact, flag, 1, 0, 0);
   // either order: the flag is only read here; the exact sequence first, so that the per-kernel
   // timing labels name the segment-parallel kernels that normally run
-  const int st = one(exact, reinterpret_cast<const float*>(sv + D.exact));
+  const Records made = records_in(fast, sv + D.fast);
+  const int st = one(exact, reinterpret_cast<const float*>(sv + D.exact), &made);
   if (st != ATLAS_MEM_OK) return st;
   return one(fast, reinterpret_cast<const float*>(sv + D.fast));
 }
@@ -586,8 +604,9 @@ static int mem_forward(const atlas_mem_problem* prob, const atlas_mem_fwd_args* 
   const void* fp[] = {args->S_ref, args->S0, args->Z0, args->buffer_in, args->S_T, args->Z_T, args->buffer_out, saved};
   for (const void* q : fp) if (misaligned(q, 16)) return ATLAS_MEM_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  auto one = [&](const Plan& q, float* sv) {
-    return p.dtype == ATLAS_DT_BF16 ? run_fwd<bf16>(q, args, sv, s, infer) : run_fwd<float>(q, args, sv, s, infer);
+  auto one = [&](const Plan& q, float* sv, const Records* made = nullptr) {
+    return p.dtype == ATLAS_DT_BF16 ? run_fwd<bf16>(q, args, sv, s, infer, made)
+                                    : run_fwd<float>(q, args, sv, s, infer, made);
   };
   if (!pl.dual) return one(pl, saved);
   Plan fast = pl, exact = make_plan(prob, true);
@@ -598,7 +617,8 @@ static int mem_forward(const atlas_mem_problem* prob, const atlas_mem_fwd_args* 
   set_flag(exact, flag, 1, 0, 0);
   const int st = one(fast, reinterpret_cast<float*>(sv + D.fast));
   if (st != ATLAS_MEM_OK) return st;
-  return one(exact, reinterpret_cast<float*>(sv + D.exact));
+  const Records made = records_in(fast, sv + D.fast);
+  return one(exact, reinterpret_cast<float*>(sv + D.exact), &made);
 }
 
 int atlas_mem_fwd(const atlas_mem_problem* prob, const atlas_mem_fwd_args* args, float* saved, void* stream) {
