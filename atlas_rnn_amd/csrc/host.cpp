@@ -10,11 +10,14 @@
 // Every function here takes what the kernels take and returns None for anything else (other shapes,
 // devices or types): the Python callers then pad, split or raise. The nodes keep their tensors with
 // save_for_backward (saved-tensor hooks and version checks apply) and refuse functorch transforms and
-// forward-mode differentiation, as autograd functions without those rules do.
+// forward-mode differentiation, as autograd functions without those rules do. torch.jit.trace cannot see
+// into them: functional._native records a call as a Python node, and an entry reached by the trace itself
+// raises (it would be recorded as the allocation of its outputs).
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cstring>
 #include <optional>
@@ -830,18 +833,27 @@ py::object omega_chain(const Tensor& s, const Tensor& decay, const Tensor& last,
   return py::make_tuple(update, update.select(1, n), obj(lm1), obj(buf1));
 }
 
+// an entry point of the module: refused while torch.jit.trace records
+template <typename R, typename... A>
+auto entry(R (*f)(A...)) {
+  return [f](A... a) -> R {
+    TORCH_CHECK(!torch::jit::tracer::isTracing(), "the native operators are not traced: call them through atlas_rnn_amd");
+    return f(std::forward<A>(a)...);
+  };
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("recurrence", &recurrence);
-  m.def("tensor_map", &tensor_map);
-  m.def("symmetrized", &symmetrized);
-  m.def("block_split", &block_split);
-  m.def("replicate", &replicate);
-  m.def("replica_sum", &replica_sum);
-  m.def("products", &products);
-  m.def("wgrads", &wgrads);
-  m.def("linear", &linear);
-  m.def("cell_prologue", &cell_prologue);
-  m.def("omega_chain", &omega_chain);
+  m.def("recurrence", entry(&recurrence));
+  m.def("tensor_map", entry(&tensor_map));
+  m.def("symmetrized", entry(&symmetrized));
+  m.def("block_split", entry(&block_split));
+  m.def("replicate", entry(&replicate));
+  m.def("replica_sum", entry(&replica_sum));
+  m.def("products", entry(&products));
+  m.def("wgrads", entry(&wgrads));
+  m.def("linear", entry(&linear));
+  m.def("cell_prologue", entry(&cell_prologue));
+  m.def("omega_chain", entry(&omega_chain));
 }

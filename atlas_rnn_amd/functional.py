@@ -53,6 +53,88 @@ def _require_gpu(*ts: Tensor | None) -> torch.device:
     return dev
 
 
+class _no_trace:
+    """torch.jit.trace's recording paused."""
+
+    def __enter__(self):
+        self.state = torch._C._get_tracing_state()
+        torch._C._set_tracing_state(None)
+
+    def __exit__(self, *exc):
+        torch._C._set_tracing_state(self.state)
+
+
+def _map_tensors(x, fn):
+    """x (tensors, lists, tuples, plain values) with fn applied to its tensors."""
+    if isinstance(x, Tensor):
+        return fn(x)
+    return type(x)(_map_tensors(y, fn) for y in x) if isinstance(x, (list, tuple)) else x
+
+
+class _NativeCall:
+    """A native operator with its plain arguments; the tensors are given to the call. The text is what
+    torch.jit.trace compares when it checks a trace by a second one."""
+
+    def __init__(self, op: str, args):
+        self.op = op
+        self.args = _map_tensors(args, lambda t: _NativeCall)   # the class itself marks a tensor's place
+
+    def __repr__(self):
+        fill = lambda a: type(a)(map(fill, a)) if isinstance(a, (list, tuple)) else '.' if a is _NativeCall else a
+        return f"{self.op}{fill(self.args)}"
+
+    def __call__(self, tensors):
+        ts = iter(tensors)
+        put = lambda a: type(a)(map(put, a)) if isinstance(a, (list, tuple)) else next(ts) if a is _NativeCall else a
+        return getattr(_lib.native(), self.op)(*put(self.args))
+
+
+class _TracedFn(torch.autograd.Function):
+    """A native operator as one Python node, which is how torch.jit.trace records an operator that is not
+    torch's own: a trace of the native call itself would hold the allocation of its outputs and nothing
+    that fills them. The native autograd graph of the call is kept for the backward."""
+
+    @staticmethod
+    def forward(ctx, call, *tensors):
+        ctx.set_materialize_grads(False)
+        with _no_trace(), torch.enable_grad():
+            ctx.ins = [t.detach().requires_grad_(need) for t, need in zip(tensors, ctx.needs_input_grad[1:])]
+            ctx.outs = []
+            _map_tensors(call(ctx.ins), ctx.outs.append)
+            outs = [o.detach() for o in ctx.outs]
+        if torch._C._is_tracing():   # outputs that the trace knows
+            known = [torch.empty(list(o.shape), dtype=o.dtype, device=o.device) for o in outs]
+            with _no_trace():
+                for e, o in zip(known, outs):
+                    e.copy_(o)
+            outs = known
+        return tuple(outs)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        live = [(o, g) for o, g in zip(ctx.outs, grads) if g is not None and o.requires_grad]
+        want = [t for t in ctx.ins if t.requires_grad]
+        got = iter(torch.autograd.grad([o for o, _ in live], want, [g for _, g in live], retain_graph=True,
+                                       allow_unused=True) if live else [None] * len(want))
+        return (None, *(next(got) if t.requires_grad else None for t in ctx.ins))
+
+
+def _native(op: str, *args):
+    """The native operator `op` (csrc/host.cpp) on args; None where it does not take them."""
+    fn = getattr(_lib.native(), op)
+    if not torch._C._is_tracing():
+        return fn(*args)
+    args = _map_tensors(args, lambda t: t)
+    with _no_trace(), torch.no_grad():   # which outputs there are, and whether the operator takes the operands
+        layout = fn(*_map_tensors(args, lambda t: t.detach()))
+    if layout is None:
+        return None
+    tensors = []
+    _map_tensors(args, tensors.append)
+    outs = iter(_TracedFn.apply(_NativeCall(op, args), *tensors))
+    return _map_tensors(layout, lambda t: next(outs))
+
+
 def check_operands(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, *, window: int,
                    dtype: torch.dtype | None = None, contiguous: bool = False) -> None:
     """Raises ValueError unless the recurrence operands have consistent shapes, one device and
@@ -174,7 +256,7 @@ def symmetrized_tables(proj: Tensor, d: int, dtype) -> tuple[Tensor, Tensor]:
     if dtype not in _DTYPES:
         raise ValueError(f"symmetrized_tables: dtype {dtype} (the kernels take bfloat16 or float32)")
     _require_gpu(proj)
-    return _lib.native().symmetrized(proj, d, dtype)
+    return _native('symmetrized', proj, d, dtype)
 
 
 class _TensorMapFn:
@@ -186,7 +268,7 @@ class _TensorMapFn:
     def apply(x, proj, degree, tables=None):
         _require_gpu(x, proj)
         ps, pst = tables if tables is not None else (None, None)
-        return _lib.native().tensor_map(x, proj, degree, ps, pst)
+        return _native('tensor_map', x, proj, degree, ps, pst)
 
 
 def _tables_ok(tables, proj: Tensor, dtype) -> bool:
@@ -235,7 +317,7 @@ class _ReplicateFn:
 
     @staticmethod
     def apply(nrep, *xs):
-        return tuple(_lib.native().replicate(nrep, list(xs)))
+        return tuple(_native('replicate', nrep, list(xs)))
 
 
 class _ReplicaSumFn:
@@ -243,7 +325,7 @@ class _ReplicaSumFn:
 
     @staticmethod
     def apply(nrep, *xs):
-        return tuple(_lib.native().replica_sum(nrep, list(xs)))
+        return tuple(_native('replica_sum', nrep, list(xs)))
 
 
 def _replicas(op: int, nrep: int, xs):
@@ -289,7 +371,7 @@ def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
     S_ref, S0, Z0, buffer = pst(S_ref), pst(S0), pst(Z0), pst(buffer)
     nb = nbv * nbk
     _dt_code(phi)   # fp32 or bf16
-    kb, qb, vb = _lib.native().block_split(phi, psi, vv, S_ref)   # its adjoint: atlas_block_merge
+    kb, qb, vb = _native('block_split', phi, psi, vv, S_ref)   # its adjoint: atlas_block_merge
 
     def stack_state(x):        # [BH, ..., Dv, Dk] -> [(i, j, bh), ..., 64, 64]
         if x is None:
@@ -451,7 +533,7 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
     """
     if clamp_every is not None and k.dim() == 3 and clamp_every >= k.shape[1]:
         clamp_every = None        # no clamp point before the last token (the final clamp is clamp_final's)
-    out = _lib.native().recurrence(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
+    out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
                                    map_degree if map_mode == 'elementwise' else 1, clamp_every, bool(clamp_final))
     if out is not None:
         return out
@@ -726,7 +808,7 @@ def _wgrads(pairs, dtype) -> list:
     summed in a fixed order): 16384 tokens x 512 x 512 took 67 us through a transposed copy and a
     batched hipBLASLt product, whose plain form (one product with K = 16384 on few output tiles)
     took 100 us. fp32 operands keep torch's product over token slices."""
-    return _lib.native().wgrads([dy for dy, _ in pairs], [x for _, x in pairs], dtype)
+    return _native('wgrads', [dy for dy, _ in pairs], [x for _, x in pairs], dtype)
 
 
 def _wgrad(dy: Tensor, x: Tensor, dtype) -> Tensor:
@@ -741,13 +823,13 @@ def _products(layout: int, acts, weights):
     """atlas_linear_batch: up to four bf16 products in one launch. NT: acts[i] [..., k] x
     weights[i] [n, k] -> [..., n] (y = x W^T); NN: acts[i] [..., k] x weights[i] [k, n] -> [..., n]
     (dx = dy W). torch's products for other dtypes or sizes that are not multiples of 8."""
-    return _lib.native().products(layout, list(acts), list(weights))
+    return _native('products', layout, list(acts), list(weights))
 
 
 def linear(x: Tensor, w: Tensor) -> Tensor:
     """x W^T without bias: the product and its input gradient on atlas_linear_batch, the weight gradient
     split over the tokens (_wgrads)."""
-    return _lib.native().linear(x, w)
+    return _native('linear', x, w)
 
 
 def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj_weights, gate_weights, gate_biases,
@@ -770,7 +852,7 @@ def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj
     if conv_weights is not None and conv_weights[0].shape[-1] > 8:
         raise ValueError("the fused prologue supports depthwise convolutions of up to 8 taps")
     # one autograd node for all of it, with the products and weight gradients batched (csrc/host.cpp)
-    out = _lib.native().cell_prologue(x, norm_weight, float(eps), list(conv_weights) if conv_weights is not None else [],
+    out = _native('cell_prologue', x, norm_weight, float(eps), list(conv_weights) if conv_weights is not None else [],
                                       list(proj_weights), list(gate_weights or ()), list(gate_biases or ()) if gate_weights
                                       else [], q_gamma, k_gamma, heads, dim_head)
     return out[0], out[1], out[2], out[3], list(out[4:])

@@ -21,8 +21,7 @@ from typing import Callable
 import torch
 from torch import Tensor
 
-from . import _lib
-from .functional import AssocScan, assoc_scan, tensor_feature_map, window_sum
+from .functional import AssocScan, _native, assoc_scan, tensor_feature_map, window_sum
 
 __all__ = ["_sliding_sum_along_n", "assoc_scan", "AssocScan", "omega_store_chain", "apply_poly_features",
            "OmegaPolyFeatures", "OMEGA_GATE_OFF", "newtonschulz5"]
@@ -75,7 +74,7 @@ def _fused_chain(surprise, decay, last_update, am, last_momentum, gate, window, 
     """The chain in one kernel each way (atlas_omega_chain_fwd / _bwd), or None where they do not apply:
     one dtype (fp32 or bf16) on one GPU for the surprises and the scalars, at most two momentum orders
     and a window of at most 16. The separate scans and window sums serve everything else."""
-    return _lib.native().omega_chain(surprise, decay, last_update, am, last_momentum, gate, window, buf)
+    return _native('omega_chain', surprise, decay, last_update, am, last_momentum, gate, window, buf)
 
 
 def omega_store_chain(surprise: Tensor, decay_factor: Tensor, last_update: Tensor, *,
