@@ -722,13 +722,39 @@ struct CellPrologueFn : public Function<CellPrologueFn> {
 variable_list cell_prologue(const Tensor& x, const Tensor& norm_weight, double eps, const variable_list& convs,
                             const variable_list& projs, variable_list gw, variable_list gb, const OptTensor& q_gamma,
                             const OptTensor& k_gamma, int64_t heads, int64_t dim_head) {
+  // every list is indexed by position below, and the kernels read what the sizes here say
+  TORCH_CHECK_VALUE(x.dim() == 3 && kernel_dtype(x.scalar_type()), "x must be an fp32 or bf16 tensor [B, T, dim]");
+  TORCH_CHECK_VALUE(convs.empty() || convs.size() == 3, "conv_weights must be three (q, k, v), got ", convs.size());
+  TORCH_CHECK_VALUE(projs.size() >= 3, "proj_weights must be three (q, k, v), got ", projs.size());
+  TORCH_CHECK_VALUE(gw.empty() == gb.empty(), "gate_weights and gate_biases must both be given, got ", gw.size(), " and ",
+                    gb.size());
+  const int64_t dim = x.size(2), inner = heads * dim_head;
+  TORCH_CHECK_VALUE(heads >= 1 && dim_head >= 1 && norm_weight.numel() == dim, "norm_weight must hold dim = ", dim,
+                    " values, got ", norm_weight.sizes());
+  for (int i = 0; i < 3; ++i)
+    TORCH_CHECK_VALUE(projs[i].sizes() == at::IntArrayRef({inner, dim}), "proj_weights must be [", inner, ", ", dim,
+                      "] (heads * dim_head, dim), got ", projs[i].sizes());
+  int64_t gate_rows = 0, bias_rows = 0;
+  for (const Tensor& t : gw) {
+    TORCH_CHECK_VALUE(t.dim() == 2 && t.size(1) == dim, "gate_weights must be [heads, dim = ", dim, "], got ", t.sizes());
+    gate_rows += t.size(0);
+  }
+  for (const Tensor& t : gb) bias_rows += t.numel();
+  TORCH_CHECK_VALUE(gate_rows == bias_rows && gate_rows % heads == 0, "the gates have ", gate_rows, " weight rows and ",
+                    bias_rows, " biases for ", heads, " heads");
+  auto on_device = [&](const Tensor& t) { return t.device() == x.device(); };
+  bool fits = x.is_cuda() && on_device(norm_weight) && (!q_gamma.has_value() || on_device(*q_gamma)) &&
+              (!k_gamma.has_value() || on_device(*k_gamma));
+  for (const variable_list* l : {&convs, &projs, (const variable_list*)&gw, (const variable_list*)&gb})
+    for (const Tensor& t : *l) fits = fits && on_device(t);
+  TORCH_CHECK(fits, "the cell prologue runs on ROCm GPU tensors of one device only");
   c10::DeviceGuard guard(x.device());
   const at::ScalarType dt = x.scalar_type();
   auto cast = [&](const Tensor& t) { return t.scalar_type() == dt ? t : t.to(dt); };
   auto ocast = [&](const OptTensor& t) { return t.has_value() ? OptTensor(cast(*t)) : OptTensor(); };
   for (Tensor& t : gw) t = cast(t);
   for (Tensor& t : gb) t = cast(t);
-  if (gw.size() > 4) {
+  if (gw.size() > 4 || gb.size() != gw.size()) {   // the biases may come in another split than the weights
     gw = {at::cat(gw)};
     gb = {at::cat(gb)};
   }

@@ -849,6 +849,8 @@ def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj
     if x.dim() != 3:
         raise ValueError(f"x must be [B, T, dim], got {tuple(x.shape)}")
     _dt_code(x)   # fp32 or bf16
+    if conv_weights is not None and len(conv_weights) != 3:
+        raise ValueError(f"conv_weights must be three (q, k, v), got {len(conv_weights)}")
     if conv_weights is not None and conv_weights[0].shape[-1] > 8:
         raise ValueError("the fused prologue supports depthwise convolutions of up to 8 taps")
     # one autograd node for all of it, with the products and weight gradients batched (csrc/host.cpp)
