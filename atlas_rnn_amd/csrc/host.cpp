@@ -258,6 +258,8 @@ py::object recurrence(const Tensor& k, const Tensor& q, const Tensor& v, const T
 // the tensor feature map (rnn_memory.py:125-130)
 // ---------------------------------------------------------------------------------------------
 std::tuple<Tensor, Tensor> symmetrized(const Tensor& proj, int64_t d, at::ScalarType dt) {
+  TORCH_CHECK_VALUE(proj.dim() == 2 && d >= 1 && proj.size(0) == d + d * d, "the projection must be [d + d*d, m] for d = ", d,
+                    ", got ", proj.sizes());
   const Tensor p = aligned(proj.detach().to(dt));
   const int64_t m = p.size(1);
   const Tensor ps = like(p), pst = plain(p, {m, p.size(0)});
@@ -312,6 +314,7 @@ enum { kReplicate = 0, kReplicaSum = 1 };
 
 // one launch per dtype and four arrays: nrep copies stacked along the first axis, or their sum
 variable_list replicas(int op, int64_t nrep, at::TensorList in) {
+  TORCH_CHECK_VALUE(nrep >= 1, "the number of replicas must be at least 1, got ", nrep);
   variable_list xs, outs;
   for (const Tensor& t : in) xs.push_back(t.contiguous());
   for (const Tensor& x : xs) {
@@ -413,6 +416,8 @@ int64_t rows_of(const Tensor& t) { return t.numel() / std::max<int64_t>(t.size(-
 // up to four products over the same rows in one launch: NT y = x W^T, NN dx = dy W; torch's for other
 // dtypes, or sizes that are not multiples of 8
 variable_list products(int layout, const variable_list& acts, const variable_list& weights) {
+  TORCH_CHECK_VALUE(!acts.empty() && acts.size() == weights.size(), "products of ", acts.size(), " activations with ",
+                    weights.size(), " weights");
   const int64_t m = rows_of(acts[0]);
   bool ok = acts.size() <= 4;
   for (size_t i = 0; i < acts.size(); ++i)
@@ -424,6 +429,11 @@ variable_list products(int layout, const variable_list& acts, const variable_lis
       outs.push_back(layout == ATLAS_GEMM_NT ? at::linear(acts[i], weights[i]) : at::matmul(acts[i], weights[i]));
     return outs;
   }
+  for (size_t i = 0; i < acts.size(); ++i)   // the kernel reads what the sizes say, on the current device
+    TORCH_CHECK(weights[i].dim() == 2 && weights[i].size(layout == ATLAS_GEMM_NT ? 1 : 0) == acts[i].size(-1) &&
+                    acts[i].device() == acts[0].device() && weights[i].device() == acts[0].device(),
+                "the products' operands do not fit: ", acts[i].sizes(), " on ", acts[i].device(), " and ",
+                weights[i].sizes(), " on ", weights[i].device());
   TORCH_CHECK(acts[0].is_cuda(), "the bf16 products run on ROCm GPU tensors only");
   variable_list a, w;
   int ns[4], ks[4];
@@ -448,6 +458,8 @@ variable_list products(int layout, const variable_list& acts, const variable_lis
 // dW = dy^T x over every leading axis, for each (dy, x) pair: bf16 pairs over the same tokens in one
 // launch (csrc/wgrad.hip); others torch's product over token slices
 variable_list wgrads(const variable_list& dys_in, const variable_list& xs_in, at::ScalarType dt) {
+  TORCH_CHECK_VALUE(!dys_in.empty() && dys_in.size() == xs_in.size(), "weight gradients of ", dys_in.size(), " and ",
+                    xs_in.size(), " activations");
   variable_list dys, xs, out;
   for (size_t i = 0; i < dys_in.size(); ++i) {
     dys.push_back(dys_in[i].reshape({-1, dys_in[i].size(-1)}));
@@ -459,6 +471,9 @@ variable_list wgrads(const variable_list& dys_in, const variable_list& xs_in, at
     ok = ok && dys[i].scalar_type() == at::kBFloat16 && xs[i].scalar_type() == at::kBFloat16 && dys[i].size(1) % 8 == 0 &&
          xs[i].size(1) % 8 == 0 && dys[i].size(0) == n && xs[i].size(0) == n;
   if (ok) {
+    for (size_t i = 0; i < dys.size(); ++i)
+      TORCH_CHECK(dys[i].device() == dys[0].device() && xs[i].device() == dys[0].device(),
+                  "the weight gradients' operands are on more than one device");
     TORCH_CHECK(dys[0].is_cuda(), "the bf16 weight gradients run on ROCm GPU tensors only");
     int os[4], is[4];
     const void *dp[4], *xp[4];
