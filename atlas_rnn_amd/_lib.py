@@ -48,6 +48,7 @@ EXPORTED_SYMBOLS = (
     "atlas_scan_bwd",
     "atlas_window_sum",
     "atlas_omega_chain_fwd",
+    "atlas_omega_chain_fwd_keep",
     "atlas_omega_chain_bwd",
     "atlas_omega_chain_workspace_bytes",
     "atlas_affine_scan_fwd",
@@ -158,6 +159,8 @@ def load(path: str | None = None) -> ctypes.CDLL:
     lib.atlas_window_sum.argtypes = [i32, i64, i64, i64, i32, i32, vp, vp, vp]
     lib.atlas_omega_chain_fwd.restype = i32
     lib.atlas_omega_chain_fwd.argtypes = [i32, i64, i64, i64, i32, i32] + [vp] * 12
+    lib.atlas_omega_chain_fwd_keep.restype = i32
+    lib.atlas_omega_chain_fwd_keep.argtypes = [i32, i64, i64, i64, i32, i32] + [vp] * 14
     lib.atlas_omega_chain_bwd.restype = i32
     lib.atlas_omega_chain_bwd.argtypes = [i32, i64, i64, i64, i32, i32] + [vp] * 18 + [i64, vp]
     lib.atlas_omega_chain_workspace_bytes.restype = i64

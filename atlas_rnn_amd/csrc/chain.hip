@@ -33,6 +33,7 @@ struct Args {
   int64_t p;
   const T *s, *decay, *last, *am, *lm0, *gate, *buf;   // am [O, bh, n], lm0 [O, bh, p], buf [bh, e-1, p]
   T *update, *moms, *lm1, *buf1;                       // forward outputs (moms null: no backward follows)
+  T *kept, *kdecay;                                    // copies of update and decay for the backward (null: none)
   const T *dup, *dlm1, *dbuf1;                         // backward: gradients of the outputs (null: zero)
   const T *upd;                                        // backward: the forward's update
   const T *msrc;                                       // backward: the momenta (order 0: unused)
@@ -106,6 +107,7 @@ __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
   const bool off = gates_off(a.gate, (int64_t)a.bh * n);
   const T* sp = a.s + rp * n + col;
   T* up = a.update + rp * (n + 1) + col;
+  T* kp = a.kept ? a.kept + rp * (n + 1) + col : nullptr;
 
   float m[O > 0 ? O : 1][V], c[V], hist[E > 1 ? E - 1 : 1][V];
   ldv<T, V>(a.last + rp + col, c);
@@ -127,6 +129,7 @@ __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
   }
   float zero[V] = {};
   if (act) stv<T, V>(up, off ? zero : c);
+  if (act && kp) stv<T, V>(kp, off ? zero : c);
 
   float cur[kU][V], nxt[kU][V];
   float sc[2 + (O > 0 ? O : 1)], scn[2 + (O > 0 ? O : 1)];   // lane u: the scalars of step u of the group
@@ -148,6 +151,7 @@ __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
 #pragma unroll
     for (int k = 0; k < 2 + O; ++k) sc[k] = scn[k];
     load(nxt, scn, t0 + kU);
+    if (a.kdecay && blockIdx.x == 0 && lane < kU && t0 + lane < n) a.kdecay[(int64_t)row * n + t0 + lane] = from_f32<T>(sc[0]);
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int t = t0 + u;
@@ -189,6 +193,7 @@ __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
 #pragma unroll
         for (int i = 0; i < V; ++i) c[i] = keep * c[i] + w[i];
         if (act) stv<T, V>(up + (int64_t)(t + 1) * p, off ? zero : c);
+        if (act && kp) stv<T, V>(kp + (int64_t)(t + 1) * p, off ? zero : c);
       }
     }
   }
@@ -211,12 +216,13 @@ __global__ __launch_bounds__(64) void k_chain_bwd(Args<T> a) {
   const bool live = act && !off && a.dup;     // dupdate reaches this column
   const T* dp = a.dup ? a.dup + rp * (n + 1) + col : nullptr;
   const T* cp = a.upd + rp * (n + 1) + col;   // row t: c_{t-1}
-  const T* bp[O > 0 ? O : 1];                 // momenta of order o (order 0: the surprises, the base)
+  const T* bp[O > 0 ? O : 1];                 // momenta of order o (order 0: the surprises, which only the gate's
+                                              // gradient needs: any readable rows where they are absent)
   if constexpr (O > 0) {
 #pragma unroll
     for (int o = 0; o < O; ++o) bp[o] = a.msrc + ((int64_t)o * a.bh + row) * n * p + col;
   } else {
-    bp[0] = a.s + rp * n + col;
+    bp[0] = a.s ? a.s + rp * n + col : cp;
   }
   float* part = a.part + ((int64_t)row * gridDim.x + blockIdx.x) * K * n;
 
@@ -440,16 +446,16 @@ int64_t atlas_omega_chain_workspace_bytes(int64_t bh, int64_t n, int64_t p, int 
   return bh * waves_per_row(p) * (2 + order) * n * (int64_t)sizeof(float);
 }
 
-int atlas_omega_chain_fwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
-                          const void* decay, const void* last_update, const void* momentum, const void* last_momentum,
-                          const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
-                          void* next_buffer, void* stream) {
+int atlas_omega_chain_fwd_keep(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
+                               const void* decay, const void* last_update, const void* momentum, const void* last_momentum,
+                               const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
+                               void* next_buffer, void* kept_update, void* kept_decay, void* stream) {
   if (bad(bh, n, p, order, window)) return ATLAS_MEM_ERR_SHAPE;
   if (!surprise || !decay || !last_update || !update || (order > 0 && (!momentum || !last_momentum || !next_momentum)) ||
       (window > 1 && !next_buffer))
     return ATLAS_MEM_ERR_NULL;
   for (const void* q : {surprise, last_update, last_momentum, buffer, (const void*)update, (const void*)moments,
-                        (const void*)next_momentum, (const void*)next_buffer})
+                        (const void*)next_momentum, (const void*)next_buffer, (const void*)kept_update})
     if (off16(q)) return ATLAS_MEM_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto go = [&](auto tag) {
@@ -459,11 +465,20 @@ int atlas_omega_chain_fwd(int dtype, int64_t bh, int64_t n, int64_t p, int order
     a.s = (const T*)surprise; a.decay = (const T*)decay; a.last = (const T*)last_update; a.am = (const T*)momentum;
     a.lm0 = (const T*)last_momentum; a.gate = (const T*)gate; a.buf = (const T*)buffer;
     a.update = (T*)update; a.moms = (T*)moments; a.lm1 = (T*)next_momentum; a.buf1 = (T*)next_buffer;
+    a.kept = (T*)kept_update; a.kdecay = (T*)kept_decay;
     return run<T>(a, order, false, s);
   };
   if (dtype != ATLAS_DT_BF16 && dtype != ATLAS_DT_F32) return ATLAS_MEM_ERR_DTYPE;
   const hipError_t err = dtype == ATLAS_DT_BF16 ? go(bf16{}) : go(float{});
   return err == hipSuccess ? ATLAS_MEM_OK : ATLAS_MEM_ERR_LAUNCH;
+}
+
+int atlas_omega_chain_fwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
+                          const void* decay, const void* last_update, const void* momentum, const void* last_momentum,
+                          const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
+                          void* next_buffer, void* stream) {
+  return atlas_omega_chain_fwd_keep(dtype, bh, n, p, order, window, surprise, decay, last_update, momentum, last_momentum,
+                                    gate, buffer, update, moments, next_momentum, next_buffer, nullptr, nullptr, stream);
 }
 
 int atlas_omega_chain_bwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
@@ -473,7 +488,8 @@ int atlas_omega_chain_bwd(int dtype, int64_t bh, int64_t n, int64_t p, int order
                           void* dlast_momentum, void* dgate, void* dbuffer, void* workspace, int64_t workspace_bytes,
                           void* stream) {
   if (bad(bh, n, p, order, window)) return ATLAS_MEM_ERR_SHAPE;
-  if (!surprise || !decay || !update || !dsurprise || !ddecay || !dlast_update || !workspace || (gate && !dgate) ||
+  if (!decay || !update || !dsurprise || !ddecay || !dlast_update || !workspace || (dgate && !gate) ||
+      (order == 0 && dgate && !surprise) ||
       (order > 0 && (!momentum || !last_momentum || !moments || !dmomentum || !dlast_momentum)))
     return ATLAS_MEM_ERR_NULL;
   for (const void* q : {surprise, update, last_momentum, moments, dupdate, dnext_momentum, dnext_buffer,
@@ -495,7 +511,7 @@ int atlas_omega_chain_bwd(int dtype, int64_t bh, int64_t n, int64_t p, int order
     if (err != hipSuccess) return err;
     const int64_t outs = bh * (2 + order) * n;
     hipLaunchKernelGGL(k_chain_sum<T>, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, (int)bh, (int)n,
-                       waves_per_row(p), order, a.part, (T*)ddecay, gate ? (T*)dgate : nullptr, (T*)dmomentum);
+                       waves_per_row(p), order, a.part, (T*)ddecay, (T*)dgate, (T*)dmomentum);
     return hipGetLastError();
   };
   if (dtype != ATLAS_DT_BF16 && dtype != ATLAS_DT_F32) return ATLAS_MEM_ERR_DTYPE;

@@ -802,12 +802,20 @@ struct OmegaChainFn : public Function<OmegaChainFn> {
     const int64_t BH = s.size(0), n = s.size(1), p = s.size(2), O = am.defined() ? am.size(0) : 0;
     const Tensor update = plain(s, {BH, n + 1, p}), moms = O && grad ? plain(s, {O, BH, n, p}) : Tensor();
     const Tensor next_lm = O ? plain(s, {O, BH, p}) : Tensor(), next_buf = window > 1 ? plain(s, {BH, window - 1, p}) : Tensor();
-    check(atlas_omega_chain_fwd(dt_code(s), BH, n, p, (int)O, (int)window, ptr(s), ptr(decay), ptr(last), ptr(am), ptr(lm),
-                                ptr(gate), ptr(buf), mptr(update), mptr(moms), mptr(next_lm), mptr(next_buf), stream_of(s)),
+    // the backward has its own copies of the updates and the decays, so that the caller may edit the returned
+    // and the given ones in place before it (a second write of the updates: 91.4 -> 93.6 us forward and backward at 16 x 64 x 8192 fp32)
+    const Tensor kept = grad ? like(update) : Tensor(), kept_decay = grad ? like(decay) : Tensor();
+    check(atlas_omega_chain_fwd_keep(dt_code(s), BH, n, p, (int)O, (int)window, ptr(s), ptr(decay), ptr(last), ptr(am),
+                                     ptr(lm), ptr(gate), ptr(buf), mptr(update), mptr(moms), mptr(next_lm), mptr(next_buf),
+                                     mptr(kept), mptr(kept_decay), stream_of(s)),
           "atlas_omega_chain_fwd");
-    ctx->save_for_backward({s, decay, am, lm, gate, update, moms});
-    ctx->saved_data["window"] = window;
-    ctx->saved_data["has_buf"] = buf.defined();
+    if (grad) {   // (only the gradient of a gate on the surprises themselves reads them)
+      const bool dgate = gate.defined() && gate.requires_grad();
+      ctx->save_for_backward({!O && dgate ? s : Tensor(), kept_decay, am, lm, gate, kept, moms});
+      ctx->saved_data["dgate"] = dgate;
+      ctx->saved_data["window"] = window;
+      ctx->saved_data["has_buf"] = buf.defined();
+    }
     variable_list out{update};
     if (O) out.push_back(next_lm);
     if (window > 1) out.push_back(next_buf);
@@ -816,18 +824,20 @@ struct OmegaChainFn : public Function<OmegaChainFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const variable_list sv = ctx->get_saved_variables();
     const Tensor &s = sv[0], &decay = sv[1], &am = sv[2], &lm = sv[3], &gate = sv[4], &update = sv[5], &moms = sv[6];
-    c10::DeviceGuard guard(s.device());
-    const int64_t BH = s.size(0), n = s.size(1), p = s.size(2), O = am.defined() ? am.size(0) : 0;
+    c10::DeviceGuard guard(update.device());
+    const int64_t BH = update.size(0), n = update.size(1) - 1, p = update.size(2), O = am.defined() ? am.size(0) : 0;
     const int64_t e = ctx->saved_data["window"].toInt();
     size_t i = 1;
     const Tensor dup = aligned(g[0]), dlm = O ? aligned(g[i++]) : Tensor(), dbo = e > 1 ? aligned(g[i++]) : Tensor();
-    const Tensor ds = like(s), dd = like(decay), dam = like(am), dlm0 = like(lm), dg = like(gate), dlast = plain(s, {BH, p});
-    const Tensor dbuf = ctx->saved_data["has_buf"].toBool() ? plain(s, {BH, e - 1, p}) : Tensor();
+    const Tensor ds = plain(update, {BH, n, p}), dd = like(decay), dam = like(am), dlm0 = like(lm),
+                 dlast = plain(update, {BH, p});
+    const Tensor dg = ctx->saved_data["dgate"].toBool() ? like(gate) : Tensor();
+    const Tensor dbuf = ctx->saved_data["has_buf"].toBool() ? plain(update, {BH, e - 1, p}) : Tensor();
     const int64_t bytes = atlas_omega_chain_workspace_bytes(BH, n, p, (int)O);
-    const Tensor ws = scratch(s, bytes);
-    check(atlas_omega_chain_bwd(dt_code(s), BH, n, p, (int)O, (int)e, ptr(s), ptr(decay), ptr(am), ptr(lm), ptr(gate),
+    const Tensor ws = scratch(update, bytes);
+    check(atlas_omega_chain_bwd(dt_code(update), BH, n, p, (int)O, (int)e, ptr(s), ptr(decay), ptr(am), ptr(lm), ptr(gate),
                                 ptr(update), ptr(moms), ptr(dup), ptr(dlm), ptr(dbo), mptr(ds), mptr(dd), mptr(dlast),
-                                mptr(dam), mptr(dlm0), mptr(dg), mptr(dbuf), mptr(ws), bytes, stream_of(s)),
+                                mptr(dam), mptr(dlm0), mptr(dg), mptr(dbuf), mptr(ws), bytes, stream_of(update)),
           "atlas_omega_chain_bwd");
     return {ds, dd, dlast, dam, dlm0, dg, dbuf, Tensor(), Tensor()};
   }

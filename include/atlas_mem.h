@@ -228,8 +228,16 @@ int atlas_omega_chain_fwd(int dtype, int64_t bh, int64_t n, int64_t p, int order
                           const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
                           void* next_buffer, void* stream);
 
+/* The same with copies of update and decay for the backward (kept_update [bh, n + 1, p], kept_decay
+ * [bh, n]; either may be NULL), so that the caller may change the originals before it. */
+int atlas_omega_chain_fwd_keep(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
+                               const void* decay, const void* last_update, const void* momentum, const void* last_momentum,
+                               const void* gate, const void* buffer, void* update, void* moments, void* next_momentum,
+                               void* next_buffer, void* kept_update, void* kept_decay, void* stream);
+
 /* Gradients of atlas_omega_chain_fwd from those of its outputs (each NULL: zero) and the forward's
- * update and moments. dgate iff gate; dbuffer NULL: not wanted. workspace: at least
+ * update and moments. dgate (with a gate) and dbuffer NULL: not wanted. surprise is read for
+ * dgate of order 0 alone and may be NULL otherwise. workspace: at least
  * atlas_omega_chain_workspace_bytes(bh, n, p, order) bytes. */
 int atlas_omega_chain_bwd(int dtype, int64_t bh, int64_t n, int64_t p, int order, int window, const void* surprise,
                           const void* decay, const void* momentum, const void* last_momentum, const void* gate,

@@ -109,3 +109,45 @@ def test_chain_route():
     assert call(omega_gate=x["omega_gate"].double()) is None
     assert call(adaptive_momentum=x["adaptive_momentum"].expand(3, -1, -1)) is None
     assert call(surprise=x["surprise"][..., :0]) is None
+
+
+@pytest.mark.parametrize("order,gate", [(0, False), (0, True), (1, True), (2, False)])
+def test_chain_edits_in_place_before_the_backward(order, gate):
+    """The returned tensors may be edited in place before the backward, and so may the surprises and decays (the
+    surprises not where the gradient of a gate on them reads them: a version error)."""
+    x = {k: v.cuda() for k, v in _inputs(2, 11, (70,), order, False, gate, 3, True, seed=8, dt=torch.float32).items()}
+
+    def run(edit):
+        leaves = {k: v.clone().requires_grad_() for k, v in x.items()}
+        ins = {k: v * 1 for k, v in leaves.items()}
+        out = omega_store_chain(**ins, omega_window=3)
+        loss = sum((o * torch.linspace(-1, 1, o.numel(), device="cuda").view(o.shape)).sum() for o in out if o is not None)
+        with torch.no_grad():
+            for t in edit(ins, out):
+                t.mul_(0.5)
+        names = sorted(leaves)
+        return torch.autograd.grad(loss, [leaves[k] for k in names])
+
+    want = run(lambda ins, out: ())
+    for edit in (lambda ins, out: (o for o in out if o is not None), lambda ins, out: (ins["decay_factor"],)):
+        assert all(torch.equal(a, b) for a, b in zip(run(edit), want))
+    edit = lambda ins, out: (ins["surprise"],)
+    if order == 0 and gate:
+        with pytest.raises(RuntimeError, match="modified by an inplace"):
+            run(edit)
+    else:
+        assert all(torch.equal(a, b) for a, b in zip(run(edit), want))
+
+
+def test_chain_without_a_gradient_of_the_gate():
+    """A gate that asks for no gradient: the other gradients are those of one that does."""
+    for order in (0, 1):
+        x = {k: v.cuda() for k, v in _inputs(3, 9, (70,), order, False, True, 4, True, seed=9, dt=torch.float32).items()}
+        grads = []
+        for ask in (True, False):
+            leaves = {k: v.clone().requires_grad_(ask or k != "omega_gate") for k, v in x.items()}
+            out = omega_store_chain(**leaves, omega_window=4)
+            names = sorted(k for k in leaves if k != "omega_gate")
+            grads.append(torch.autograd.grad(sum((o * o).sum() for o in out if o is not None), [leaves[k] for k in names]))
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(*grads))
