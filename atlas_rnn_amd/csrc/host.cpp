@@ -226,8 +226,11 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
   if (at::GradMode::is_enabled())
     for (const Tensor* t : {&kc, &qc, &vc, &lc, &dc, &bc, &gc, &Src, &S0c, &Zc, &Bc})
       grad = grad || (t->defined() && t->requires_grad());
-  if (T == 1) {
-    if (!grad) {   // decode: one launch, no saved buffer (rnn_transformer.py:863-900 through the cell at T = 1)
+  if (T == 1 && !grad) {
+    bool tangent = false;   // (a forward-mode tangent: the node refuses it)
+    for (const Tensor* t : {&kc, &qc, &vc, &lc, &dc, &bc, &gc, &Src, &S0c, &Zc, &Bc})
+      tangent = tangent || (t->defined() && t->_fw_grad(0).defined());
+    if (!tangent) {   // decode: one launch, no saved buffer (rnn_transformer.py:863-900 through the cell at T = 1)
       o = rec_outputs(p, kc);
       const atlas_mem_fwd_args a = fwd_args(kc, qc, vc, lc, dc, bc, gc, Src, S0c, Zc, Bc, o);
       check(atlas_mem_step(&p, &a, stream_of(kc)), "atlas_mem_step");

@@ -53,6 +53,9 @@ def _require_gpu(*ts: Tensor | None) -> torch.device:
     return dev
 
 
+_is_tracing = torch._C._is_tracing
+
+
 class _no_trace:
     """torch.jit.trace's recording paused."""
 
@@ -102,7 +105,7 @@ class _TracedFn(torch.autograd.Function):
             ctx.outs = []
             _map_tensors(call(ctx.ins), ctx.outs.append)
             outs = [o.detach() for o in ctx.outs]
-        if torch._C._is_tracing():   # outputs that the trace knows
+        if _is_tracing():   # outputs that the trace knows
             known = [torch.empty(list(o.shape), dtype=o.dtype, device=o.device) for o in outs]
             with _no_trace():
                 for e, o in zip(known, outs):
@@ -122,7 +125,7 @@ class _TracedFn(torch.autograd.Function):
 def _native(op: str, *args):
     """The native operator `op` (csrc/host.cpp) on args; None where it does not take them."""
     fn = getattr(_lib.native(), op)
-    if not torch._C._is_tracing():
+    if not _is_tracing():
         return fn(*args)
     args = _map_tensors(args, lambda t: t)
     with _no_trace(), torch.no_grad():   # which outputs there are, and whether the operator takes the operands

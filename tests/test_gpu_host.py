@@ -67,6 +67,18 @@ def test_refusals_stay():
         am.memory_recurrence(x["k"], x["q"], x["v"], x["lr"], x["decay"], window=34)
 
 
+@pytest.mark.parametrize("name", ["k", "beta", "S0", "buffer"])
+def test_one_token_refuses_transforms_too(name):
+    x = _ops(t=1)
+    call = lambda t: am.memory_recurrence(**{**x, name: t}, window=E)[0]
+    with fwd_ad.dual_level(), pytest.raises(RuntimeError):
+        call(fwd_ad.make_dual(x[name], torch.ones_like(x[name])))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: call(t).float().sum())(x[name])
+    with pytest.raises(RuntimeError):
+        torch.vmap(call)(torch.stack([x[name], x[name]]))
+
+
 def test_hooks_versions_and_partial_gradients():
     x = _ops(seed=1)
     packed = []
