@@ -598,6 +598,27 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
     raise RuntimeError("memory_recurrence: a valid problem was not taken by the native path")
 
 
+class MemoryRecurrenceFn:
+    """The recurrence on operands as the kernels take them: y, S_T, Z_T, buffer_out = apply(k, q, v, lr, decay,
+    beta, gate, S_ref, S0, Z0, buffer, cfg).
+
+    k, q, v, lr, decay, beta, gate: one dtype (fp32 or bf16), contiguous; states fp32. Nothing is cast, padded or
+    split: other operands raise. Z_T / buffer_out are empty tensors when momentum is off / window == 1."""
+
+    @staticmethod
+    def apply(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg: RecurrenceConfig):
+        check_operands(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, window=cfg.window, dtype=k.dtype,
+                       contiguous=True)
+        dev = _require_gpu(k, q, v, lr, decay, S_ref, S0)
+        prob = _problem(cfg, *k.shape, v.shape[-1], beta is not None, gate, buf is not None, k.dtype)
+        _lib.check(_lib.load().atlas_mem_validate(ctypes.byref(prob)), "atlas_mem_validate")
+        y, S_T, Z_T, buf_out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg.window,
+                                       cfg.map_degree if cfg.map_mode == 'elementwise' else 1, cfg.clamp_every or None,
+                                       bool(cfg.clamp_final))
+        empty = torch.empty(0, device=dev)
+        return y, S_T, Z_T if Z_T is not None else empty, buf_out if buf_out is not None else empty
+
+
 class AtlasOmegaFunction:
     """Drop-in for atlas_pytorch/cuda/atlas_omega_autograd.py:87-204.
 

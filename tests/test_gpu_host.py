@@ -122,3 +122,25 @@ def test_side_stream_uses_its_own_stream():
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("clamp", [None, 16])
+def test_recurrence_function_on_canonical_operands(clamp):
+    x = _ops(seed=3)
+    cfg = F.RecurrenceConfig(window=E, clamp_every=clamp, clamp_final=False)
+    names = ("k", "q", "v", "lr", "decay", "beta", "gate", "S_ref", "S0", "Z0", "buffer")
+    grads, outs = [], []
+    for call in (lambda o: F.MemoryRecurrenceFn.apply(*o, cfg),
+                 lambda o: am.memory_recurrence(*o, window=E, clamp_every=clamp, clamp_final=False)):
+        o = [x[n].clone().requires_grad_() for n in names]
+        out = call(o)
+        outs.append(out)
+        grads.append(torch.autograd.grad(sum(t.float().square().sum() for t in out), o))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs)) and all(torch.equal(a, b) for a, b in zip(*grads))
+    y, S, Z, B = F.MemoryRecurrenceFn.apply(*[x[n] for n in names[:5]], None, None, x["S_ref"], x["S0"], None, None,
+                                            F.RecurrenceConfig(window=1))
+    assert y.shape == x["v"].shape and S.shape == x["S0"].shape and Z.numel() == 0 and B.numel() == 0
+    with pytest.raises(RuntimeError, match="status"):   # a buffer without a window
+        F.MemoryRecurrenceFn.apply(*[x[n] for n in names[:5]], None, None, x["S_ref"], x["S0"], None, x["buffer"],
+                                   F.RecurrenceConfig(window=1))

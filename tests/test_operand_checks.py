@@ -5,7 +5,7 @@ memory_recurrence, MemoryRecurrenceFn and RecurrencePlan)."""
 import pytest
 import torch
 
-from atlas_rnn_amd.functional import check_operands
+from atlas_rnn_amd.functional import MemoryRecurrenceFn, RecurrenceConfig, check_operands
 
 BH, T, D, E = 4, 10, 8, 4
 
@@ -75,3 +75,17 @@ def test_dtype_and_contiguity_when_requested():
     bad_state[7] = bad_state[7].to(torch.bfloat16)
     with pytest.raises(ValueError, match="S_ref must be torch.float32"):
         check_operands(*bad_state, window=E, dtype=torch.bfloat16)
+
+
+def test_recurrence_function_takes_canonical_operands_only():
+    o = _ops(**{n: torch.zeros(*s) for n, s in (("k", (BH, T, 32)), ("q", (BH, T, 32)), ("v", (BH, T, 32)),
+                                               ("S_ref", (BH, 32, 32)), ("S0", (BH, 32, 32)), ("Z0", (BH, 32, 32)),
+                                               ("buffer", (BH, E - 1, 32, 32)))})
+    names = ("k", "q", "v", "lr", "decay", "beta", "gate", "S_ref", "S0", "Z0", "buffer")
+    call = lambda **kw: MemoryRecurrenceFn.apply(*[{**o, **kw}[n] for n in names], RecurrenceConfig(window=E))
+    with pytest.raises(ValueError, match="contiguous"):
+        call(q=torch.zeros(BH, 32, T).transpose(1, 2))
+    with pytest.raises(ValueError, match="must be torch.float32"):
+        call(S0=o["S0"].double())
+    with pytest.raises(RuntimeError, match="GPU"):
+        call()
