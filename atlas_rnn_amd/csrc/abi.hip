@@ -218,8 +218,9 @@ Plan make_plan_shared(const atlas_mem_problem* p, bool serial_clamp, int share) 
   int Lc = CH;
   if (p->clamp_every > 0 && p->clamp_every % CH != 0) Lc = largest_divisor_at_most(p->clamp_every, CH);
   const int Lb = largest_divisor_at_most(Lc, bwd_chunk_cap(p->dtype));
-  // the forward saves the state at every backward-chunk boundary: at most one inside a chunk
-  if (Lc / Lb > 2) Lc = Lb;
+  // the forward saves the state at every backward-chunk boundary: at most one inside a chunk, on a group of eight
+  // tokens (the records' chains run in such groups); clamp_every 100 in bf16 takes chunks of 25, not 2 x 25
+  if (Lc / Lb > 2 || (Lc / Lb == 2 && Lb % 8 != 0)) Lc = Lb;
   const int H = p->window - 1;
   if (Lb < H) { pl.status = ATLAS_MEM_ERR_UNSUPPORTED; return pl; }
   // clamp_every with no divisor of at least kMinClampChunk in range (37, 74, ...) would walk the
@@ -409,10 +410,7 @@ int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream
   float* coef = reinterpret_cast<float*>(rec.coef);
   T* wsh = reinterpret_cast<T*>(rec.wsh);
   Geom g = pl.g;
-  if (infer) {
-    if (g.Lmid % 8 != 0) return ATLAS_MEM_ERR_LAUNCH;   // refused with a backward: refused here too
-    g.Lmid = 0;
-  }
+  if (infer) g.Lmid = 0;
   const bool brec = !pl.cbwd && !infer;
   // chunk coefficient records of the forward and of the backward (one launch, inputs only)
   constexpr int CHF = sizeof(T) == 2 ? 64 : 32, CHB = sizeof(T) == 2 ? 32 : 16;

@@ -88,6 +88,17 @@ def test_clamp_every_saved_bytes_stay_bounded(lib, every):
     assert lib.atlas_mem_saved_bytes(ctypes.byref(p)) <= 32 * (4096 // 8) * 2 * st + 64 * 2 ** 20
 
 
+@pytest.mark.parametrize("dtype,every,chunk", [(_lib.DT_BF16, 40, 20), (_lib.DT_BF16, 50, 25), (_lib.DT_BF16, 100, 25),
+                                               (_lib.DT_BF16, 300, 30), (_lib.DT_F32, 20, 10), (_lib.DT_F32, 48, 12),
+                                               (_lib.DT_F32, 120, 15)])
+def test_clamp_every_whose_half_chunk_is_no_group_of_eight(lib, dtype, every, chunk):
+    # a forward chunk may hold two backward chunks only where they meet on a group of eight tokens; these take
+    # the backward's chunk on both sides, the plan of clamp_every = chunk
+    sizes = [lib.atlas_mem_saved_bytes(ctypes.byref(_prob(dtype=dtype, clamp_every=c, seq_len=every * chunk)))
+             for c in (every, chunk)]
+    assert sizes[0] == sizes[1] > 0
+
+
 def test_sizes(lib):
     p = _prob()
     st = 64 * 64 * 4
