@@ -279,7 +279,8 @@ size_t coef_rec_floats(int ch) { return (size_t)2 * ch + 8 + 4 * (ch + kHaloPad)
 // floats per backward chunk of the scalar-gradient inputs (ScalarBlock: Lm, hS, hZ, fS, fZ, Grams)
 size_t scalar_block_floats(int ch) { return (size_t)ch * (ch + kHaloPad) + 2 * (ch + kHaloPad) + 2 * ch + 4; }
 
-SavedLayout saved_layout(const Plan& pl) {
+// records: whether the plan has coefficient records of its own (the exact sequence of a dual plan reads the fast one's).
+SavedLayout saved_layout(const Plan& pl, bool records = true) {
   const Geom& g = pl.g;
   SavedLayout L{};
   const size_t st = (size_t)g.DV * g.DK * sizeof(float);
@@ -292,11 +293,11 @@ SavedLayout saved_layout(const Plan& pl) {
   const bool brec = !pl.cbwd;
   L.rw = off; off += align256(brec ? (size_t)g.BH * g.ncb * 2 * st : chunk_bwd_states_bytes(g));
   // forward scratch: per-chunk coefficient records and Ws[s, t-1] blocks
-  L.coef = off; off += align256((size_t)g.BH * g.nc * coef_rec_floats(pl.CH) * sizeof(float));
-  L.wsh = off; off += align256((size_t)g.BH * g.nc * pl.CH * (pl.CH + kHaloPad) * pl.esize);
+  L.coef = off; off += align256(records ? (size_t)g.BH * g.nc * coef_rec_floats(pl.CH) * sizeof(float) : 0);
+  L.wsh = off; off += align256(records ? (size_t)g.BH * g.nc * pl.CH * (pl.CH + kHaloPad) * pl.esize : 0);
   // the backward's chunk records (input-only: formed in the forward's coefficient launch)
-  L.bcoef = off; off += align256(brec ? (size_t)g.BH * pl.gb.nc * coef_rec_floats(pl.CHB) * sizeof(float) : 0);
-  L.bwsh = off; off += align256(brec ? (size_t)g.BH * pl.gb.nc * pl.CHB * (pl.CHB + kHaloPad) * pl.esize : 0);
+  L.bcoef = off; off += align256(brec && records ? (size_t)g.BH * pl.gb.nc * coef_rec_floats(pl.CHB) * sizeof(float) : 0);
+  L.bwsh = off; off += align256(brec && records ? (size_t)g.BH * pl.gb.nc * pl.CHB * (pl.CHB + kHaloPad) * pl.esize : 0);
   L.bufc = off; off += align256(walk_with_buffer(pl) ? (size_t)g.BH * bufw::kCorrFloats * sizeof(float) : 0);
   L.total = off;
   return L;
@@ -343,7 +344,7 @@ Plan make_plan(const atlas_mem_problem* p, bool serial_clamp) {
 }
 
 // `saved` of a dual plan: the flag (256 bytes), then the segment-parallel sequence's layout, then the
-// exact sequence's.
+// exact sequence's, without records of its own.
 struct DualLayout {
   size_t fast, exact, total;
 };
@@ -351,7 +352,7 @@ DualLayout dual_layout(const Plan& fast, const Plan& exact) {
   DualLayout D{};
   D.fast = 256;
   D.exact = D.fast + saved_layout(fast).total;
-  D.total = D.exact + saved_layout(exact).total;
+  D.total = D.exact + saved_layout(exact, false).total;
   return D;
 }
 
@@ -398,7 +399,7 @@ int run_fwd(const Plan& pl, const atlas_mem_fwd_args* x, float* saved, hipStream
   a.k = (const T*)x->k; a.q = (const T*)x->q; a.v = (const T*)x->v;
   a.lr = (const T*)x->lr; a.decay = (const T*)x->decay; a.beta = (const T*)x->beta; a.gate = (const T*)x->gate;
   a.S_ref = x->S_ref; a.S0 = x->S0; a.Z0 = x->Z0; a.buf_in = x->buffer_in;
-  const SavedLayout SL = saved_layout(pl);
+  const SavedLayout SL = saved_layout(pl, !made);
   unsigned char* sv = reinterpret_cast<unsigned char*>(saved);
   a.y = (T*)x->y; a.S_T = x->S_T; a.Z_T = x->Z_T; a.buf_out = x->buffer_out;
   a.buf_corr = nullptr;
@@ -453,7 +454,7 @@ int run_bwd(const Plan& pl, const atlas_mem_bwd_args* x, const float* saved, voi
             const Records* made = nullptr) {
   const Geom& gb = pl.gb;
   const BwdLayout L = bwd_layout(pl);
-  const SavedLayout SL = saved_layout(pl);
+  const SavedLayout SL = saved_layout(pl, !made);
   unsigned char* w = static_cast<unsigned char*>(ws);
   const unsigned char* sv = reinterpret_cast<const unsigned char*>(saved);
   BwdPtrs<T> a{};

@@ -99,6 +99,17 @@ def test_clamp_every_whose_half_chunk_is_no_group_of_eight(lib, dtype, every, ch
     assert sizes[0] == sizes[1] > 0
 
 
+def test_dual_plan_keeps_one_set_of_records(lib):
+    # clamp points on chunk ends: the flag, the unclamped plan's buffer, and of the exact sequence its start states,
+    # aggregates, final state and the states at every backward chunk; its coefficient records are the former's
+    up = lambda n: -(-n // 256) * 256
+    bh, t, st = 24, 1000, 64 * 64 * 4
+    kw = dict(dtype=_lib.DT_F32, bh=bh, seq_len=t, gate_mode=_lib.GATE_TOKEN, has_buffer=1)
+    exact = up(bh * 2 * st) + up(bh * (2 * 64 * 64 + 16) * 4) + up(bh * st) + up(bh * -(-t // 16) * 2 * st)
+    plain, dual = (lib.atlas_mem_saved_bytes(ctypes.byref(_prob(clamp_every=c, **kw))) for c in (0, 32))
+    assert dual == 256 + plain + exact
+
+
 def test_sizes(lib):
     p = _prob()
     st = 64 * 64 * 4
