@@ -232,19 +232,22 @@ def load(path: str | None = None) -> ctypes.CDLL:
 
 
 _NATIVE = None
+_BOUND = None
 
 
 def native():
     """The extension module atlas_rnn_amd._host (csrc/host.cpp): the host path of the operators in native
-    code. Raises LibraryMissing if it is not built; there is no other implementation."""
-    global _NATIVE
-    if _NATIVE is None:
-        load()
+    code, on the library that load() has loaded. Raises LibraryMissing if it is not built; there is no other
+    implementation."""
+    global _NATIVE, _BOUND
+    lib = load()
+    if _BOUND is not lib:
         try:
             from . import _host
         except ImportError as exc:
             raise LibraryMissing(f"atlas_rnn_amd._host is not built ({exc}); run `python -m atlas_rnn_amd.build`") from exc
-        _NATIVE = _host
+        _host.bind(os.path.abspath(lib._name))
+        _NATIVE, _BOUND = _host, lib
     return _NATIVE
 
 

@@ -1,4 +1,4 @@
-"""Ahead-of-time build of libatlas_mem.so for gfx950 (hipcc, no JIT, no torch extension).
+"""Ahead-of-time build of libatlas_mem.so for gfx950 (hipcc, no JIT) and of the extension module _host.so.
 
     python -m atlas_rnn_amd.build          # builds atlas_rnn_amd/libatlas_mem.so in place
 
@@ -59,8 +59,8 @@ def _hipcc() -> str:
 
 
 def _host_cmds(obj: str, out: str) -> tuple[list[str], list[str]]:
-    """The compile and link commands of the extension module: host code only, against torch's headers
-    and libatlas_mem.so beside it."""
+    """The compile and link commands of the extension module: host code only, against torch's headers (it looks
+    libatlas_mem.so's entry points up in the library that the package loads)."""
     import sysconfig
 
     import torch
@@ -72,7 +72,7 @@ def _host_cmds(obj: str, out: str) -> tuple[list[str], list[str]]:
                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
                    "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj]
     link_cmd = [cxx, "-shared", obj, "-o", out, *(f"-L{p}" for p in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch",
-                "-ltorch_python", "-lc10_hip", "-ltorch_hip", f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN"]
+                "-ltorch_python", "-lc10_hip", "-ltorch_hip", "-ldl"]
     return compile_cmd, link_cmd
 
 
@@ -89,7 +89,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 def build(verbose: bool = False) -> str:
     """Compile every HIP source for gfx950, link libatlas_mem.so and build the extension module
-    atlas_rnn_amd._host on it. Always recompiles."""
+    atlas_rnn_amd._host. Always recompiles."""
     hipcc = _hipcc()
     obj_dir = os.path.join(PKG_DIR, "_build")
     os.makedirs(obj_dir, exist_ok=True)

@@ -19,7 +19,12 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
+#include <dlfcn.h>
+
+#include <atomic>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -38,8 +43,51 @@ typedef std::optional<Tensor> OptTensor;
 // ---------------------------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------------------------
+// libatlas_mem.so's entry points, looked up in the library that the Python package has loaded (bind): one
+// library serves both, also where a program has chosen another file than the one beside this module.
+#define ATLAS_LIBRARY(X) \
+  X(atlas_block_merge) X(atlas_block_parts) X(atlas_block_split) X(atlas_heads_bwd) X(atlas_heads_fwd) \
+  X(atlas_linear_batch) X(atlas_linear_wgrad_batch) X(atlas_linear_wgrad_batch_workspace_bytes) X(atlas_mem_bwd) \
+  X(atlas_mem_bwd_workspace_bytes) X(atlas_mem_fwd) X(atlas_mem_infer) X(atlas_mem_saved_bytes) X(atlas_mem_step) \
+  X(atlas_mem_strerror) X(atlas_mem_validate) X(atlas_omega_chain_bwd) X(atlas_omega_chain_fwd_keep) \
+  X(atlas_omega_chain_workspace_bytes) X(atlas_partials_sum) X(atlas_prologue_bwd) X(atlas_prologue_fwd) \
+  X(atlas_prologue_num_workgroups) X(atlas_replicas) X(atlas_tensor_map_bwd_sym) X(atlas_tensor_map_fwd_sym) \
+  X(atlas_tensor_map_symmetrize)
+struct Library {
+#define ATLAS_FIELD(name) decltype(&::name) name;
+  ATLAS_LIBRARY(ATLAS_FIELD)
+#undef ATLAS_FIELD
+  std::string path;
+};
+std::atomic<const Library*> bound{nullptr};
+
+void bind(const std::string& path) {
+  static std::mutex mu;
+  static std::map<std::string, Library> known;   // never dropped: a backward may still be running on one
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = known.find(path);
+  if (it == known.end()) {
+    void* h = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    TORCH_CHECK(h, "cannot load ", path, ": ", dlerror());
+    Library l{};
+#define ATLAS_FIND(name)                                        \
+  l.name = reinterpret_cast<decltype(&::name)>(dlsym(h, #name)); \
+  TORCH_CHECK(l.name, path, " has no " #name);
+    ATLAS_LIBRARY(ATLAS_FIND)
+#undef ATLAS_FIND
+    l.path = path;
+    it = known.emplace(path, std::move(l)).first;
+  }
+  bound.store(&it->second, std::memory_order_release);
+}
+const Library& lib() {
+  const Library* l = bound.load(std::memory_order_acquire);
+  TORCH_CHECK(l, "no library is bound: call through atlas_rnn_amd");
+  return *l;
+}
+
 void check(int status, const char* what) {
-  TORCH_CHECK(status == ATLAS_MEM_OK, what, " failed: ", atlas_mem_strerror(status), " (status ", status, ")");
+  TORCH_CHECK(status == ATLAS_MEM_OK, what, " failed: ", lib().atlas_mem_strerror(status), " (status ", status, ")");
 }
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -122,16 +170,16 @@ struct RecurrenceFn : public Function<RecurrenceFn> {
     // outputs a loss does not use get no gradient tensor (a missing one counts as zero)
     ctx->set_materialize_grads(false);
     const RecOut o = rec_outputs(prob, k);
-    const Tensor saved = scratch(k, (int64_t)atlas_mem_saved_bytes(&prob));
+    const Tensor saved = scratch(k, (int64_t)lib().atlas_mem_saved_bytes(&prob));
     const atlas_mem_fwd_args a = fwd_args(k, q, v, lr, decay, get(beta), get(gate), S_ref, S0, get(Z0), get(buf), o);
     if (infer) {   // no input asks for a gradient: nothing for a backward is formed or kept
-      check(atlas_mem_infer(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
+      check(lib().atlas_mem_infer(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
       variable_list out{o.y, o.S_T};
       if (o.Z_T.defined()) out.push_back(o.Z_T);
       if (o.buf.defined()) out.push_back(o.buf);
       return out;
     }
-    check(atlas_mem_fwd(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
+    check(lib().atlas_mem_fwd(&prob, &a, mfptr(saved), stream_of(k)), "atlas_mem_fwd");
     ctx->save_for_backward({k, q, v, lr, decay, get(beta), get(gate), S_ref, S0, get(Z0), get(buf), saved});
     ctx->saved_data["prob"] = std::string(reinterpret_cast<const char*>(&prob), sizeof(prob));
     variable_list out{o.y, o.S_T};
@@ -155,7 +203,7 @@ struct RecurrenceFn : public Function<RecurrenceFn> {
     const Tensor dk = like(k), dq = like(q), dv = like(v), dlr = like(lr), dd = like(decay), db = like(beta),
                  dg = like(gate), dbuf = like(buf);
     const Tensor dS_ref = like(S_ref), dS0 = like(S0), dZ0 = prob.momentum ? like(S0) : Tensor();
-    const size_t ws_bytes = atlas_mem_bwd_workspace_bytes(&prob);
+    const size_t ws_bytes = lib().atlas_mem_bwd_workspace_bytes(&prob);
     const Tensor ws = scratch(k, (int64_t)ws_bytes);
     atlas_mem_bwd_args a{};
     a.k = ptr(k); a.q = ptr(q); a.v = ptr(v); a.lr = ptr(lr); a.decay = ptr(decay); a.beta = ptr(beta);
@@ -163,7 +211,7 @@ struct RecurrenceFn : public Function<RecurrenceFn> {
     a.dy = ptr(dy); a.dS_T = fptr(dS_T); a.dZ_T = fptr(dZ_T); a.dbuffer_out = fptr(dbuf_out);
     a.dk = mptr(dk); a.dq = mptr(dq); a.dv = mptr(dv); a.dlr = mptr(dlr); a.ddecay = mptr(dd); a.dbeta = mptr(db);
     a.dgate = mptr(dg); a.dS_ref = mfptr(dS_ref); a.dS0 = mfptr(dS0); a.dZ0 = mfptr(dZ0); a.dbuffer_in = mfptr(dbuf);
-    check(atlas_mem_bwd(&prob, &a, fptr(saved), mptr(ws), ws_bytes, stream_of(k)), "atlas_mem_bwd");
+    check(lib().atlas_mem_bwd(&prob, &a, fptr(saved), mptr(ws), ws_bytes, stream_of(k)), "atlas_mem_bwd");
     return {dk, dq, dv, dlr, dd, db, dg, dS_ref, dS0, Z0.defined() ? dZ0 : Tensor(), dbuf, Tensor(), Tensor()};
   }
 };
@@ -213,7 +261,7 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
   p.clamp_every = (int)clamp_every.value_or(0);
   p.clamp_final = clamp_final;
   p.dtype = dt == at::kBFloat16 ? ATLAS_DT_BF16 : ATLAS_DT_F32;
-  if (atlas_mem_validate(&p) != ATLAS_MEM_OK) return std::nullopt;
+  if (lib().atlas_mem_validate(&p) != ATLAS_MEM_OK) return std::nullopt;
   c10::DeviceGuard guard(k.device());
   const Tensor kc = canon(k, dt), qc = canon(q, dt), vc = canon(v, dt), lc = canon(lr, dt), dc = canon(decay, dt),
                bc = canon(beta, dt), gc = canon(gate, dt);
@@ -233,7 +281,7 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
     if (!tangent) {   // decode: one launch, no saved buffer (rnn_transformer.py:863-900 through the cell at T = 1)
       o = rec_outputs(p, kc);
       const atlas_mem_fwd_args a = fwd_args(kc, qc, vc, lc, dc, bc, gc, Src, S0c, Zc, Bc, o);
-      check(atlas_mem_step(&p, &a, stream_of(kc)), "atlas_mem_step");
+      check(lib().atlas_mem_step(&p, &a, stream_of(kc)), "atlas_mem_step");
       return o;
     }
   }
@@ -266,7 +314,7 @@ std::tuple<Tensor, Tensor> symmetrized(const Tensor& proj, int64_t d, at::Scalar
   const Tensor p = aligned(proj.detach().to(dt));
   const int64_t m = p.size(1);
   const Tensor ps = like(p), pst = plain(p, {m, p.size(0)});
-  check(atlas_tensor_map_symmetrize(dt_code(p), (int)d, (int)m, ptr(p), mptr(ps), mptr(pst), stream_of(p)),
+  check(lib().atlas_tensor_map_symmetrize(dt_code(p), (int)d, (int)m, ptr(p), mptr(ps), mptr(pst), stream_of(p)),
         "atlas_tensor_map_symmetrize");
   return {ps, pst};
 }
@@ -276,7 +324,7 @@ struct TensorMapFn : public Function<TensorMapFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& ps, const Tensor& pst, int64_t degree) {
     const int64_t n = x.size(0), d = x.size(1), m = ps.size(1);
     const Tensor out = plain(x, {n, m}), pre = degree > 1 ? plain(x, {n, m}) : Tensor();
-    check(atlas_tensor_map_fwd_sym(dt_code(x), n, (int)d, (int)m, (int)degree, ptr(x), ptr(pst), mptr(out), mptr(pre),
+    check(lib().atlas_tensor_map_fwd_sym(dt_code(x), n, (int)d, (int)m, (int)degree, ptr(x), ptr(pst), mptr(out), mptr(pre),
                                    stream_of(x)), "atlas_tensor_map_fwd_sym");
     ctx->save_for_backward({x, ps, pre});
     ctx->saved_data["degree"] = degree;
@@ -288,7 +336,7 @@ struct TensorMapFn : public Function<TensorMapFn> {
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
     c10::DeviceGuard guard(x.device());
     const Tensor dout = canon(g[0], x.scalar_type()), dx = like(x);
-    check(atlas_tensor_map_bwd_sym(dt_code(x), x.size(0), (int)x.size(1), (int)ps.size(1),
+    check(lib().atlas_tensor_map_bwd_sym(dt_code(x), x.size(0), (int)x.size(1), (int)ps.size(1),
                                    (int)ctx->saved_data["degree"].toInt(), ptr(x), ptr(ps), ptr(pre), ptr(dout), mptr(dx),
                                    stream_of(x)), "atlas_tensor_map_bwd_sym");
     return {dx, Tensor(), Tensor(), Tensor()};
@@ -340,7 +388,7 @@ variable_list replicas(int op, int64_t nrep, at::TensorList in) {
         dst[cnt++] = mptr(outs[i]);
       }
       if (cnt > 0 && (cnt == 4 || i == xs.size())) {
-        check(atlas_replicas(op == kReplicate ? ATLAS_REPLICATE : ATLAS_REPLICA_SUM,
+        check(lib().atlas_replicas(op == kReplicate ? ATLAS_REPLICATE : ATLAS_REPLICA_SUM,
                              dt == at::kBFloat16 ? ATLAS_DT_BF16 : ATLAS_DT_F32, cnt, (int)nrep, n, src, dst,
                              stream_of(xs[0])), "atlas_replicas");
         cnt = 0;
@@ -379,7 +427,7 @@ struct BlockSplitFn : public Function<BlockSplitFn> {
     const int64_t bh = phi.size(0), T = phi.size(1), dk = phi.size(2), dv = v.size(2);
     const int64_t nb = (dk / kBlock) * (dv / kBlock);
     const Tensor a = plain(phi, {nb * bh, T, kBlock}), b = like(a), c = like(a);
-    check(atlas_block_split(dt_code(phi), (int)bh, (int)T, (int)dk, (int)dv, ptr(phi), ptr(psi), ptr(v), fptr(S_ref),
+    check(lib().atlas_block_split(dt_code(phi), (int)bh, (int)T, (int)dk, (int)dv, ptr(phi), ptr(psi), ptr(v), fptr(S_ref),
                             mptr(a), mptr(b), mptr(c), stream_of(phi)), "atlas_block_split");
     ctx->save_for_backward({phi, S_ref});
     ctx->saved_data["dv"] = dv;
@@ -395,8 +443,8 @@ struct BlockSplitFn : public Function<BlockSplitFn> {
       d[i] = g[i].defined() ? canon(g[i], phi.scalar_type())
                             : at::zeros({(dk / kBlock) * (dv / kBlock) * bh, T, kBlock}, phi.options());
     const Tensor dphi = like(phi), dpsi = like(phi), dvv = plain(phi, {bh, T, dv});
-    const Tensor parts = f32(phi, {bh, atlas_block_parts((int)T), dv, dk});
-    check(atlas_block_merge(dt_code(phi), (int)bh, (int)T, (int)dk, (int)dv, ptr(phi), fptr(S_ref), ptr(d[0]), ptr(d[1]),
+    const Tensor parts = f32(phi, {bh, lib().atlas_block_parts((int)T), dv, dk});
+    check(lib().atlas_block_merge(dt_code(phi), (int)bh, (int)T, (int)dk, (int)dv, ptr(phi), fptr(S_ref), ptr(d[0]), ptr(d[1]),
                             ptr(d[2]), mptr(dphi), mptr(dpsi), mptr(dvv), mfptr(parts), stream_of(phi)),
           "atlas_block_merge");
     return {dphi, dpsi, dvv, parts.sum(1)};
@@ -454,7 +502,7 @@ variable_list products(int layout, const variable_list& acts, const variable_lis
     wp[i] = ptr(w[i]);
     op[i] = mptr(outs[i]);
   }
-  check(atlas_linear_batch(layout, (int)acts.size(), m, ns, ks, ap, wp, op, stream_of(a[0])), "atlas_linear_batch");
+  check(lib().atlas_linear_batch(layout, (int)acts.size(), m, ns, ks, ap, wp, op, stream_of(a[0])), "atlas_linear_batch");
   return outs;
 }
 
@@ -492,9 +540,9 @@ variable_list wgrads(const variable_list& dys_in, const variable_list& xs_in, at
       xp[i] = ptr(xs[i]);
       wp[i] = mptr(out[i]);
     }
-    const int64_t bytes = atlas_linear_wgrad_batch_workspace_bytes(cnt, n, os, is);
+    const int64_t bytes = lib().atlas_linear_wgrad_batch_workspace_bytes(cnt, n, os, is);
     const Tensor ws = scratch(dys[0], bytes);
-    check(atlas_linear_wgrad_batch(dt == at::kBFloat16 ? ATLAS_DT_BF16 : ATLAS_DT_F32, cnt, n, os, is, dp, xp, wp, mptr(ws),
+    check(lib().atlas_linear_wgrad_batch(dt == at::kBFloat16 ? ATLAS_DT_BF16 : ATLAS_DT_F32, cnt, n, os, is, dp, xp, wp, mptr(ws),
                                    bytes, stream_of(dys[0])), "atlas_linear_wgrad_batch");
     return out;
   }
@@ -554,7 +602,7 @@ variable_list sum_partials(const std::vector<Partial>& items) {
     src[i] = ptr(keep[i]);
     dst[i] = mptr(outs[i]);
   }
-  check(atlas_partials_sum((int)items.size(), (int)keep[0].size(0), cols, src, dst, dts, stream_of(keep[0])),
+  check(lib().atlas_partials_sum((int)items.size(), (int)keep[0].size(0), cols, src, dst, dts, stream_of(keep[0])),
         "atlas_partials_sum");
   return outs;
 }
@@ -588,7 +636,7 @@ struct CellPrologueFn : public Function<CellPrologueFn> {
       const OptTensor* w[3] = {&wq, &wk, &wv};
       for (int i = 0; i < 3; ++i) taps[i] = aligned((*w[i])->reshape({dim, K}));
     }
-    check(atlas_prologue_fwd(dt, (int)B, (int)T, (int)dim, (int)K, (float)dims.eps, ptr(x), ptr(norm_w), ptr(taps[0]),
+    check(lib().atlas_prologue_fwd(dt, (int)B, (int)T, (int)dim, (int)K, (float)dims.eps, ptr(x), ptr(norm_w), ptr(taps[0]),
                              ptr(taps[1]), ptr(taps[2]), mptr(xn), mptr(qi), mptr(ki), mptr(vi), mptr(inv), st),
           "atlas_prologue_fwd");
     if (!conv) qi = ki = vi = xn;
@@ -615,7 +663,7 @@ struct CellPrologueFn : public Function<CellPrologueFn> {
     const Tensor kg = kg_in.has_value() ? aligned(kg_in->reshape({H, d})) : Tensor();
     const Tensor q = plain(x, {B * H, T, d}), k = like(q), v = like(q);
     const Tensor gates = nG ? plain(x, {nG, B * H, T}) : Tensor();
-    check(atlas_heads_fwd(dt, (int)B, (int)T, (int)H, (int)d, (int)nG, ptr(p[0]), ptr(p[1]), ptr(p[2]),
+    check(lib().atlas_heads_fwd(dt, (int)B, (int)T, (int)H, (int)d, (int)nG, ptr(p[0]), ptr(p[1]), ptr(p[2]),
                           nG ? ptr(p[3]).p : nullptr, ptr(qg), ptr(kg), ptr(bg), mptr(q), mptr(k), mptr(v), mptr(gates), st),
           "atlas_heads_fwd");
     ctx->save_for_backward({x, norm_w, taps[0], taps[1], taps[2], inv, qi, ki, vi, xn, Wq, Wk, Wv, Wg, p[0], p[1], qg, kg,
@@ -660,12 +708,12 @@ struct CellPrologueFn : public Function<CellPrologueFn> {
       for (int64_t i = 0; i < nG; ++i) parts.push_back(or_zero(g[4 + i], {B * H, T}));
       dg = at::stack(parts);
     }
-    const int64_t nwg = atlas_prologue_num_workgroups((int)B, (int)T);
+    const int64_t nwg = lib().atlas_prologue_num_workgroups((int)B, (int)T);
     const Tensor dql = like(ql), dkl = like(kl), dvl = like(ql);
     const Tensor dzl = nG ? plain(x, {B, T, nG * H}) : Tensor();
     const Tensor dqg = norm ? f32(x, {nwg, H, d}) : Tensor(), dkg = norm ? f32(x, {nwg, H, d}) : Tensor();
     const Tensor dbias = nG ? f32(x, {nwg, nG * H}) : Tensor();
-    check(atlas_heads_bwd(dt, (int)B, (int)T, (int)H, (int)d, (int)nG, ptr(ql), ptr(kl), ptr(qg), ptr(kg), ptr(gates),
+    check(lib().atlas_heads_bwd(dt, (int)B, (int)T, (int)H, (int)d, (int)nG, ptr(ql), ptr(kl), ptr(qg), ptr(kg), ptr(gates),
                           ptr(dq), ptr(dk), ptr(dv), ptr(dg), mptr(dql), mptr(dkl), mptr(dvl), mptr(dzl), mptr(dqg),
                           mptr(dkg), mptr(dbias), st), "atlas_heads_bwd");
     // ---- projections
@@ -689,7 +737,7 @@ struct CellPrologueFn : public Function<CellPrologueFn> {
     }
     const Tensor dxn = or_zero(dsum, x.sizes());
     const Tensor dx = like(x), dnw = f32(x, {nwg, dim}), dcv = conv ? f32(x, {nwg, 3, dim, K}) : Tensor();
-    check(atlas_prologue_bwd(dt, (int)B, (int)T, (int)dim, (int)K, ptr(x), ptr(norm_w), ptr(tq), ptr(tk), ptr(tv), ptr(inv),
+    check(lib().atlas_prologue_bwd(dt, (int)B, (int)T, (int)dim, (int)K, ptr(x), ptr(norm_w), ptr(tq), ptr(tk), ptr(tv), ptr(inv),
                              ptr(dxn), ptr(dci[0]), ptr(dci[1]), ptr(dci[2]), mptr(dx), mptr(dnw), mptr(dcv), st),
           "atlas_prologue_bwd");
     // ---- every parameter gradient of the two kernels from their partials, in one launch
@@ -808,7 +856,7 @@ struct OmegaChainFn : public Function<OmegaChainFn> {
     // the backward has its own copies of the updates and the decays, so that the caller may edit the returned
     // and the given ones in place before it (a second write of the updates: 91.4 -> 93.6 us forward and backward at 16 x 64 x 8192 fp32)
     const Tensor kept = grad ? like(update) : Tensor(), kept_decay = grad ? like(decay) : Tensor();
-    check(atlas_omega_chain_fwd_keep(dt_code(s), BH, n, p, (int)O, (int)window, ptr(s), ptr(decay), ptr(last), ptr(am),
+    check(lib().atlas_omega_chain_fwd_keep(dt_code(s), BH, n, p, (int)O, (int)window, ptr(s), ptr(decay), ptr(last), ptr(am),
                                      ptr(lm), ptr(gate), ptr(buf), mptr(update), mptr(moms), mptr(next_lm), mptr(next_buf),
                                      mptr(kept), mptr(kept_decay), stream_of(s)),
           "atlas_omega_chain_fwd");
@@ -836,9 +884,9 @@ struct OmegaChainFn : public Function<OmegaChainFn> {
                  dlast = plain(update, {BH, p});
     const Tensor dg = ctx->saved_data["dgate"].toBool() ? like(gate) : Tensor();
     const Tensor dbuf = ctx->saved_data["has_buf"].toBool() ? plain(update, {BH, e - 1, p}) : Tensor();
-    const int64_t bytes = atlas_omega_chain_workspace_bytes(BH, n, p, (int)O);
+    const int64_t bytes = lib().atlas_omega_chain_workspace_bytes(BH, n, p, (int)O);
     const Tensor ws = scratch(update, bytes);
-    check(atlas_omega_chain_bwd(dt_code(update), BH, n, p, (int)O, (int)e, ptr(s), ptr(decay), ptr(am), ptr(lm), ptr(gate),
+    check(lib().atlas_omega_chain_bwd(dt_code(update), BH, n, p, (int)O, (int)e, ptr(s), ptr(decay), ptr(am), ptr(lm), ptr(gate),
                                 ptr(update), ptr(moms), ptr(dup), ptr(dlm), ptr(dbo), mptr(ds), mptr(dd), mptr(dlast),
                                 mptr(dam), mptr(dlm0), mptr(dg), mptr(dbuf), mptr(ws), bytes, stream_of(update)),
           "atlas_omega_chain_bwd");
@@ -899,6 +947,8 @@ auto entry(R (*f)(A...)) {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("bind", &bind);
+  m.def("library", [] { return lib().path; });
   m.def("recurrence", entry(&recurrence));
   m.def("tensor_map", entry(&tensor_map));
   m.def("symmetrized", entry(&symmetrized));
