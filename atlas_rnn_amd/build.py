@@ -89,7 +89,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 def build(verbose: bool = False) -> str:
     """Compile every HIP source for gfx950, link libatlas_mem.so and build the extension module
-    atlas_rnn_amd._host. Always recompiles."""
+    atlas_rnn_amd._host. Always recompiles; the two built before stay where a step fails."""
     hipcc = _hipcc()
     obj_dir = os.path.join(PKG_DIR, "_build")
     os.makedirs(obj_dir, exist_ok=True)
@@ -106,8 +106,8 @@ def build(verbose: bool = False) -> str:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs], verbose)
-    os.replace(tmp, LIB_PATH)
     _run(host_link, verbose)
+    os.replace(tmp, LIB_PATH)
     os.replace(host_tmp, HOST_PATH)
     return LIB_PATH
 

@@ -647,20 +647,20 @@ def check_cuda_availability():
     if not torch.cuda.is_available():
         return False, "no ROCm GPU visible"
     try:
-        _lib.load()
+        _lib.native()
     except Exception as exc:  # noqa: BLE001
-        return False, f"libatlas_mem.so not loaded: {exc}"
+        return False, f"libatlas_mem.so or the extension module on it not loaded: {exc}"
     props = torch.cuda.get_device_properties(0)
     return True, f"atlas_rnn_amd ready (GPU: {props.name}, library: {_lib.LIB_PATH})"
 
 
 def get_cuda_status() -> dict:
     """atlas_pytorch/cuda/atlas_omega_autograd.py:16-22: the backend's load status for logging, with
-    the reference's keys. `available`: libatlas_mem.so is loaded (its ABI version checked);
-    `loaded_via`: the library's path, or "none"; `error`: why it could not be loaded ("" when
-    available). Touches no GPU (it loads the library only)."""
+    the reference's keys. `available`: libatlas_mem.so (its ABI version checked) and the extension module
+    on it are loaded; `loaded_via`: the library's path, or "none"; `error`: why one could not be loaded (""
+    when available). Touches no GPU (it loads the two only)."""
     try:
-        _lib.load()
+        _lib.native()
     except Exception as exc:  # noqa: BLE001
         return {"available": False, "loaded_via": "none", "error": str(exc)}
     return {"available": True, "loaded_via": _lib.LIB_PATH, "error": ""}
