@@ -270,8 +270,8 @@ class _CellBase(Module):
             k, q, v, lr, decay, beta, gate, S_ref=S0, S0=S0, Z0=Z0, buffer=buf, window=window,
             map_mode='elementwise' if self.phi.fused_elementwise else 'off', map_degree=self.phi.degree,
             clamp_every=chunk, clamp_final=True)
-        y = y.to(x.dtype).reshape(batch, self.heads, seq_len, -1).transpose(1, 2).reshape(batch, seq_len, -1)
-        out = linear(y, self.to_out.weight)   # to_out on the library's bf16 products
+        y = y.to(x.dtype).reshape(batch, self.heads, seq_len, -1)
+        out = linear(self.merge_heads(y), self.to_out.weight)   # to_out on the library's bf16 products
         dt = x.dtype if fresh else S0.dtype   # init_state's dtype for a fresh state
         next_state = RNNMemState(
             seq_index=(0 if fresh else state.seq_index) + seq_len,

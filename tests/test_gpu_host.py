@@ -144,3 +144,14 @@ def test_recurrence_function_on_canonical_operands(clamp):
     with pytest.raises(RuntimeError, match="status"):   # a buffer without a window
         F.MemoryRecurrenceFn.apply(*[x[n] for n in names[:5]], None, None, x["S_ref"], x["S0"], None, x["buffer"],
                                    F.RecurrenceConfig(window=1))
+
+
+def test_the_cell_runs_its_merge_heads_module():
+    cell = am.OmegaRNNMemoryCell(dim=32, dim_head=32, heads=2, omega_window=2).cuda()
+    seen = []
+    cell.merge_heads.register_forward_hook(lambda m, args, out: seen.append((args[0].shape, out.shape)) or 2 * out)
+    x = torch.randn(3, 5, 32, device="cuda")
+    doubled = cell(x)[0]
+    assert seen == [((3, 2, 5, 32), (3, 5, 64))]
+    cell.merge_heads._forward_hooks.clear()
+    assert torch.allclose(doubled, 2 * cell(x)[0])
