@@ -12,7 +12,7 @@
 // accumulator. With hipcc 7.2 on gfx950 such a join after a conditionally issued
 // v_mfma_f32_16x16x4_f32 got too few wait states before v_accvgpr_read, returning the value
 // from before the last MFMA. Optional terms are therefore computed unconditionally with zero
-// operands (frag_ld_or_zero) instead of being skipped.
+// operands instead of being skipped.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -104,20 +104,6 @@ __device__ __forceinline__ typename MM<OT>::frag frag_ld(const ST* p, int rs, in
   return f;
 }
 
-// frag_ld, or a zero fragment when p is null (keeps the MFMA itself unconditional).
-template <typename OT, typename ST>
-__device__ __forceinline__ typename MM<OT>::frag frag_ld_or_zero(const ST* p, int rs, int cs, int r0, int k0) {
-  if (p) return frag_ld<OT>(p, rs, cs, r0, k0);
-  typename MM<OT>::frag f;
-  if constexpr (MM<OT>::KL == 1) {
-    f = static_cast<OT>(0.f);
-  } else {
-#pragma unroll
-    for (int e = 0; e < MM<OT>::KL; ++e) f[e] = static_cast<OT>(0.f);
-  }
-  return f;
-}
-
 // Row-major, k contiguous, same element type: one 16-byte load per lane for bf16.
 // Requires rs % 8 == 0 and 16-byte aligned p.
 template <typename OT>
@@ -170,21 +156,6 @@ __device__ __forceinline__ typename MM<OT>::frag frag_ld_tr(const OT* p, int ld,
     const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(typename MM<OT>::frag, v);
   }
-}
-
-// frag_ld_tr with each k value multiplied by s[k] (fp32) before rounding to OT.
-template <typename OT>
-__device__ __forceinline__ typename MM<OT>::frag frag_ld_tr_kscaled(const OT* p, int ld, int r0, int k0,
-                                                                   const float* s) {
-  typename MM<OT>::frag f = frag_ld_tr<OT>(p, ld, r0, k0);
-  const int kb = k0 + (lane_id() >> 4) * MM<OT>::KL;
-  if constexpr (MM<OT>::KL == 1) {
-    f = static_cast<OT>(to_f32(f) * s[kb]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < MM<OT>::KL; ++e) f[e] = static_cast<OT>(to_f32(f[e]) * s[kb + e]);
-  }
-  return f;
 }
 
 // Fragment f with its k values scaled by w[k] (w: the KL weights of this lane's k slots).

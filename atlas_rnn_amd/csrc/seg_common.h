@@ -79,12 +79,6 @@ struct SrcRows {
   static_assert(SP % 16 == 0 && HP <= kHaloPad, "whole tiles of sources");
 };
 
-// Window weight of the source t - j for target t: the token gate of the source, the lag gate
-// w[t][j], or 1.
-__device__ __forceinline__ float src_w(int gate_mode, float ug, const float* wl, int e, int t, int j) {
-  return gate_mode == GATE_TOKEN ? ug : (gate_mode == GATE_LAG ? wl[t * e + j] : 1.f);
-}
-
 // Eight consecutive elements: one 16-byte (bf16) or two 16-byte (fp32) vector accesses.
 template <typename T>
 struct Vec8 {
@@ -178,13 +172,10 @@ __device__ __forceinline__ Vec8<T> vec8_load(const T* p) {
   return r;
 }
 
-// Per-chunk scalars and coefficients in LDS.
+// A chunk's coefficients in LDS.
 template <int CH>
 struct ChunkScalars {
   static constexpr int SPM = CH + kHaloPad;
-  float alpha[CH], eta[CH], beta[CH];   // padded targets: alpha = beta = 1, eta = 0
-  float ug[SPM];                        // token-mode gate of each source
-  float wl[CH * kMaxWindow];            // lag-mode weights [tau][j]
   // the coefficient record (same order as CoefRec, one contiguous 16-byte aligned block)
   alignas(16) float acoef[CH];          // a_{tau-1}
   float kcoef[CH];                      // kappa_{tau-1}
@@ -196,7 +187,7 @@ struct ChunkScalars {
 
 // Per-chunk coefficient record in HBM (fp32), written by k_chunk_coef for every chunk of every row:
 // acoef[CH], kcoef[CH], endc[4], wsend[SPM], wzend[SPM], wsmid[SPM], wzmid[SPM], midc[4] - the
-// layout of ChunkScalars from acoef on.
+// layout of ChunkScalars.
 template <int CH>
 struct CoefRec {
   static constexpr int SPM = CH + kHaloPad;
@@ -204,59 +195,9 @@ struct CoefRec {
   static_assert(SIZE % 4 == 0, "record copied as float4");
 };
 
-// Decay tables of one chunk, stored [c][t] with source column c = t' + 1 (column 0 is the chunk
-// start, t' = -1) and target row t:
-//   A[c][t] = prod_{u = t'+1 .. t} alpha_u,   B[c][t] = prod_{u = t'+1 .. t} beta_u,
-//   C[c][t] = response of Ws at t to a unit input into Wz at t':
-//             C[c][t'] = eta_t',  C[c][t] = alpha_t C[c][t-1] + eta_t B[c][t]   (t > t'),
-// and zero for t < t'. Column 0 holds the chunk-start coefficients a_t, b_t, kappa_t. Every linear
-// recurrence along the chunk (Wz / Ws of a source, and the adjoint recurrences of the scalar
-// gradients) is a sum over these columns, so it runs in parallel instead of step by step.
-// The pitch CH + 1 keeps row-wise and column-wise accesses free of bank conflicts.
-template <int CH>
-struct DecayTab {
-  float A[CH + 1][CH + 1], B[CH + 1][CH + 1], C[CH + 1][CH + 1];
-};
-
 // Lane t's value of x, in every lane (v_readlane; t is a wave-uniform constant).
 __device__ __forceinline__ float lane_bcast(float x, int t) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), t));
-}
-
-// Decay tables of a chunk, computed by one wave with one column per lane (lane c = 0..CH;
-// lanes above CH run the same chain and write nothing). Column c (tp = c - 1), for t >= tp:
-//   A[c][t] = prod_{r=c..t} alpha_r,  B[c][t] = prod_{r=c..t} beta_r,
-//   C[c][t] = alpha_t C[c][t-1] + eta_t B[c][t]   (C[c][tp] = eta_tp),
-// zero for t < tp. Lane 0 also writes B1[t] = b_{t-1} (t = 0..CH, B1[0] = 1). The step scalars
-// are read once into lane t's registers and broadcast with v_readlane, so the chains never wait
-// on LDS reads (the table writes are not waited on).
-template <int CH>
-__device__ __forceinline__ void decay_columns_wave(DecayTab<CH>& tab, const ChunkScalars<CH>& sc, float* B1) {
-  static_assert(CH < kWave, "one lane per column");
-  const int c = lane_id(), tp = c - 1;
-  const bool writer = c <= CH;
-  const int ts = c < CH ? c : 0;
-  const float al_v = sc.alpha[ts], et_v = sc.eta[ts], be_v = sc.beta[ts];
-  float a = 1.f, b = 1.f, m = 0.f;
-  if (c == 0) B1[0] = 1.f;
-#pragma unroll
-  for (int t = 0; t < CH; ++t) {
-    const float al = lane_bcast(al_v, t), et = lane_bcast(et_v, t), be = lane_bcast(be_v, t);
-    if (t == tp) {
-      m = et;
-    } else if (t > tp) {
-      b = be * b;
-      a = al * a;
-      m = al * m + et * b;
-    }
-    const bool on = t >= tp;
-    if (writer) {
-      tab.A[c][t] = on ? a : 0.f;
-      tab.B[c][t] = on ? b : 0.f;
-      tab.C[c][t] = on ? m : 0.f;
-    }
-    if (c == 0) B1[t + 1] = b;
-  }
 }
 
 }  // namespace atlas

@@ -627,8 +627,6 @@ __global__ __launch_bounds__(kSegThreads) void k_walk_bwd(const Geom g, const Bw
     for (int r = 0; r < 4; ++r) dst[(size_t)(32 * qw + 16 * u + 4 * gq + r) * D + 16 * kt + m] = dsr[u][r];
 }
 
-size_t walk_bwd_smem_bytes() { return sizeof(wb::Smem); }
-
 template <bool MAPE, int HC, bool BUF = false>
 hipError_t launch_walk_bwd_h(const Geom& g, const BwdPtrs<bf16>& a, const SegGeom& sg, const BwdSegPtrs& p,
                              hipStream_t stream) {

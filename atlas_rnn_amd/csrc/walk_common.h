@@ -43,9 +43,6 @@ __device__ __forceinline__ u32x4v bld16(rsrc_t r, uint32_t off) {
 __device__ __forceinline__ u32x2v bld8(rsrc_t r, uint32_t off) {
   return __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
 }
-__device__ __forceinline__ unsigned short bld2(rsrc_t r, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0);
-}
 __device__ __forceinline__ void bst8(rsrc_t r, uint32_t off, u32x2v v) {
   __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)off, 0, 0);
 }
