@@ -1,5 +1,5 @@
-// affine.hip - right-affine scan H_t = H_{t-1} A_t + B_t (atlas_pytorch/affine_scan.py:36-158),
-// chunked on the fp32 matrix cores (v_mfma_f32_16x16x4_f32).
+// affine.hip - right-affine scan H_t = H_{t-1} A_t + B_t (atlas_pytorch/affine_scan.py:36-158) on the fp32
+// matrix cores (v_mfma_f32_16x16x4_f32), in one pass over the steps or in chunks.
 //
 // A: [N][T][D][D], B: [N][T][R][D], prev = H_0: [N][R][D] (zero when absent); out = H_1 .. H_T as
 // [N][T][R][D]; fp32, D, R <= 64 (zero-padded to 64 x 64 operands inside LDS).
@@ -115,6 +115,7 @@ __device__ __forceinline__ void acc_store(const f32x4 (&acc)[4], float* out, int
 
 // ---- the scan kernel ----
 constexpr int kDepth = 4;
+constexpr int kAny = 0, kTiny = -1;   // D that the kernel is not built for
 constexpr int threads(int d) { return d == 48 ? 192 : 256; }   // of a scan workgroup
 
 struct ScanArgs {
@@ -144,16 +145,20 @@ __device__ __forceinline__ void bst4(rsrc_t r, uint32_t off, uint32_t v) {
 using aff::Geo;
 
 // One unit = the steps of one chunk of one n; KD waves = 16 rows of its state, each wave 16 columns.
-// DC: D, or 0 for any D up to 64 that is not a multiple of 16 (element loads).
+// DC: D, or kAny / kTiny for a D of 4 .. 63 / 1 .. 3 that is not a multiple of 16. The rows of a kAny matrix are not
+// aligned to the lanes' groups of four: the group that crosses the end of a row is loaded as the row's last four
+// elements and shifted where it is used, so that a group is one 16-byte load as elsewhere. Element by element it
+// was four times the loads (16 x 512 steps of 64 x 63, forward and backward: 1140 -> 620 us, three passes of 64-step
+// chunks 932); a shift where it is loaded waits for every load (1520).
 template <bool REV, int DC>
 __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs a) {
   using namespace aff;
-  constexpr int KD = DC ? DC / 16 : 4;
+  constexpr int KD = DC > 0 ? DC / 16 : 4;
   constexpr int TH = threads(DC);
   constexpr int RB = TH / (64 * KD);                  // row blocks of a workgroup
   constexpr int NG = 64 * KD * KD;                    // 4-element groups of a matrix
   constexpr int NU = (NG + TH - 1) / TH;              // of them a thread's
-  constexpr int DEPTH = DC ? kDepth : 2;   // steps whose operands are in flight in registers (4, 6 and 8 take the same time)
+  constexpr int DEPTH = DC != kTiny ? kDepth : 2;   // steps whose operands are in flight in registers (4, 6 and 8 take the same time)
   constexpr int SP = REV ? 64 : 68;
   static_assert(DEPTH % 2 == 0, "the LDS buffers alternate");
   __shared__ __align__(16) float S[2][16 * KD][SP];
@@ -163,7 +168,7 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
   if (unit >= a.units) return;
   const int l = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id()), tl = l & 15, kq = l >> 4;
   const int rb = w / KD, cw = w % KD;
-  const int D = DC ? DC : g.D, R = g.R;
+  const int D = DC > 0 ? DC : g.D, R = g.R;
   const size_t cs = (size_t)R * D, ds = (size_t)D * D;
 
   // the unit's steps and operands
@@ -237,9 +242,12 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
     return b;
   };
   auto at = [&](const Blk& b, uint32_t st, int u) { return REV ? b.o - (uint32_t)u * st : b.o + (uint32_t)u * st; };
+  const int rem = D & 3;   // kAny: elements of the crossing group
   auto ld4 = [&](rsrc_t r, uint32_t off, int col) {
-    if constexpr (DC != 0) {
+    if constexpr (DC > 0) {
       return __builtin_bit_cast(f32x4, bld16(r, off));
+    } else if constexpr (DC == kAny) {
+      return __builtin_bit_cast(f32x4, bld16(r, col < D && col + 4 > D ? off - 4u * (uint32_t)(4 - rem) : off));
     } else {
       f32x4 v;
 #pragma unroll
@@ -247,9 +255,24 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
       return v;
     }
   };
+  // what ld4 loaded, in place: where it is used, so that the loads stay in flight
+  auto placed = [&](f32x4 v, int col) {
+    if constexpr (DC == kAny) {   // (rem is the same in every lane)
+      if (col < D && col + 4 > D) {
+        const float a = rem == 3 ? v[1] : rem == 2 ? v[2] : v[3], b = rem == 3 ? v[2] : v[3];
+        v = f32x4{a, rem > 1 ? b : 0.f, rem == 3 ? v[3] : 0.f, 0.f};
+      }
+    }
+    return v;
+  };
   auto st4 = [&](f32x4 v, rsrc_t r, uint32_t off, int col) {
-    if constexpr (DC != 0) {
+    if constexpr (DC > 0) {
       bst16(r, off, __builtin_bit_cast(u32x4v, v));
+    } else if constexpr (DC == kAny) {
+      const bool cross = col < D && col + 4 > D;
+      bst16(r, cross ? kOob : off, __builtin_bit_cast(u32x4v, v));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) bst4(r, cross && i < rem ? off + 4u * i : kOob, __builtin_bit_cast(uint32_t, (float)v[i]));
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) bst4(r, col + i < D ? off + 4u * i : kOob, __builtin_bit_cast(uint32_t, (float)v[i]));
@@ -263,7 +286,7 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
   auto load_c = [&](int u, const Blk& b) { cv[u] = ld4(b.r, xo + at(b, cb, u), xc); };
   auto stage = [&](int u, int v, int b) {   // slot u's matrix into LDS buffer b
     const int i = threadIdx.x + TH * v, r = i / (4 * KD), q = i % (4 * KD);
-    if (NG % TH == 0 || i < NG) *reinterpret_cast<f32x4*>(&S[b][r][4 * (REV ? q ^ (r & 15) : q)]) = ps[u][v];
+    if (NG % TH == 0 || i < NG) *reinterpret_cast<f32x4*>(&S[b][r][4 * (REV ? q ^ (r & 15) : q)]) = placed(ps[u][v], 4 * q);
   };
   // A step's matrix as operands: s[4 i + e] = S(16 ((cw + i) % KD) + 4 kq + e, 16 cw + tl). The wave's own
   // 16 columns of the state come first: their products need no exchange.
@@ -288,7 +311,7 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
   };
   auto write_x = [&](int b, f32x4 v) { *reinterpret_cast<f32x4*>(&X[b][rb][tl][4 * ((4 * cw + kq) ^ tl)]) = v; };
 
-  f32x4 x = ld4(make_rsrc(start, start ? cb : 0u), xo, xc);
+  f32x4 x = placed(ld4(make_rsrc(start, start ? cb : 0u), xo, xc), xc);
   if (ident) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = xr < D && xr == xc + i ? 1.f : 0.f;
@@ -348,8 +371,9 @@ __global__ __launch_bounds__(aff::threads(DC), 2) void k_aff_scan(aff::ScanArgs 
       for (int o = j * NO / NM; o < (j + 1) * NO / NM; ++o) other(o);
       __builtin_amdgcn_sched_barrier(0);
     }
+    const f32x4 c = placed(cv[u], xc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = (acc[0][i] + acc[1][i]) + (own[0][i] + own[1][i]) + cv[u][i];
+    for (int i = 0; i < 4; ++i) x[i] = (acc[0][i] + acc[1][i]) + (own[0][i] + own[1][i]) + c[i];
     write_x((u + 1) & 1, x);
     st4(y, bo.r, wo + at(bo, cb, u), wc);   // the state before step k
     load_c(u, bc);
@@ -458,7 +482,7 @@ size_t affine_ws_bytes(const Geo& g) {
 
 template <bool REV, int DC>
 void launch_scan_d(aff::ScanArgs& a, int blocks, hipStream_t s) {
-  const int rb = DC ? aff::threads(DC) / (4 * DC) : 1;   // 16-row blocks of a workgroup
+  const int rb = DC > 0 ? aff::threads(DC) / (4 * DC) : 1;   // 16-row blocks of a workgroup
   a.parts = (blocks + rb - 1) / rb;
   hipLaunchKernelGGL((k_aff_scan<REV, DC>), dim3((unsigned)((a.units + 7) / 8 * 8 * a.parts)), dim3(aff::threads(DC)),
                      0, s, a);
@@ -470,7 +494,9 @@ void launch_scan(aff::ScanArgs& a, int blocks, hipStream_t s) {
     case 48: return launch_scan_d<REV, 48>(a, blocks, s);
     case 32: return launch_scan_d<REV, 32>(a, blocks, s);
     case 16: return launch_scan_d<REV, 16>(a, blocks, s);
-    default: return launch_scan_d<REV, 0>(a, blocks, s);
+    default:
+      if (a.g.D < 4) return launch_scan_d<REV, aff::kTiny>(a, blocks, s);
+      return launch_scan_d<REV, aff::kAny>(a, blocks, s);
   }
 }
 

@@ -50,3 +50,19 @@ def test_affine_chunks(N, T, R, D, with_prev, offset):
     compare("affine.out", out.detach().cpu(), ref.detach(), 8e-5)
     for nm, a, b in zip(("dA", "dB", "dprev"), gg, rg):
         compare(f"affine.{nm}", a.cpu(), b, 8e-5)
+
+
+@pytest.mark.parametrize("N,T,R,D,with_prev,offset", [
+    (2, 37, 5, 3, True, 1),        # rows shorter than a group of four
+    (3, 50, 2, 2, False, 0),
+    (2, 41, 17, 4, True, 1),       # one group a row
+    (2, 60, 64, 5, True, 0),       # a row's last group holds one, two and three of its elements
+    (3, 33, 16, 6, False, 2),
+    (2, 70, 33, 7, True, 3),
+    (4, 90, 64, 61, True, 1),
+    (40, 20, 64, 62, True, 0),     # one chunk
+    (16, 130, 64, 60, True, 0),
+    (3, 129, 64, 50, True, 2),
+])
+def test_affine_sizes_between(N, T, R, D, with_prev, offset):
+    test_affine_chunks(N, T, R, D, with_prev, offset)
