@@ -8,13 +8,20 @@
 //
 // Bound: HBM. The separate scans, products, window sums and copies moved about 30 tensors of [BH, n, P]
 // per forward + backward in 32 launches; here the forward reads the surprises and writes the updates
-// (and the momenta, when a backward follows), the backward reads dupdate, update and the momenta and
-// writes dsurprise. One wave owns 64 * V columns of one row and walks n with every recurrence in
-// registers; U steps of loads are in flight ahead of the step they feed, so that about 16 KB per wave
-// hide the latency without more waves than BH * P / 128.
-// The scalars' gradients are dot products over P: each wave sums its columns (DPP) into a per-wave
-// partial and a second launch adds the partials in a fixed order (no atomics: bitwise reproducible).
+// (and, when a backward follows, the momenta and a second copy of the updates), the backward reads dupdate,
+// that copy and the momenta and writes dsurprise. One wave owns 64 * V columns of one row and walks n with every
+// recurrence in registers. The operands of the kU = 8 steps ahead are in flight: per wave 4 KB (fp32, V = 2; bf16
+// half) in the forward, 12 KB (order 2: 16) in the backward.
+// What the walk leaves out of a step, since one wave to a SIMD issues it alone where BH * P is small: no load whose
+// value outlives a branch and no store under a condition (the wave would wait there for every access in flight),
+// addresses are a wave-uniform pointer and a fixed lane offset, and eight steps' sums over the lanes are formed
+// together (sums8). 16 x 64 x 8192 fp32, order 1: backward 48 -> 26.4 us, 5.1 TB/s, forward 24.6, 5.4 TB/s; 1 x 4096 x 64
+// of order 0 without gate or window, where the separate scans took 1012 us forward and backward: 1428 -> 831.
+// The scalars' gradients are dot products over P: each wave leaves its columns' sums as a partial and a second launch
+// adds the partials in a fixed order (no atomics: bitwise reproducible).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "../../include/atlas_mem.h"
 #include "mem_common.h"
@@ -41,46 +48,61 @@ struct Args {
   float *part;                                         // [bh, nblk, K, n], K = 1 (decay) + O + 1 (gate)
 };
 
+// V elements at a wave-uniform address plus the lane's byte offset.
 template <typename T, int V>
-__device__ __forceinline__ void ldv(const T* p, float* v) {
+__device__ __forceinline__ void ldv(const T* p, uint32_t lo, float* v) {
   typedef T vt __attribute__((ext_vector_type(V)));
+  const char* q = reinterpret_cast<const char*>(p) + lo;
   if constexpr (V == 1) {
-    v[0] = to_f32(p[0]);
+    v[0] = to_f32(*reinterpret_cast<const T*>(q));
   } else {
-    const vt u = *reinterpret_cast<const vt*>(p);
+    const vt u = *reinterpret_cast<const vt*>(q);
 #pragma unroll
     for (int i = 0; i < V; ++i) v[i] = to_f32(u[i]);
   }
 }
 template <typename T, int V>
-__device__ __forceinline__ void stv(T* p, const float* v) {
+__device__ __forceinline__ void stv(T* p, uint32_t lo, const float* v) {
   typedef T vt __attribute__((ext_vector_type(V)));
+  char* q = reinterpret_cast<char*>(p) + lo;
   if constexpr (V == 1) {
-    p[0] = from_f32<T>(v[0]);
+    *reinterpret_cast<T*>(q) = from_f32<T>(v[0]);
   } else {
     vt u;
 #pragma unroll
     for (int i = 0; i < V; ++i) u[i] = from_f32<T>(v[i]);
-    *reinterpret_cast<vt*>(p) = u;
+    *reinterpret_cast<vt*>(q) = u;
   }
 }
 __device__ __forceinline__ float lane_of(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dppz(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xf, false));
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
-// Sum over the 64 lanes, valid in lane 63.
-__device__ __forceinline__ float sum63(float v) {
-  v += dppz<0x111, 0xf>(v);
-  v += dppz<0x112, 0xf>(v);
-  v += dppz<0x114, 0xf>(v);
-  v += dppz<0x118, 0xf>(v);
-  v += dppz<0x142, 0xa>(v);
-  v += dppz<0x143, 0xc>(v);
-  return v;
+// The sums over the 64 lanes of eight values: lanes exchange halves of them (quad permutations), add up within their
+// row (rotations) and across the rows (the swaps of 32 and of 16 lanes), 27 instructions instead of the 6 dependent
+// ones of a sum each. Lane l returns the sum of value 4 (l & 1) + (l & 2) + (l >> 5).
+__device__ __forceinline__ float sums8(const float (&v)[8]) {
+  const int l = lane_id();
+  const bool b0 = l & 1, b1 = l & 2;
+  float w[4], x[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = (b0 ? v[i + 4] : v[i]) + dpp<0xb1>(b0 ? v[i] : v[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) x[i] = (b1 ? w[i + 2] : w[i]) + dpp<0x4e>(b1 ? w[i] : w[i + 2]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    x[i] += dpp<0x128>(x[i]);   // row_ror 8, 4
+    x[i] += dpp<0x124>(x[i]);
+  }
+  const auto h = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x[0]), __builtin_bit_cast(unsigned, x[1]), false, false);
+  const float y = __builtin_bit_cast(float, (unsigned)h[0]) + __builtin_bit_cast(float, (unsigned)h[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, y), __builtin_bit_cast(unsigned, y), false, false);
+  return __builtin_bit_cast(float, (unsigned)q[0]) + __builtin_bit_cast(float, (unsigned)q[1]);
 }
+__device__ __forceinline__ int sums8_value(int l) { return 4 * (l & 1) + (l & 2) + (l >> 5); }
 
 // Every gate of the batch below the threshold (a NaN is not). The first 64 gates settle it for any
 // memory that is in use; all of them are read only when the chunk is really switched off.
@@ -95,86 +117,99 @@ __device__ __forceinline__ bool gates_off(const T* gate, int64_t count) {
   return true;
 }
 
+// The wave's columns: lanes past the row's end stand in for lane 0, whose values they compute and store a second time
+// (a wave's stores are then the same for every wave, under no condition).
+template <typename T, int V>
+struct Cols {
+  bool act;
+  uint32_t lo;        // the lane's byte offset
+  int64_t first;      // the wave's first column
+  __device__ __forceinline__ Cols(int64_t p) {
+    first = (int64_t)blockIdx.x * (64 * V);
+    act = first + lane_id() * V < p;
+    lo = act ? (uint32_t)(lane_id() * V * (int)sizeof(T)) : 0u;
+  }
+};
+
 // E: window capacity (e <= E), O: momentum order, V: columns per lane
 template <typename T, int V, int E, int O>
 __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
   const int row = blockIdx.y, lane = lane_id();
-  const int64_t col0 = ((int64_t)blockIdx.x * 64 + lane) * V;
-  const bool act = col0 < a.p;
-  const int64_t col = act ? col0 : 0;
+  const Cols<T, V> col(a.p);
+  const uint32_t lo = col.lo;
   const int n = a.n, e = a.e;
   const int64_t p = a.p, rp = (int64_t)row * p;
   const bool off = gates_off(a.gate, (int64_t)a.bh * n);
-  const T* sp = a.s + rp * n + col;
-  T* up = a.update + rp * (n + 1) + col;
-  T* kp = a.kept ? a.kept + rp * (n + 1) + col : nullptr;
+  const T* sp = a.s + rp * n + col.first;
+  T* up = a.update + rp * (n + 1) + col.first;
+  T* kp = a.kept ? a.kept + rp * (n + 1) + col.first : nullptr;
+  const T* gate = (a.gate ? a.gate : a.decay) + (int64_t)row * n;   // (loaded without a branch)
+  const T* decay = a.decay + (int64_t)row * n;
 
   float m[O > 0 ? O : 1][V], c[V], hist[E > 1 ? E - 1 : 1][V];
-  ldv<T, V>(a.last + rp + col, c);
+  ldv<T, V>(a.last + rp + col.first, lo, c);
 #pragma unroll
-  for (int o = 0; o < O; ++o) ldv<T, V>(a.lm0 + ((int64_t)o * a.bh + row) * p + col, m[o]);
+  for (int o = 0; o < O; ++o) ldv<T, V>(a.lm0 + ((int64_t)o * a.bh + row) * p + col.first, lo, m[o]);
   if constexpr (E > 1) {
 #pragma unroll
     for (int j = 0; j < E - 1; ++j) {
 #pragma unroll
       for (int i = 0; i < V; ++i) hist[j][i] = 0.f;
-      if (j < e - 1 && a.buf) ldv<T, V>(a.buf + ((int64_t)row * (e - 1) + (e - 2 - j)) * p + col, hist[j]);
+      if (j < e - 1 && a.buf) ldv<T, V>(a.buf + ((int64_t)row * (e - 1) + (e - 2 - j)) * p + col.first, lo, hist[j]);
     }
     // the buffer's slots that stay in the window (fewer tokens than slots)
     for (int i = n; i < e - 1; ++i) {
       float b[V] = {};
-      if (a.buf) ldv<T, V>(a.buf + ((int64_t)row * (e - 1) + i) * p + col, b);
-      if (act) stv<T, V>(a.buf1 + ((int64_t)row * (e - 1) + (i - n)) * p + col, b);
+      if (a.buf) ldv<T, V>(a.buf + ((int64_t)row * (e - 1) + i) * p + col.first, lo, b);
+      stv<T, V>(a.buf1 + ((int64_t)row * (e - 1) + (i - n)) * p + col.first, lo, b);
     }
   }
   float zero[V] = {};
-  if (act) stv<T, V>(up, off ? zero : c);
-  if (act && kp) stv<T, V>(kp, off ? zero : c);
+  stv<T, V>(up, lo, off ? zero : c);
+  if (kp) stv<T, V>(kp, lo, off ? zero : c);
 
-  float cur[kU][V], nxt[kU][V];
-  float sc[2 + (O > 0 ? O : 1)], scn[2 + (O > 0 ? O : 1)];   // lane u: the scalars of step u of the group
-  auto load = [&](float (&x)[kU][V], float* s, int t0) {
+  // step u of a group of kU: the surprises of the step kU later take its registers as it is done, the scalars of
+  // the next group are in flight (lane u: step u's)
+  float x[kU][V], sc[2 + O], scn[2 + O];
+  auto load_scalars = [&](int t0) {
     const int tl = min(t0 + (lane & (kU - 1)), n - 1);
-    s[0] = to_f32(a.decay[(int64_t)row * n + tl]);
-    s[1] = a.gate ? to_f32(a.gate[(int64_t)row * n + tl]) : 1.f;
+    scn[0] = to_f32(decay[tl]);
+    scn[1] = to_f32(gate[tl]);
 #pragma unroll
-    for (int o = 0; o < O; ++o) s[2 + o] = to_f32(a.am[((int64_t)o * a.bh + row) * n + tl]);
-#pragma unroll
-    for (int u = 0; u < kU; ++u) ldv<T, V>(sp + (int64_t)min(t0 + u, n - 1) * p, x[u]);
+    for (int o = 0; o < O; ++o) scn[2 + o] = to_f32(a.am[((int64_t)o * a.bh + row) * n + tl]);
   };
-  load(nxt, scn, 0);
-  for (int t0 = 0; t0 < n; t0 += kU) {
+  load_scalars(0);
 #pragma unroll
-    for (int u = 0; u < kU; ++u)
-#pragma unroll
-      for (int i = 0; i < V; ++i) cur[u][i] = nxt[u][i];
+  for (int u = 0; u < kU; ++u) ldv<T, V>(sp + (int64_t)min(u, n - 1) * p, lo, x[u]);
+  auto group = [&](auto whole, int t0) {
 #pragma unroll
     for (int k = 0; k < 2 + O; ++k) sc[k] = scn[k];
-    load(nxt, scn, t0 + kU);
+    load_scalars(t0 + kU);
     if (a.kdecay && blockIdx.x == 0 && lane < kU && t0 + lane < n) a.kdecay[(int64_t)row * n + t0 + lane] = from_f32<T>(sc[0]);
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int t = t0 + u;
-      if (t < n) {
+      if (decltype(whole)::value || t < n) {
         const float keep = 1.f - lane_of(sc[0], u), g = lane_of(sc[1], u);
-        float x[V], w[V];
+        float y[V], w[V];
 #pragma unroll
-        for (int i = 0; i < V; ++i) x[i] = cur[u][i];
+        for (int i = 0; i < V; ++i) y[i] = x[u][i];
+        ldv<T, V>(sp + (int64_t)min(t + kU, n - 1) * p, lo, x[u]);
 #pragma unroll
         for (int o = 0; o < O; ++o) {
           const float am = lane_of(sc[2 + o], u);
 #pragma unroll
-          for (int i = 0; i < V; ++i) x[i] = m[o][i] = am * m[o][i] + x[i];
-          if (a.moms && act) stv<T, V>(a.moms + (((int64_t)o * a.bh + row) * n + t) * p + col, x);
+          for (int i = 0; i < V; ++i) y[i] = m[o][i] = am * m[o][i] + y[i];
+          if (a.moms) stv<T, V>(a.moms + (((int64_t)o * a.bh + row) * n + t) * p + col.first, lo, y);
         }
         if (a.gate) {
 #pragma unroll
-          for (int i = 0; i < V; ++i) x[i] *= g;
+          for (int i = 0; i < V; ++i) y[i] *= g;
         }
 #pragma unroll
-        for (int i = 0; i < V; ++i) w[i] = E > 1 ? 0.f : x[i];
+        for (int i = 0; i < V; ++i) w[i] = E > 1 ? 0.f : y[i];
         if constexpr (E > 1) {
-          if (t + e - 1 >= n && act) stv<T, V>(a.buf1 + ((int64_t)row * (e - 1) + (t + e - 1 - n)) * p + col, x);
+          if (t + e - 1 >= n) stv<T, V>(a.buf1 + ((int64_t)row * (e - 1) + (t + e - 1 - n)) * p + col.first, lo, y);
 #pragma unroll
           for (int j = E - 2; j >= 0; --j)   // oldest first, as atlas_window_sum adds
             if (j < e - 1) {
@@ -182,103 +217,105 @@ __global__ __launch_bounds__(64) void k_chain_fwd(Args<T> a) {
               for (int i = 0; i < V; ++i) w[i] += hist[j][i];
             }
 #pragma unroll
-          for (int i = 0; i < V; ++i) w[i] += x[i];
+          for (int i = 0; i < V; ++i) w[i] += y[i];
 #pragma unroll
           for (int j = E - 2; j > 0; --j)
 #pragma unroll
             for (int i = 0; i < V; ++i) hist[j][i] = hist[j - 1][i];
 #pragma unroll
-          for (int i = 0; i < V; ++i) hist[0][i] = x[i];
+          for (int i = 0; i < V; ++i) hist[0][i] = y[i];
         }
 #pragma unroll
         for (int i = 0; i < V; ++i) c[i] = keep * c[i] + w[i];
-        if (act) stv<T, V>(up + (int64_t)(t + 1) * p, off ? zero : c);
-        if (act && kp) stv<T, V>(kp + (int64_t)(t + 1) * p, off ? zero : c);
+        stv<T, V>(up + (int64_t)(t + 1) * p, lo, off ? zero : c);
+        if (kp) stv<T, V>(kp + (int64_t)(t + 1) * p, lo, off ? zero : c);
       }
     }
-  }
+  };
+  int t0 = 0;
+  for (; t0 + kU <= n; t0 += kU) group(std::true_type{}, t0);
+  if (t0 < n) group(std::false_type{}, t0);
 #pragma unroll
-  for (int o = 0; o < O; ++o)
-    if (act) stv<T, V>(a.lm1 + ((int64_t)o * a.bh + row) * p + col, m[o]);
+  for (int o = 0; o < O; ++o) stv<T, V>(a.lm1 + ((int64_t)o * a.bh + row) * p + col.first, lo, m[o]);
 }
 
 // The reverse walk: lc the adjoint of c, lm[o] of m_o; hist[j] = du_{t+1+j}.
 template <typename T, int V, int E, int O>
 __global__ __launch_bounds__(64) void k_chain_bwd(Args<T> a) {
-  constexpr int K = 2 + O;
+  constexpr int K = 2 + O, B = O > 0 ? O : 1;
   const int row = blockIdx.y, lane = lane_id();
-  const int64_t col0 = ((int64_t)blockIdx.x * 64 + lane) * V;
-  const bool act = col0 < a.p;
-  const int64_t col = act ? col0 : 0;
+  const Cols<T, V> col(a.p);
+  const uint32_t lo = col.lo;
   const int n = a.n, e = a.e;
   const int64_t p = a.p, rp = (int64_t)row * p;
   const bool off = gates_off(a.gate, (int64_t)a.bh * n);
-  const bool live = act && !off && a.dup;     // dupdate reaches this column
-  const T* dp = a.dup ? a.dup + rp * (n + 1) + col : nullptr;
-  const T* cp = a.upd + rp * (n + 1) + col;   // row t: c_{t-1}
-  const T* bp[O > 0 ? O : 1];                 // momenta of order o (order 0: the surprises, which only the gate's
-                                              // gradient needs: any readable rows where they are absent)
+  const bool live = !off && a.dup;            // dupdate reaches the columns
+  const T* cp = a.upd + rp * (n + 1) + col.first;   // row t: c_{t-1}
+  const T* dp = a.dup ? a.dup + rp * (n + 1) + col.first : cp;   // (absent: readable rows, not used)
+  const T* gate = (a.gate ? a.gate : a.decay) + (int64_t)row * n;
+  const T* decay = a.decay + (int64_t)row * n;
+  const T *bp[B], *b0[B];                     // momenta of order o and the one before the first step (order 0: the
+                                              // surprises, which only the gate's gradient needs: readable rows where
+                                              // they are absent, and before the first step)
   if constexpr (O > 0) {
 #pragma unroll
-    for (int o = 0; o < O; ++o) bp[o] = a.msrc + ((int64_t)o * a.bh + row) * n * p + col;
+    for (int o = 0; o < O; ++o) {
+      bp[o] = a.msrc + ((int64_t)o * a.bh + row) * n * p + col.first;
+      b0[o] = a.lm0 + ((int64_t)o * a.bh + row) * p + col.first;
+    }
   } else {
-    bp[0] = a.s ? a.s + rp * n + col : cp;
+    bp[0] = b0[0] = a.s ? a.s + rp * n + col.first : cp;
   }
+  T* ds = a.ds + rp * n + col.first;
   float* part = a.part + ((int64_t)row * gridDim.x + blockIdx.x) * K * n;
 
-  float lc[V] = {}, lm[O > 0 ? O : 1][V] = {}, hist[E > 1 ? E - 1 : 1][V] = {};
-  float base[O > 0 ? O : 1][V];               // m_o at the step (order 0: the surprise)
-  constexpr int B = O > 0 ? O : 1;
+  float lc[V] = {}, lm[B][V] = {}, hist[E > 1 ? E - 1 : 1][V] = {};
+  float base[B][V];                           // m_o at the step (order 0: the surprise)
 #pragma unroll
-  for (int o = 0; o < B; ++o) ldv<T, V>(bp[o] + (int64_t)(n - 1) * p, base[o]);
+  for (int o = 0; o < B; ++o) ldv<T, V>(bp[o] + (int64_t)(n - 1) * p, lo, base[o]);
 
-  // group [t1 - U, t1) walked from its end: step u is t = t1 - 1 - u
-  float dn[kU][V], cn[kU][V], bn[B][kU][V], sn[K];
-  float dc[kU][V], cc[kU][V], bc[B][kU][V], sc[K];
-  auto load = [&](int t1) {
+  // groups [t1 - kU, t1) walked from their end, step u at t = t1 - 1 - u; the operands of the step kU further take a
+  // step's registers as it is done. No load whose value outlives a branch is in the walk: at the join the wave would
+  // wait for every access in flight, its own stores included.
+  float dn[kU][V], cn[kU][V], bn[B][kU][V], sn[K], sc[K];
+  auto load = [&](int u, int t) {             // t may lie before the first step (read from it, not used)
+    const int64_t r = (int64_t)max(t, 0) * p;
+    ldv<T, V>(dp + r + p, lo, dn[u]);
+    ldv<T, V>(cp + r, lo, cn[u]);
+#pragma unroll
+    for (int o = 0; o < B; ++o) ldv<T, V>(t > 0 ? bp[o] + r - p : b0[o], lo, bn[o][u]);   // the step before
+  };
+  auto load_scalars = [&](int t1) {
     const int tl = max(t1 - 1 - (lane & (kU - 1)), 0);
-    sn[0] = to_f32(a.decay[(int64_t)row * n + tl]);
-    sn[1] = a.gate ? to_f32(a.gate[(int64_t)row * n + tl]) : 1.f;
+    sn[0] = to_f32(decay[tl]);
+    sn[1] = to_f32(gate[tl]);
 #pragma unroll
     for (int o = 0; o < O; ++o) sn[2 + o] = to_f32(a.am[((int64_t)o * a.bh + row) * n + tl]);
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t t = max(t1 - 1 - u, 0);
-#pragma unroll
-      for (int i = 0; i < V; ++i) dn[u][i] = 0.f;
-      if (dp) ldv<T, V>(dp + (t + 1) * p, dn[u]);
-      ldv<T, V>(cp + t * p, cn[u]);
-#pragma unroll
-      for (int o = 0; o < B; ++o) ldv<T, V>(bp[o] + max(t - 1, (int64_t)0) * p, bn[o][u]);   // the step before
-    }
   };
-  load(n);
-  float keep_next = 0.f, am_next[O > 0 ? O : 1] = {};
-  for (int t1 = n; t1 > 0; t1 -= kU) {
+  load_scalars(n);
 #pragma unroll
-    for (int u = 0; u < kU; ++u)
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        dc[u][i] = dn[u][i];
-        cc[u][i] = cn[u][i];
-#pragma unroll
-        for (int o = 0; o < B; ++o) bc[o][u][i] = bn[o][u][i];
-      }
+  for (int u = 0; u < kU; ++u) load(u, n - 1 - u);
+  float keep_next = 0.f, am_next[B] = {};
+  auto group = [&](auto whole, int t1) {
+    float acc[K][kU] = {};
 #pragma unroll
     for (int k = 0; k < K; ++k) sc[k] = sn[k];
-    load(t1 - kU);
+    load_scalars(t1 - kU);
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int t = t1 - 1 - u;
-      if (t >= 0) {
+      if (decltype(whole)::value || t >= 0) {
         const float keep = 1.f - lane_of(sc[0], u), g = lane_of(sc[1], u);
-        float dx[V], acc[K] = {};
+        float dx[V], prev[B][V];
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-          lc[i] = (live ? dc[u][i] : 0.f) + keep_next * lc[i];
+          lc[i] = (live ? dn[u][i] : 0.f) + keep_next * lc[i];
           dx[i] = lc[i];
-          acc[0] -= lc[i] * cc[u][i];
+          acc[0][u] -= lc[i] * cn[u][i];
+#pragma unroll
+          for (int o = 0; o < B; ++o) prev[o][i] = bn[o][u][i];
         }
+        load(u, t - kU);
         if constexpr (E > 1) {
 #pragma unroll
           for (int j = 0; j < E - 1; ++j)
@@ -294,68 +331,66 @@ __global__ __launch_bounds__(64) void k_chain_bwd(Args<T> a) {
           for (int i = 0; i < V; ++i) hist[0][i] = lc[i];
           if (a.dbuf1 && t + e - 1 >= n) {
             float b[V];
-            ldv<T, V>(a.dbuf1 + ((int64_t)row * (e - 1) + (t + e - 1 - n)) * p + col, b);
+            ldv<T, V>(a.dbuf1 + ((int64_t)row * (e - 1) + (t + e - 1 - n)) * p + col.first, lo, b);
 #pragma unroll
-            for (int i = 0; i < V; ++i) dx[i] += act ? b[i] : 0.f;
+            for (int i = 0; i < V; ++i) dx[i] += b[i];
           }
         }
         if (a.gate) {
 #pragma unroll
           for (int i = 0; i < V; ++i) {
-            acc[1] += dx[i] * base[B - 1][i];
+            acc[1][u] += dx[i] * base[B - 1][i];
             dx[i] *= g;
           }
         }
 #pragma unroll
         for (int o = O - 1; o >= 0; --o) {
-          float prev[V];
-          if (t > 0) {
-#pragma unroll
-            for (int i = 0; i < V; ++i) prev[i] = bc[o][u][i];
-          } else {
-            ldv<T, V>(a.lm0 + ((int64_t)o * a.bh + row) * p + col, prev);
-          }
           if (a.dlm1 && t == n - 1) {
             float b[V];
-            ldv<T, V>(a.dlm1 + ((int64_t)o * a.bh + row) * p + col, b);
+            ldv<T, V>(a.dlm1 + ((int64_t)o * a.bh + row) * p + col.first, lo, b);
 #pragma unroll
-            for (int i = 0; i < V; ++i) dx[i] += act ? b[i] : 0.f;
+            for (int i = 0; i < V; ++i) dx[i] += b[i];
           }
 #pragma unroll
           for (int i = 0; i < V; ++i) {
             lm[o][i] = dx[i] + am_next[o] * lm[o][i];
             dx[i] = lm[o][i];
-            acc[2 + o] += lm[o][i] * prev[i];
-            base[o][i] = prev[i];
+            acc[2 + o][u] += lm[o][i] * prev[o][i];
           }
           am_next[o] = lane_of(sc[2 + o], u);
         }
-        if constexpr (O == 0) {
 #pragma unroll
-          for (int i = 0; i < V; ++i) base[0][i] = bc[0][u][i];
-        }
+        for (int o = 0; o < B; ++o)
+#pragma unroll
+          for (int i = 0; i < V; ++i) base[o][i] = prev[o][i];
         keep_next = keep;
-        if (act) stv<T, V>(a.ds + (rp * n + (int64_t)t * p) + col, dx);
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          if (k == 1 && !a.gate) continue;
-          const float s = sum63(act ? acc[k] : 0.f);
-          if (lane == 63) part[(int64_t)k * n + t] = s;
-        }
+        stv<T, V>(ds + (int64_t)t * p, lo, dx);
       }
     }
-  }
-  if (!act) return;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k == 1 && !a.gate) continue;
+      float v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) v[u] = col.act ? acc[k][u] : 0.f;
+      const float s = sums8(v);
+      const int t = t1 - 1 - sums8_value(lane);
+      if ((lane & 28) == 0 && t >= 0) part[(int64_t)k * n + t] = s;
+    }
+  };
+  int t1 = n;
+  for (; t1 >= kU; t1 -= kU) group(std::true_type{}, t1);
+  if (t1 > 0) group(std::false_type{}, t1);
   float d0[V] = {};
-  if (live) ldv<T, V>(dp, d0);
+  if (live) ldv<T, V>(dp, lo, d0);
 #pragma unroll
   for (int i = 0; i < V; ++i) d0[i] += keep_next * lc[i];
-  stv<T, V>(a.dlast + rp + col, d0);
+  stv<T, V>(a.dlast + rp + col.first, lo, d0);
 #pragma unroll
   for (int o = 0; o < O; ++o) {
 #pragma unroll
     for (int i = 0; i < V; ++i) lm[o][i] *= am_next[o];
-    stv<T, V>(a.dlm0 + ((int64_t)o * a.bh + row) * p + col, lm[o]);
+    stv<T, V>(a.dlm0 + ((int64_t)o * a.bh + row) * p + col.first, lo, lm[o]);
   }
   if constexpr (E > 1) {
     if (a.dbuf) {   // slot i: du_0 .. du_min(n - 1, i) (hist[t] = du_t now, zero past n) and its copy in the next buffer
@@ -364,13 +399,13 @@ __global__ __launch_bounds__(64) void k_chain_bwd(Args<T> a) {
       for (int j = 0; j < E - 1; ++j) {
         if (j < e - 1) {
           float b[V] = {}, o[V];
-          if (a.dbuf1 && j >= n) ldv<T, V>(a.dbuf1 + ((int64_t)row * (e - 1) + (j - n)) * p + col, b);
+          if (a.dbuf1 && j >= n) ldv<T, V>(a.dbuf1 + ((int64_t)row * (e - 1) + (j - n)) * p + col.first, lo, b);
 #pragma unroll
           for (int i = 0; i < V; ++i) {
             run[i] += hist[j][i];
             o[i] = run[i] + b[i];
           }
-          stv<T, V>(a.dbuf + ((int64_t)row * (e - 1) + j) * p + col, o);
+          stv<T, V>(a.dbuf + ((int64_t)row * (e - 1) + j) * p + col.first, lo, o);
         }
       }
     }

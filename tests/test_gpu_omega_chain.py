@@ -151,3 +151,14 @@ def test_chain_without_a_gradient_of_the_gate():
             grads.append(torch.autograd.grad(sum((o * o).sum() for o in out if o is not None), [leaves[k] for k in names]))
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("BH,n,p,O,gate,e,dt", [
+    (2, 16, (64,), 0, False, 1, torch.float32),    # whole groups of steps alone; half a wave of columns
+    (1, 24, (130,), 2, True, 1, torch.float32),    # a second wave of one lane
+    (3, 25, (129,), 1, False, 2, torch.float32),   # a step past the groups; one column a lane
+    (2, 33, (256,), 0, True, 1, BF16),
+])
+def test_chain_groups_of_steps(BH, n, p, O, gate, e, dt):
+    print("chain groups", BH, n, p, O, gate, e, dt, flush=True)
+    _check(_inputs(BH, n, p, O, False, gate, e, e > 1, seed=n, dt=dt), e, dt, f"chain_groups_{n}")
