@@ -223,11 +223,11 @@ bool shape_is(const Tensor& t, at::IntArrayRef want) { return !t.defined() || t.
 std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const Tensor& v, const Tensor& lr,
                                          const Tensor& decay, const Tensor& beta, const Tensor& gate, Tensor S_ref,
                                          Tensor S0, Tensor Z0, Tensor buf, int64_t window, int64_t map_degree,
-                                         std::optional<int64_t> clamp_every, bool clamp_final) {
+                                         std::optional<int64_t> clamp_every, int64_t clamp_final) {
   if (k.dim() != 3 || v.dim() != 3 || !k.is_cuda()) return std::nullopt;
   const int64_t bh = k.size(0), T = k.size(1), dk = k.size(2), dv = v.size(2);
   if (dk != dv || (dk != 32 && dk != 64) || window < 1 || window > 64 || bh < 1 || T < 1 || bh > INT32_MAX ||
-      T > INT32_MAX || map_degree < INT32_MIN || map_degree > INT32_MAX)
+      T > INT32_MAX || map_degree < INT32_MIN || map_degree > INT32_MAX || clamp_final < 0 || clamp_final > 1)
     return std::nullopt;
   int gate_mode = ATLAS_GATE_NONE;
   if (gate.defined()) {
@@ -259,7 +259,7 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
   if (!p.momentum) Z0 = Tensor();
   p.has_buffer = buf.defined();
   p.clamp_every = (int)clamp_every.value_or(0);
-  p.clamp_final = clamp_final;
+  p.clamp_final = (int)clamp_final;
   p.dtype = dt == at::kBFloat16 ? ATLAS_DT_BF16 : ATLAS_DT_F32;
   if (lib().atlas_mem_validate(&p) != ATLAS_MEM_OK) return std::nullopt;
   c10::DeviceGuard guard(k.device());
@@ -298,7 +298,7 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
 py::object recurrence(const Tensor& k, const Tensor& q, const Tensor& v, const Tensor& lr, const Tensor& decay,
                       const OptTensor& beta, const OptTensor& gate, const OptTensor& S_ref, const OptTensor& S0,
                       const OptTensor& Z0, const OptTensor& buffer, int64_t window, int64_t map_degree,
-                      std::optional<int64_t> clamp_every, bool clamp_final) {
+                      std::optional<int64_t> clamp_every, int64_t clamp_final) {
   const std::optional<RecOut> o = recurrence_or_none(k, q, v, lr, decay, get(beta), get(gate), get(S_ref), get(S0), get(Z0),
                                                      get(buffer), window, map_degree, clamp_every, clamp_final);
   if (!o.has_value()) return py::none();

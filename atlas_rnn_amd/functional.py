@@ -537,7 +537,7 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
     if clamp_every is not None and k.dim() == 3 and clamp_every >= k.shape[1]:
         clamp_every = None        # no clamp point before the last token (the final clamp is clamp_final's)
     out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
-                                   map_degree if map_mode == 'elementwise' else 1, clamp_every, bool(clamp_final))
+                                   map_degree if map_mode == 'elementwise' else 1, clamp_every, int(clamp_final))
     if out is not None:
         return out
     # everything the kernels do not take as it is: other head sizes, calls in pieces, and the errors
@@ -614,7 +614,7 @@ class MemoryRecurrenceFn:
         _lib.check(_lib.load().atlas_mem_validate(ctypes.byref(prob)), "atlas_mem_validate")
         y, S_T, Z_T, buf_out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg.window,
                                        cfg.map_degree if cfg.map_mode == 'elementwise' else 1, cfg.clamp_every or None,
-                                       bool(cfg.clamp_final))
+                                       int(cfg.clamp_final))
         empty = torch.empty(0, device=dev)
         return y, S_T, Z_T if Z_T is not None else empty, buf_out if buf_out is not None else empty
 

@@ -158,3 +158,11 @@ def test_the_cell_runs_its_merge_heads_module():
     assert seen == [((3, 2, 5, 32), (3, 5, 64))]
     cell.merge_heads._forward_hooks.clear()
     assert torch.allclose(doubled, 2 * cell(x)[0])
+
+
+def test_clamp_final_is_a_truth_value():
+    x = _ops(t=8)
+    for bad, error in ((None, TypeError), ("yes", ValueError), (2, RuntimeError)):
+        with pytest.raises(error):
+            am.memory_recurrence(**x, window=E, clamp_final=bad)
+    assert torch.equal(am.memory_recurrence(**x, window=E, clamp_final=1)[1], am.memory_recurrence(**x, window=E)[1])
