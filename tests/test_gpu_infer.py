@@ -53,3 +53,14 @@ def test_same_results_without_a_backward(name, c):
         assert not x.requires_grad
     if name == "clamp_acts":
         assert b[1].abs().max() == 100
+
+
+@pytest.mark.parametrize("name,c", [
+    ("walk", dict(BH=300, T=333, e=4)),                              # one segment of six chunks a row
+    ("walk_buffer", dict(BH=260, T=200, e=4, buffer=True)),          # two saved states a chunk
+    ("clamp", dict(BH=257, T=321, e=2, clamp=64)),                   # the same, checked at every chunk's end
+    ("walk_segments", dict(BH=40, T=1500, e=9, gate=True)),          # several segments of several chunks
+    ("d32", dict(BH=600, T=200, d=32, e=4)),
+], ids=lambda v: v if isinstance(v, str) else "")
+def test_same_results_over_several_chunks_a_segment(name, c):
+    test_same_results_without_a_backward(name, {"d": 64, "dtype": BF16, **c})
