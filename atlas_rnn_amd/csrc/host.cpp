@@ -132,8 +132,6 @@ Tensor plain(const Tensor& ref, at::IntArrayRef sizes) { return at::empty(sizes,
 // a workspace of at least `bytes` bytes, as fp32
 Tensor scratch(const Tensor& ref, int64_t bytes) { return f32(ref, {(std::max<int64_t>(bytes, 16) + 3) / 4}); }
 
-py::object obj(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
-
 // ---------------------------------------------------------------------------------------------
 // the recurrence (atlas_pytorch/rnn_memory.py:300-406, :605-730)
 // ---------------------------------------------------------------------------------------------
@@ -295,14 +293,17 @@ std::optional<RecOut> recurrence_or_none(const Tensor& k, const Tensor& q, const
   return o;
 }
 
-py::object recurrence(const Tensor& k, const Tensor& q, const Tensor& v, const Tensor& lr, const Tensor& decay,
-                      const OptTensor& beta, const OptTensor& gate, const OptTensor& S_ref, const OptTensor& S0,
-                      const OptTensor& Z0, const OptTensor& buffer, int64_t window, int64_t map_degree,
-                      std::optional<int64_t> clamp_every, int64_t clamp_final) {
+// y, S_T, Z_T, buffer_out (None: absent)
+typedef std::tuple<Tensor, Tensor, OptTensor, OptTensor> Four;
+
+std::optional<Four> recurrence(const Tensor& k, const Tensor& q, const Tensor& v, const Tensor& lr, const Tensor& decay,
+                               const OptTensor& beta, const OptTensor& gate, const OptTensor& S_ref, const OptTensor& S0,
+                               const OptTensor& Z0, const OptTensor& buffer, int64_t window, int64_t map_degree,
+                               std::optional<int64_t> clamp_every, int64_t clamp_final) {
   const std::optional<RecOut> o = recurrence_or_none(k, q, v, lr, decay, get(beta), get(gate), get(S_ref), get(S0), get(Z0),
                                                      get(buffer), window, map_degree, clamp_every, clamp_final);
-  if (!o.has_value()) return py::none();
-  return py::make_tuple(o->y, o->S_T, obj(o->Z_T), obj(o->buf));
+  if (!o.has_value()) return std::nullopt;
+  return Four{o->y, o->S_T, opt(o->Z_T), opt(o->buf)};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -897,13 +898,13 @@ struct OmegaChainFn : public Function<OmegaChainFn> {
 // None where the fused kernels do not apply: one dtype (fp32 or bf16) on one GPU for the surprises and
 // the scalars, at most two momentum orders and a window of at most 16 (both are held in registers),
 // and sizes inside their index ranges.
-py::object omega_chain(const Tensor& s, const Tensor& decay, const Tensor& last, const OptTensor& am, const OptTensor& lm,
-                       const OptTensor& gate, int64_t window, const OptTensor& buf) {
+std::optional<Four> omega_chain(const Tensor& s, const Tensor& decay, const Tensor& last, const OptTensor& am,
+                                const OptTensor& lm, const OptTensor& gate, int64_t window, const OptTensor& buf) {
   const at::ScalarType dt = s.scalar_type();
-  if (!kernel_dtype(dt) || !s.is_cuda() || window < 1 || window > 16 || s.dim() < 2 || s.numel() == 0) return py::none();
+  if (!kernel_dtype(dt) || !s.is_cuda() || window < 1 || window > 16 || s.dim() < 2 || s.numel() == 0) return std::nullopt;
   const int64_t BH = s.size(0), n = s.size(1), p = s.numel() / (BH * n), O = am.has_value() ? am->size(0) : 0;
   if ((am.has_value() && (O < 1 || O > 2 || !lm.has_value())) || BH > 65535 || n > (1 << 24) || p > ((int64_t)1 << 31))
-    return py::none();
+    return std::nullopt;
   bool grad = false;
   auto ok = [&](const Tensor& t, bool scalar) {
     grad = grad || t.requires_grad();
@@ -912,7 +913,7 @@ py::object omega_chain(const Tensor& s, const Tensor& decay, const Tensor& last,
   auto ook = [&](const OptTensor& t, bool scalar) { return !t.has_value() || ok(*t, scalar); };
   if (!ok(s, true) || !ok(decay, true) || !ok(last, false) || !ook(am, true) || !ook(lm, false) || !ook(gate, true) ||
       !ook(buf, false))
-    return py::none();
+    return std::nullopt;
   c10::DeviceGuard guard(s.device());
   // views only where the shape differs: each is a node of the autograd graph
   auto shaped = [](const Tensor& t, at::IntArrayRef sizes) { return t.sizes() == sizes ? t : t.reshape(sizes); };
@@ -932,14 +933,15 @@ py::object omega_chain(const Tensor& s, const Tensor& decay, const Tensor& last,
   const Tensor update = full(out[0], {BH, n + 1});
   size_t i = 1;
   const Tensor lm1 = O ? full(out[i++], {O, BH}) : Tensor(), buf1 = window > 1 ? full(out[i++], {BH, window - 1}) : Tensor();
-  return py::make_tuple(update, update.select(1, n), obj(lm1), obj(buf1));
+  return Four{update, update.select(1, n), opt(lm1), opt(buf1)};
 }
 
-// an entry point of the module: refused while torch.jit.trace records
+// an entry point of the module: refused while torch.jit.trace records, other Python threads run meanwhile
 template <typename R, typename... A>
 auto entry(R (*f)(A...)) {
   return [f](A... a) -> R {
     TORCH_CHECK(!torch::jit::tracer::isTracing(), "the native operators are not traced: call them through atlas_rnn_amd");
+    py::gil_scoped_release threads;
     return f(std::forward<A>(a)...);
   };
 }

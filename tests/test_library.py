@@ -1,14 +1,18 @@
-"""Which library the operators run on, and what is said and left behind when a part is missing (no GPU)."""
+"""Which library the operators run on, what is said and left behind when a part is missing, and that other threads
+run during a call (no GPU)."""
 
 import os
 import shutil
 import sys
+import threading
+import time
 
 import pytest
 import torch
 
 import atlas_rnn_amd
 from atlas_rnn_amd import _lib, build
+from atlas_rnn_amd import functional as F
 
 
 def test_the_operators_run_on_the_loaded_library(tmp_path, monkeypatch):
@@ -54,3 +58,29 @@ def test_a_missing_extension_module_is_reported(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
     ready, message = atlas_rnn_amd.check_cuda_availability()
     assert not ready and "_host" in message
+
+
+def test_other_threads_run_during_a_call():
+    x, w = torch.randn(2048, 2048), torch.randn(2048, 2048)
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(1e-3)
+
+    thread = threading.Thread(target=tick)
+    threads = torch.get_num_threads()
+    torch.set_num_threads(1)
+    thread.start()
+    try:
+        t0 = time.perf_counter()
+        for _ in range(2):
+            F.linear(x, w)         # some tens of milliseconds in one native call
+        t1 = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+        torch.set_num_threads(threads)
+    inside = [t for t in ticks if t0 < t < t1]
+    assert t1 - t0 > 0.02 and len(inside) > 5
