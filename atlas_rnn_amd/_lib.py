@@ -240,8 +240,8 @@ def native():
     code, on the library that load() has loaded. Raises LibraryMissing if it is not built; there is no other
     implementation."""
     global _NATIVE, _BOUND
-    lib = load()
-    if _BOUND is not lib:
+    if _BOUND is None or _BOUND is not _LIB:
+        lib = load()
         try:
             from . import _host
         except ImportError as exc:

@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
+from functools import partial
 
 import torch
 from torch import Tensor
@@ -122,12 +123,8 @@ class _TracedFn(torch.autograd.Function):
         return (None, *(next(got) if t.requires_grad else None for t in ctx.ins))
 
 
-def _native(op: str, *args):
-    """The native operator `op` (csrc/host.cpp) on args; None where it does not take them."""
-    fn = getattr(_lib.native(), op)
-    if not _is_tracing():
-        return fn(*args)
-    args = _map_tensors(args, lambda t: t)
+def _traced(op: str, fn, *args):
+    """The native operator fn (named op) while torch.jit.trace records."""
     with _no_trace(), torch.no_grad():   # which outputs there are, and whether the operator takes the operands
         layout = fn(*_map_tensors(args, lambda t: t.detach()))
     if layout is None:
@@ -136,6 +133,12 @@ def _native(op: str, *args):
     _map_tensors(args, tensors.append)
     outs = iter(_TracedFn.apply(_NativeCall(op, args), *tensors))
     return _map_tensors(layout, lambda t: next(outs))
+
+
+def _native(op: str):
+    """The native operator `op` (csrc/host.cpp); it returns None for operands that it does not take."""
+    fn = getattr(_lib.native(), op)
+    return partial(_traced, op, fn) if _is_tracing() else fn
 
 
 def check_operands(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, *, window: int,
@@ -259,7 +262,7 @@ def symmetrized_tables(proj: Tensor, d: int, dtype) -> tuple[Tensor, Tensor]:
     if dtype not in _DTYPES:
         raise ValueError(f"symmetrized_tables: dtype {dtype} (the kernels take bfloat16 or float32)")
     _require_gpu(proj)
-    return _native('symmetrized', proj, d, dtype)
+    return _native('symmetrized')(proj, d, dtype)
 
 
 class _TensorMapFn:
@@ -271,7 +274,7 @@ class _TensorMapFn:
     def apply(x, proj, degree, tables=None):
         _require_gpu(x, proj)
         ps, pst = tables if tables is not None else (None, None)
-        return _native('tensor_map', x, proj, degree, ps, pst)
+        return _native('tensor_map')(x, proj, degree, ps, pst)
 
 
 def _tables_ok(tables, proj: Tensor, dtype) -> bool:
@@ -320,7 +323,7 @@ class _ReplicateFn:
 
     @staticmethod
     def apply(nrep, *xs):
-        return tuple(_native('replicate', nrep, list(xs)))
+        return tuple(_native('replicate')(nrep, list(xs)))
 
 
 class _ReplicaSumFn:
@@ -328,7 +331,7 @@ class _ReplicaSumFn:
 
     @staticmethod
     def apply(nrep, *xs):
-        return tuple(_native('replica_sum', nrep, list(xs)))
+        return tuple(_native('replica_sum')(nrep, list(xs)))
 
 
 def _replicas(op: int, nrep: int, xs):
@@ -374,7 +377,7 @@ def block_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor,
     S_ref, S0, Z0, buffer = pst(S_ref), pst(S0), pst(Z0), pst(buffer)
     nb = nbv * nbk
     _dt_code(phi)   # fp32 or bf16
-    kb, qb, vb = _native('block_split', phi, psi, vv, S_ref)   # its adjoint: atlas_block_merge
+    kb, qb, vb = _native('block_split')(phi, psi, vv, S_ref)   # its adjoint: atlas_block_merge
 
     def stack_state(x):        # [BH, ..., Dv, Dk] -> [(i, j, bh), ..., 64, 64]
         if x is None:
@@ -536,7 +539,7 @@ def memory_recurrence(k: Tensor, q: Tensor, v: Tensor, lr: Tensor, decay: Tensor
     """
     if clamp_every is not None and k.dim() == 3 and clamp_every >= k.shape[1]:
         clamp_every = None        # no clamp point before the last token (the final clamp is clamp_final's)
-    out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
+    out = _native('recurrence')(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buffer, window,
                                    map_degree if map_mode == 'elementwise' else 1, clamp_every, int(clamp_final))
     if out is not None:
         return out
@@ -612,7 +615,7 @@ class MemoryRecurrenceFn:
         dev = _require_gpu(k, q, v, lr, decay, S_ref, S0)
         prob = _problem(cfg, *k.shape, v.shape[-1], beta is not None, gate, buf is not None, k.dtype)
         _lib.check(_lib.load().atlas_mem_validate(ctypes.byref(prob)), "atlas_mem_validate")
-        y, S_T, Z_T, buf_out = _native('recurrence', k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg.window,
+        y, S_T, Z_T, buf_out = _native('recurrence')(k, q, v, lr, decay, beta, gate, S_ref, S0, Z0, buf, cfg.window,
                                        cfg.map_degree if cfg.map_mode == 'elementwise' else 1, cfg.clamp_every or None,
                                        int(cfg.clamp_final))
         empty = torch.empty(0, device=dev)
@@ -832,7 +835,7 @@ def _wgrads(pairs, dtype) -> list:
     summed in a fixed order): 16384 tokens x 512 x 512 took 67 us through a transposed copy and a
     batched hipBLASLt product, whose plain form (one product with K = 16384 on few output tiles)
     took 100 us. fp32 operands keep torch's product over token slices."""
-    return _native('wgrads', [dy for dy, _ in pairs], [x for _, x in pairs], dtype)
+    return _native('wgrads')([dy for dy, _ in pairs], [x for _, x in pairs], dtype)
 
 
 def _wgrad(dy: Tensor, x: Tensor, dtype) -> Tensor:
@@ -847,13 +850,13 @@ def _products(layout: int, acts, weights):
     """atlas_linear_batch: up to four bf16 products in one launch. NT: acts[i] [..., k] x
     weights[i] [n, k] -> [..., n] (y = x W^T); NN: acts[i] [..., k] x weights[i] [k, n] -> [..., n]
     (dx = dy W). torch's products for other dtypes or sizes that are not multiples of 8."""
-    return _native('products', layout, list(acts), list(weights))
+    return _native('products')(layout, list(acts), list(weights))
 
 
 def linear(x: Tensor, w: Tensor) -> Tensor:
     """x W^T without bias: the product and its input gradient on atlas_linear_batch, the weight gradient
     split over the tokens (_wgrads)."""
-    return _native('linear', x, w)
+    return _native('linear')(x, w)
 
 
 def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj_weights, gate_weights, gate_biases,
@@ -878,7 +881,7 @@ def cell_prologue(x: Tensor, norm_weight: Tensor, eps: float, conv_weights, proj
     if conv_weights is not None and conv_weights[0].shape[-1] > 8:
         raise ValueError("the fused prologue supports depthwise convolutions of up to 8 taps")
     # one autograd node for all of it, with the products and weight gradients batched (csrc/host.cpp)
-    out = _native('cell_prologue', x, norm_weight, float(eps), list(conv_weights) if conv_weights is not None else [],
+    out = _native('cell_prologue')(x, norm_weight, float(eps), list(conv_weights) if conv_weights is not None else [],
                                       list(proj_weights), list(gate_weights or ()), list(gate_biases or ()) if gate_weights
                                       else [], q_gamma, k_gamma, heads, dim_head)
     return out[0], out[1], out[2], out[3], list(out[4:])

@@ -74,7 +74,7 @@ def _fused_chain(surprise, decay, last_update, am, last_momentum, gate, window, 
     """The chain in one kernel each way (atlas_omega_chain_fwd / _bwd), or None where they do not apply:
     one dtype (fp32 or bf16) on one GPU for the surprises and the scalars, at most two momentum orders
     and a window of at most 16. The separate scans and window sums serve everything else."""
-    return _native('omega_chain', surprise, decay, last_update, am, last_momentum, gate, window, buf)
+    return _native('omega_chain')(surprise, decay, last_update, am, last_momentum, gate, window, buf)
 
 
 def omega_store_chain(surprise: Tensor, decay_factor: Tensor, last_update: Tensor, *,
