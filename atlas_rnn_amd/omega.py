@@ -2,10 +2,11 @@
 
 `OmegaNeuralMemory.store_memories` (omega.py:120-330) turns per-chunk surprises of each memory-MLP
 parameter, `[(B H), n, *param]`, into per-chunk weight updates. Its Omega section
-(omega.py:262-318) is provided here as `omega_store_chain`, a function over plain tensors built on
-the library's primitives: the scalar-gated scan (`atlas_scan_fwd` / `_bwd`: the momentum scans and
-the `1 - decay` scan with `remove_prev=False`) and the inclusive window sum along n
-(`atlas_window_sum`: the omega window over the carried `__omega_buf` and the chunk). The
+(omega.py:262-318) is provided here as `omega_store_chain`, a function over plain tensors: one fused
+chain (`atlas_omega_chain_fwd` / `_bwd`: the momentum scans, the gate, the window over the carried
+`__omega_buf` and the chunk, the `1 - decay` scan), or, for what that does not take (learned combinations, the
+orthogonalisers, more orders, longer windows, other dtypes), the scalar-gated scan (`atlas_scan_fwd` / `_bwd`)
+and the inclusive window sum along n (`atlas_window_sum`) one after another. The
 per-sample gradients that produce the surprises (torch.func vmap over the memory MLP) stay in
 PyTorch, as does NeuralMemory itself.
 
