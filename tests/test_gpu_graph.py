@@ -83,3 +83,63 @@ def test_cell_step_graph_replays_match_eager(carried):
             assert torch.equal(got, want), \
                 f"replay {r}: {name} differs from the eager step (normwise {_normwise(got, want):.3e})"
     del graph
+
+
+def _chain_step():
+    from atlas_rnn_amd.omega import omega_store_chain
+    g = torch.Generator(device=DEV).manual_seed(5)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    x = dict(surprise=r(4, 19, 300), decay_factor=r(4, 19).sigmoid(), last_update=r(4, 300),
+             adaptive_momentum=r(2, 4, 19).sigmoid(), last_momentum=r(2, 4, 300), omega_gate=r(4, 19).sigmoid(),
+             omega_buf=r(4, 2, 300))
+    return lambda ins: omega_store_chain(**ins, omega_window=3), x
+
+
+def _affine_step():
+    g = torch.Generator(device=DEV).manual_seed(6)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    return lambda ins: (am.affine_associative_scan(ins["A"], ins["B"], prev=ins["prev"]),), \
+        dict(A=0.1 * r(3, 60, 21, 21), B=r(3, 60, 17, 21), prev=r(3, 17, 21))
+
+
+def _clamp_step():
+    g = torch.Generator(device=DEV).manual_seed(7)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g).to(torch.bfloat16)
+    x = dict(k=0.1 * r(3, 230, 32), q=r(3, 230, 32), v=r(3, 230, 32), lr=0.1 * r(3, 230).sigmoid(),
+             decay=r(3, 230).sigmoid(), beta=r(3, 230).sigmoid())
+    return lambda ins: [t for t in am.memory_recurrence(**ins, window=2, clamp_every=100) if t is not None], x
+
+
+@pytest.mark.parametrize("make", [_chain_step, _affine_step, _clamp_step], ids=["chain", "affine", "clamp100"])
+def test_operator_graph_replays_match_eager(make):
+    """Forward and gradients of an operator, captured and replayed on changed inputs."""
+    _say(f"graph capture of {make.__name__}")
+    torch.cuda.set_device(DEV)
+    f, x = make()
+    x = {n: t.requires_grad_() for n, t in x.items()}
+
+    def step():
+        outs = f(x)
+        return [o.detach() for o in outs] + list(torch.autograd.grad([o.float().sum() for o in outs], list(x.values())))
+
+    side = torch.cuda.Stream()   # default priority
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static = step()
+    for r in range(3):
+        with torch.no_grad():
+            for t in x.values():
+                t.mul_(0.9)
+        want = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(static, want)):
+            assert torch.isfinite(a.double()).all() and torch.equal(a, b), f"replay {r}: tensor {i}"
+    del graph
